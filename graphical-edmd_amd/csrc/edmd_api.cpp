@@ -152,6 +152,12 @@ struct edmd_batch {
      * one only for calendars of depth <= 2 without walls, field or damping,
      * and not for the growing systems' launch) */
     int loop_wpb = 1;
+    /* the wide loop (one system per workgroup of several wavefronts), of the
+     * Normal [0] and growing [1] launches: its wavefronts (0: not used),
+     * whether its arrays are in LDS, and its dynamic LDS */
+    int wide_waves[2] = {0, 0};
+    bool wide_lds[2] = {false, false};
+    size_t wide_dyn[2] = {0, 0};
 };
 
 struct edmd_ctx {
@@ -159,6 +165,7 @@ struct edmd_ctx {
 };
 
 static int choose_residency(edmd_batch* b);
+static int choose_wide(edmd_batch* b);
 static void set_sweep_variant(edmd_batch* b, int v);
 static int default_sweep_variant(const edmd_batch* b);
 
@@ -677,6 +684,44 @@ static int choose_residency(edmd_batch* b) {
                     b->lds_dyn[1] > b->lds_dyn[0] ? b->lds_dyn[1] : b->lds_dyn[0]);
     b->use_lds = b->residency == EDMD_RES_LDS ||
                  (b->residency == EDMD_RES_AUTO && b->lds_fit && b->nsys <= b->lds_slots);
+    return choose_wide(b);
+}
+
+/* Whether the loop runs each system on a workgroup of several wavefronts
+ * (edmd_wide.hip): while the device has wavefront slots to spare, i.e. for
+ * batches of at most EDMD_WIDE_PER_CU systems a CU, all of them resident at
+ * once.  With the arrays in LDS where that mode is in use and they fit beside
+ * the window; asked for LDS and not fitting, the loop of one wavefront runs. */
+static int choose_wide(edmd_batch* b) {
+    b->wide_waves[0] = b->wide_waves[1] = 0;
+    int dev = 0, ncu = 0;
+    HIPCHK(hipGetDevice(&dev));
+    HIPCHK(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
+    const int per_cu = (b->nsys + ncu - 1) / ncu;
+    if (per_cu > EDMD_WIDE_PER_CU) return EDMD_OK;
+    size_t cal = 0, both[2] = {0, 0};
+    for (int s = 0; s < b->nsys; s++) {
+        const EdmdConst& c = b->hs[s].c;
+        /* the scan of cells in LDS takes rows of whole 16-byte chunks */
+        if (edmd_wide_level(&c) < 0 || c.cap > EDMD_STAGE_CAP || (c.cap & 3) != 0) return EDMD_OK;
+        const size_t w = (size_t)edmd_wide_bytes(&c);
+        cal = std::max(cal, w);
+        for (int g = 0; g < 2; g++)
+            both[g] = std::max(both[g], (size_t)edmd_lds_layout(&c, g).total + w);
+    }
+    const int waves = per_cu <= 1 ? 8 : 4;
+    for (int g = 0; g < (b->any_grow ? 2 : 1); g++) {
+        int fit = 0;
+        b->wide_lds[g] = b->use_lds;
+        b->wide_dyn[g] = b->use_lds ? both[g] : cal;
+        HIPCHK(edmd_wide_occupancy(g, b->any_walls ? 1 : 0, waves, b->wide_lds[g], b->wide_dyn[g], &fit));
+        if (fit < per_cu && b->use_lds && b->residency != EDMD_RES_LDS) {
+            b->wide_lds[g] = false;
+            b->wide_dyn[g] = cal;
+            HIPCHK(edmd_wide_occupancy(g, b->any_walls ? 1 : 0, waves, 0, cal, &fit));
+        }
+        if (fit >= per_cu) b->wide_waves[g] = waves;
+    }
     return EDMD_OK;
 }
 
@@ -686,6 +731,11 @@ static bool packable(const edmd_batch* b) { return !b->any_walls && b->max_nlev 
 /* One launch of the event loop over every system (grow: the growing ones). */
 static hipError_t launch_loop(edmd_batch* b, int grow, const EdmdRunArgs& ra) {
     const int walls = b->any_walls ? 1 : 0;
+    const int g = grow ? 1 : 0;
+    /* (several systems per workgroup, where asked for, is the other loop's) */
+    if (b->wide_waves[g] && (grow || b->loop_wpb == 1))
+        return edmd_launch_run_wide(b->d_sys, b->nsys, grow, walls, b->wide_waves[g],
+                                    b->wide_lds[g] ? 1 : 0, b->wide_dyn[g], ra, b->stream);
     if (b->use_lds)
         return edmd_launch_run_lds(b->d_sys, b->nsys, b->max_nlev, grow, walls,
                                    b->lds_dyn[grow ? 1 : 0], ra, b->stream);
@@ -855,12 +905,15 @@ extern "C" int edmd_batch_autotune(edmd_batch* b, int sweep_reps, int64_t trial_
         ra.max_coll = ~(uint64_t)0;
         ra.tmax = 1e300;
         /* trials: HBM with 1, 2 and 4 systems per workgroup, then LDS */
+        const int asked = b->residency;
         const int wpbs[4] = {1, 2, 4, 1};
         double t[4] = {-1, -1, -1, -1};
         for (int m = 0; m < 4 && !rc; m++) {
             if (m == 3 ? !b->lds_fit : (m > 0 && !packable(b))) continue;
             b->use_lds = m == 3;
             b->loop_wpb = wpbs[m];
+            b->residency = m == 3 ? EDMD_RES_LDS : EDMD_RES_HBM;
+            if ((rc = choose_wide(b))) break;
             e = edmd_launch_epoch_begin(b->d_sys, b->nsys, trial_events, ~(uint64_t)0, b->stream);
             if (e == hipSuccess) e = hipEventRecord(e0, b->stream);
             if (e == hipSuccess && b->any_grow) e = launch_loop(b, 1, ra);
@@ -883,6 +936,7 @@ extern "C" int edmd_batch_autotune(edmd_batch* b, int sweep_reps, int64_t trial_
          * held over longer runs */
         if (best != 0 && t[0] > 0 && t[best] > 0.97 * t[0]) best = 0;
         b->loop_wpb = wpbs[best];
+        b->residency = asked;
         if (!rc) {
             r.loop_ms_hbm = t[0];
             r.loop_ms_packed[0] = t[1];

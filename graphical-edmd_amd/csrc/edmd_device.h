@@ -62,12 +62,17 @@ __device__ __forceinline__ int64_t lane_value64(int64_t v, int l) {
                      (uint32_t)__builtin_amdgcn_readlane((int)v, l));
 }
 
-/* A double moved across lanes by a DPP pattern (both halves). */
+/* A word or a double (both words) moved across lanes by a DPP pattern in which
+ * every lane has a source: no value to keep, so no move to set one up. */
+template <int CTRL>
+__device__ __forceinline__ int dpp_i32(int v) {
+    return __builtin_amdgcn_mov_dpp(v, CTRL, 0xf, 0xf, true);
+}
+
 template <int CTRL>
 __device__ __forceinline__ double dpp_f64(double v) {
     const long long b = __double_as_longlong(v);
-    const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, 0xf, 0xf, false);
-    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, 0xf, 0xf, false);
+    const int lo = dpp_i32<CTRL>((int)b), hi = dpp_i32<CTRL>((int)(b >> 32));
     return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
 }
 
@@ -94,10 +99,10 @@ __device__ __forceinline__ int imin(int a, int b) { return b < a ? b : a; }
 /* Minimum of an int over the wave, on every lane: the same DPP pattern as
  * wave_min, each step a single v_min_i32 with a DPP source. */
 __device__ __forceinline__ int wave_min_i32(int v) {
-    v = imin(v, __builtin_amdgcn_update_dpp(0x7fffffff, v, 0xb1, 0xf, 0xf, false));
-    v = imin(v, __builtin_amdgcn_update_dpp(0x7fffffff, v, 0x4e, 0xf, 0xf, false));
-    v = imin(v, __builtin_amdgcn_update_dpp(0x7fffffff, v, 0x141, 0xf, 0xf, false));
-    v = imin(v, __builtin_amdgcn_update_dpp(0x7fffffff, v, 0x140, 0xf, 0xf, false));
+    v = imin(v, dpp_i32<0xb1>(v));
+    v = imin(v, dpp_i32<0x4e>(v));
+    v = imin(v, dpp_i32<0x141>(v));
+    v = imin(v, dpp_i32<0x140>(v));
     const int r0 = __builtin_amdgcn_readlane(v, 0), r1 = __builtin_amdgcn_readlane(v, 16);
     const int r2 = __builtin_amdgcn_readlane(v, 32), r3 = __builtin_amdgcn_readlane(v, 48);
     return imin(imin(r0, r1), imin(r2, r3));
@@ -136,14 +141,14 @@ __device__ __forceinline__ int wave_argmin_lane(double v, double base, double& v
  * wave_min_i32 with the two chains interleaved, so each DPP step's latency
  * is covered by the other chain's step. */
 __device__ __forceinline__ void wave_min_i32x2(int& a, int& b) {
-    a = imin(a, __builtin_amdgcn_update_dpp(0x7fffffff, a, 0xb1, 0xf, 0xf, false));
-    b = imin(b, __builtin_amdgcn_update_dpp(0x7fffffff, b, 0xb1, 0xf, 0xf, false));
-    a = imin(a, __builtin_amdgcn_update_dpp(0x7fffffff, a, 0x4e, 0xf, 0xf, false));
-    b = imin(b, __builtin_amdgcn_update_dpp(0x7fffffff, b, 0x4e, 0xf, 0xf, false));
-    a = imin(a, __builtin_amdgcn_update_dpp(0x7fffffff, a, 0x141, 0xf, 0xf, false));
-    b = imin(b, __builtin_amdgcn_update_dpp(0x7fffffff, b, 0x141, 0xf, 0xf, false));
-    a = imin(a, __builtin_amdgcn_update_dpp(0x7fffffff, a, 0x140, 0xf, 0xf, false));
-    b = imin(b, __builtin_amdgcn_update_dpp(0x7fffffff, b, 0x140, 0xf, 0xf, false));
+    a = imin(a, dpp_i32<0xb1>(a));
+    b = imin(b, dpp_i32<0xb1>(b));
+    a = imin(a, dpp_i32<0x4e>(a));
+    b = imin(b, dpp_i32<0x4e>(b));
+    a = imin(a, dpp_i32<0x141>(a));
+    b = imin(b, dpp_i32<0x141>(b));
+    a = imin(a, dpp_i32<0x140>(a));
+    b = imin(b, dpp_i32<0x140>(b));
     const int a0 = __builtin_amdgcn_readlane(a, 0), a1 = __builtin_amdgcn_readlane(a, 16);
     const int a2 = __builtin_amdgcn_readlane(a, 32), a3 = __builtin_amdgcn_readlane(a, 48);
     const int b0 = __builtin_amdgcn_readlane(b, 0), b1 = __builtin_amdgcn_readlane(b, 16);
@@ -848,12 +853,15 @@ __device__ __forceinline__ void cross_time(const EdmdConst& C, double t, double 
 __device__ __forceinline__ int64_t rank_of(double t_ev, double paul, double dtp, double horizon,
                                            int64_t ctr) {
     const double dt = t_ev - paul;
-    /* without branches (the loop files 4-6 events per collision):
-     * bucket D - 1 - ctr, plus 2 ctr + 1 for the tree and the overflow
-     * list, plus 2^61 for the overflow list */
-    const int64_t up = (int64_t)(dt < dtp) | (int64_t)(dt >= horizon);
-    const int64_t ovf = (int64_t)(dt >= horizon);
-    return EDMD_RANK_DIRECT - 1 - ctr + (-up & (2 * ctr + 1)) + (ovf << 61);
+    /* bucket D - 1 - ctr = D + ~ctr, tree D + ctr, overflow list D + 2^61 +
+     * ctr: the low word of D is 0, so the words do not carry (the loop files
+     * 4-6 events per collision: no branches, and half the instructions of
+     * 64-bit sums) */
+    const bool up = (dt < dtp) | (dt >= horizon);
+    const uint32_t flip = up ? 0u : 0xffffffffu;
+    const uint32_t top = (uint32_t)(EDMD_RANK_DIRECT >> 32) + (dt >= horizon ? 0x20000000u : 0u);
+    const uint32_t lo = (uint32_t)ctr ^ flip, hi = ((uint32_t)(ctr >> 32) ^ flip) + top;
+    return (int64_t)((uint64_t)hi << 32 | lo);
 }
 
 /* Calendar leaf of a particle: its earlier slot by (time, rank) (a NaN key
@@ -942,366 +950,6 @@ __device__ __forceinline__ double predict_seq(const EdmdConst& C, const AR& A, d
     }
     partner = wall ? EDMD_WALL_CODE(xy) : best;
     return dt;
-}
-
-struct Owner {
-    int p;
-    double x, y, vx, vy, r;
-    int cx, cy;
-    double vr; /* radius growth rate (growth starts only) */
-};
-
-/* Wave-cooperative neighbour scan for one or two owners at once.
- *
- * Lanes 0-8 read the nine cell counts of owner a, lanes 16-24 those of
- * owner b; a segmented scan lays each owner's candidates out in traversal
- * order (y offset outer, x offset inner, newest list entry first, EDMD.c:
- * 2959-3003).  Lane f evaluates candidate f of a and candidate f of b, so
- * both owners share the slot and record round trips.  The minimum over
- * (time, traversal rank) among candidates with time < NEVER is the
- * reference's strict-less first minimum; no candidate gives NEVER and
- * partner 0 (EDMD.c:2830-2831, 3091-3093).  Results are uniform. */
-template <bool G, bool W = true, class AR>
-__device__ __forceinline__ void predict_owners_gather(const EdmdConst& C, const AR& A,
-                                                      int lane, double t, int nown,
-                                                      const Owner& a, const Owner& b, double& dta,
-                                                      int& pa, uint32_t& ca, double& dtb, int& pb,
-                                                      uint32_t& cb, bool& overlap) {
-    const int sub = lane & 15;
-    const int grp = lane >> 4;
-    int cell = 0, cnt = 0;
-    if (sub < 9 && (grp == 0 || (grp == 1 && nown == 2))) {
-        const int ocx = grp ? b.cx : a.cx;
-        const int ocy = grp ? b.cy : a.cy;
-        cell = wrap_cell(ocy + sub / 3 - 1, C.ncy) * C.ncx + wrap_cell(ocx + sub % 3 - 1, C.ncx);
-        cnt = A.ccnt[cell];
-    }
-    /* inclusive scan within each row of 16 lanes: DPP row shifts right by
-     * 1, 2, 4, 8, zeros shifted in at the row start */
-    int incl = cnt;
-    incl += __builtin_amdgcn_update_dpp(0, incl, 0x111, 0xf, 0xf, true);
-    incl += __builtin_amdgcn_update_dpp(0, incl, 0x112, 0xf, 0xf, true);
-    incl += __builtin_amdgcn_update_dpp(0, incl, 0x114, 0xf, 0xf, true);
-    incl += __builtin_amdgcn_update_dpp(0, incl, 0x118, 0xf, 0xf, true);
-    const int excl = incl - cnt;
-    /* slot index of candidate f of the cell this lane read is rowbase - f
-     * (newest entry first) */
-    const int64_t rowbase = (int64_t)cell * C.cap + cnt - 1 + excl;
-    const int totA = __builtin_amdgcn_readlane(incl, 8);
-    const int totB = (nown == 2) ? __builtin_amdgcn_readlane(incl, 24) : 0;
-    const int tot = totA > totB ? totA : totB;
-
-    /* running minimum, uniform: candidates come in traversal order, so a
-     * later pass only wins with a strictly earlier time, and within a pass
-     * the lowest lane among equal times is the earliest in traversal */
-    const double lim = G ? EDMD_GROW_NONE : EDMD_NEVER;
-    double btA = INF_D, btB = INF_D;
-    int bqA = 0, bqB = 0;
-    uint32_t bcA = 0, bcB = 0;
-    for (int base = 0; base < tot; base += 64) {
-        const int f = base + lane;
-        /* the cell holding candidate f: the last of the nine whose
-         * exclusive prefix is <= f (scalar reads and selects, no LDS) */
-        int64_t rbA = lane_value64(rowbase, 0), rbB = lane_value64(rowbase, 16);
-#pragma unroll
-        for (int s = 1; s < 9; ++s) {
-            const int64_t ra = lane_value64(rowbase, s), rb = lane_value64(rowbase, 16 + s);
-            if (f >= __builtin_amdgcn_readlane(excl, s)) rbA = ra;
-            if (f >= __builtin_amdgcn_readlane(excl, 16 + s)) rbB = rb;
-        }
-        int qA = -1, qB = -1;
-        if (f < totA) qA = A.cslot[rbA - f];
-        if (f < totB) qB = A.cslot[rbB - f];
-        const bool vA = qA >= 0 && qA != a.p;
-        const bool vB = qB >= 0 && qB != b.p;
-        EdmdPart rA, rB;
-        double gA = 0, gB = 0;
-        uint32_t cA = 0, cB = 0;
-        if (vA) { rA = A.p[qA]; cA = rA.coll; }
-        if (vB) { rB = A.p[qB]; cB = rB.coll; }
-        if (W && !G && (C.field_on || C.damping)) {
-            /* the neighbours flown to t and stored (EDMD.c:2664-2666) */
-            if (vA) {
-                fly_v<true>(C, t, rA.x, rA.y, rA.vx, rA.vy, rA.tl);
-                const auto w = A.p + qA;
-                w->x = rA.x; w->y = rA.y; w->vx = rA.vx; w->vy = rA.vy; w->tl = rA.tl;
-            }
-            if (vB) {
-                fly_v<true>(C, t, rB.x, rB.y, rB.vx, rB.vy, rB.tl);
-                const auto w = A.p + qB;
-                w->x = rB.x; w->y = rB.y; w->vx = rB.vx; w->vy = rB.vy; w->tl = rB.tl;
-            }
-        }
-        if (G && vA) gA = A.vr[qA];
-        if (G && vB) gB = A.vr[qB];
-        double tA = INF_D, tB = INF_D;
-        if (vA) {
-            double tt;
-            if (G)
-                tt = coll_time_grow(C, t, a.x, a.y, a.vx, a.vy, a.r, a.vr, rA.x, rA.y, rA.vx,
-                                    rA.vy, rA.tl, rA.rad, gA, overlap);
-            else
-                tt = log_time<W>(C, coll_time_nb(C, t, a.x, a.y, a.vx, a.vy, a.r, rA.x, rA.y,
-                                                 rA.vx, rA.vy, rA.tl, rA.rad, overlap));
-            if (tt < lim) tA = tt;
-        }
-        if (vB) {
-            double tt;
-            if (G)
-                tt = coll_time_grow(C, t, b.x, b.y, b.vx, b.vy, b.r, b.vr, rB.x, rB.y, rB.vx,
-                                    rB.vy, rB.tl, rB.rad, gB, overlap);
-            else
-                tt = log_time<W>(C, coll_time_nb(C, t, b.x, b.y, b.vx, b.vy, b.r, rB.x, rB.y,
-                                                 rB.vx, rB.vy, rB.tl, rB.rad, overlap));
-            if (tt < lim) tB = tt;
-        }
-        double mA;
-        const int wA = wave_argmin_lane(tA, 0.0, mA);
-        if (mA < btA) {
-            const int w = wA;
-            btA = mA;
-            bqA = __builtin_amdgcn_readlane(qA, w);
-            bcA = (uint32_t)__builtin_amdgcn_readlane((int)cA, w);
-        }
-        if (nown == 2) {
-            double mB;
-            const int wB = wave_argmin_lane(tB, 0.0, mB);
-            if (mB < btB) {
-                const int w = wB;
-                btB = mB;
-                bqB = __builtin_amdgcn_readlane(qB, w);
-                bcB = (uint32_t)__builtin_amdgcn_readlane((int)cB, w);
-            }
-        }
-    }
-    if (btA < lim) {
-        dta = btA; pa = bqA; ca = bcA;
-    } else {
-        dta = lim; pa = 0; ca = A.p[0].coll;
-    }
-    if (btB < lim) {
-        dtb = btB; pb = bqB; cb = bcB;
-    } else {
-        dtb = lim; pb = 0; cb = A.p[0].coll;
-    }
-}
-
-/* Largest cell capacity the staged scan handles (six 16-byte row chunks
- * per cell), and its LDS stage: every slot of 18 cells. */
-#define EDMD_STAGE_CAP 24
-#define EDMD_STAGE_MAX (18 * EDMD_STAGE_CAP)
-
-/* Inclusive prefix sum over the wave of values held by lanes 0-31 (rows 0
- * and 1): DPP row shifts within each row of 16, then row 0's total added
- * to row 1 (row_bcast:15). */
-__device__ __forceinline__ int scan32(int v) {
-    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, true);
-    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, true);
-    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, true);
-    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, true);
-    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);
-    return v;
-}
-
-/* Neighbour scan for one or two owners, candidates staged in LDS.
- *
- * Lane e < 9 reads cell e of owner a's 3x3 block, lane 9 + e cell e of
- * owner b's (y offset outer, x offset inner): its count and its whole slot
- * row in the same round trip.  A scan over the 18 counts places every
- * candidate at its traversal position -- owner a's first, then owner b's,
- * each cell's newest entry first (EDMD.c:2959-3003) -- and each lane writes
- * its cell's entries there in LDS.  Lane f then evaluates candidate f
- * against its owner, so the two owners share one pass when their
- * candidates fit in 64 lanes.  Per owner, the minimum time over eligible
- * candidates (time < NEVER), the lowest lane among equal times, and across
- * passes only a strictly earlier time: the reference's strict-less first
- * minimum.  Requires cap <= EDMD_STAGE_CAP, cap % 4 == 0 and cell rows
- * aligned to 16 bytes. */
-template <bool G, bool W = true, bool PF = false, class AR>
-__device__ __forceinline__ void predict_owners_staged(const EdmdConst& C, const AR& A,
-                                                      int lane, double t, int nown,
-                                                      const Owner& a, const Owner& b, double& dta,
-                                                      int& pa, uint32_t& ca, double& dtb, int& pb,
-                                                      uint32_t& cb, bool& overlap,
-                                                      int32_t* stage) {
-    const int nent = 9 * nown;
-    const bool ent = lane < nent;
-    const bool inB = lane >= 9;
-    const int sub = inB ? lane - 9 : lane;
-    int cnt = 0;
-    int4 row[EDMD_STAGE_CAP / 4];
-    if (ent) {
-        const int ocx = inB ? b.cx : a.cx;
-        const int ocy = inB ? b.cy : a.cy;
-        const int cell =
-            wrap_cell(ocy + sub / 3 - 1, C.ncy) * C.ncx + wrap_cell(ocx + sub % 3 - 1, C.ncx);
-        const int4* src = (const int4*)(A.cslot + (int64_t)cell * C.cap);
-        cnt = A.ccnt[cell];
-#pragma unroll
-        for (int c = 0; c < EDMD_STAGE_CAP / 4; ++c)
-            if (4 * c < C.cap) row[c] = src[c];
-    }
-    const int incl = scan32(cnt);
-    const int excl = incl - cnt;
-    const int totA = __builtin_amdgcn_readlane(incl, 8);
-    const int tot = __builtin_amdgcn_readlane(incl, nent - 1);
-    if (ent) {
-        /* slot k (k-th oldest) goes to excl + cnt - 1 - k */
-        const int top = excl + cnt - 1;
-#pragma unroll
-        for (int c = 0; c < EDMD_STAGE_CAP / 4; ++c) {
-            if (4 * c >= cnt) break;
-            stage[top - 4 * c] = row[c].x;
-            if (4 * c + 1 < cnt) stage[top - 4 * c - 1] = row[c].y;
-            if (4 * c + 2 < cnt) stage[top - 4 * c - 2] = row[c].z;
-            if (4 * c + 3 < cnt) stage[top - 4 * c - 3] = row[c].w;
-        }
-    }
-    WAVE_SYNC();
-
-    const double lim = G ? EDMD_GROW_NONE : EDMD_NEVER;
-    double btA = INF_D, btB = INF_D;
-    int bqA = 0, bqB = 0;
-    uint32_t bcA = 0, bcB = 0;
-    /* PF: the next pass's candidate records are read while this pass is
-     * evaluated (one fewer dependent round trip per extra pass; the records
-     * cost registers, so only the loop of large systems does it) */
-    EdmdPart rnext;
-    int qnext = -1;
-    if (PF) {
-        qnext = lane < tot ? stage[lane] : -1;
-        const int own0 = lane >= totA ? b.p : a.p;
-        if (qnext >= 0 && qnext != own0) rnext = A.p[qnext];
-    }
-    for (int base = 0; base < tot; base += 64) {
-        const int f = base + lane;
-        const bool isB = f >= totA;
-        int q;
-        EdmdPart rcur;
-        if (PF) {
-            q = qnext;
-            rcur = rnext;
-            const int fn = f + 64;
-            qnext = fn < tot ? stage[fn] : -1;
-            const int ownn = fn >= totA ? b.p : a.p;
-            if (qnext >= 0 && qnext != ownn) rnext = A.p[qnext];
-        } else {
-            q = f < tot ? stage[f] : -1;
-        }
-        const int own = isB ? b.p : a.p;
-        const bool v = q >= 0 && q != own;
-        double tq = INF_D;
-        uint32_t cq = 0;
-        if (v) {
-            EdmdPart r = PF ? rcur : A.p[q];
-            if (W && !G && (C.field_on || C.damping)) {
-                /* the neighbour flown to t and stored (EDMD.c:2664-2666); a
-                 * disk listed for both owners is written twice alike */
-                fly_v<true>(C, t, r.x, r.y, r.vx, r.vy, r.tl);
-                const auto w = A.p + q;
-                w->x = r.x;
-                w->y = r.y;
-                w->vx = r.vx;
-                w->vy = r.vy;
-                w->tl = r.tl;
-            }
-            cq = r.coll;
-            const double ox = isB ? b.x : a.x, oy = isB ? b.y : a.y;
-            const double ovx = isB ? b.vx : a.vx, ovy = isB ? b.vy : a.vy;
-            const double orad = isB ? b.r : a.r;
-            double tt;
-            if (G) {
-                const double ovr = isB ? b.vr : a.vr;
-                tt = coll_time_grow(C, t, ox, oy, ovx, ovy, orad, ovr, r.x, r.y, r.vx, r.vy, r.tl,
-                                    r.rad, A.vr[q], overlap);
-            } else {
-                tt = log_time<W>(C, coll_time_nb(C, t, ox, oy, ovx, ovy, orad, r.x, r.y, r.vx,
-                                                 r.vy, r.tl, r.rad, overlap));
-            }
-            if (tt < lim) tq = tt;
-        }
-        const bool hasA = base < totA, hasB = base + 64 > totA && nown == 2;
-        const double tA = isB ? INF_D : tq;
-        const double tB = isB ? tq : INF_D;
-        if (hasA && hasB) {
-            double mA, mB;
-            int wA, wB;
-            wave_argmin_lane2(tA, tB, 0.0, mA, wA, mB, wB);
-            if (mA < btA) {
-                btA = mA;
-                bqA = __builtin_amdgcn_readlane(q, wA);
-                bcA = (uint32_t)__builtin_amdgcn_readlane((int)cq, wA);
-            }
-            if (mB < btB) {
-                btB = mB;
-                bqB = __builtin_amdgcn_readlane(q, wB);
-                bcB = (uint32_t)__builtin_amdgcn_readlane((int)cq, wB);
-            }
-        } else if (hasA) {
-            double mA;
-            const int w = wave_argmin_lane(tA, 0.0, mA);
-            if (mA < btA) {
-                btA = mA;
-                bqA = __builtin_amdgcn_readlane(q, w);
-                bcA = (uint32_t)__builtin_amdgcn_readlane((int)cq, w);
-            }
-        } else if (hasB) {
-            double mB;
-            const int w = wave_argmin_lane(tB, 0.0, mB);
-            if (mB < btB) {
-                btB = mB;
-                bqB = __builtin_amdgcn_readlane(q, w);
-                bcB = (uint32_t)__builtin_amdgcn_readlane((int)cq, w);
-            }
-        }
-    }
-    WAVE_SYNC();
-    if (btA < lim) {
-        dta = btA; pa = bqA; ca = bcA;
-    } else {
-        dta = lim; pa = 0; ca = A.p[0].coll;
-    }
-    if (btB < lim) {
-        dtb = btB; pb = bqB; cb = bcB;
-    } else {
-        dtb = lim; pb = 0; cb = A.p[0].coll;
-    }
-}
-
-/* The staged scan where the cell capacity allows it, else the gather scan
- * from HBM; both give the reference's result bit for bit. */
-template <bool G, bool W = true, bool PF = false, class AR>
-__device__ __forceinline__ void predict_owners(const EdmdConst& C, const AR& A, int lane,
-                                               double t, int nown, const Owner& a, const Owner& b,
-                                               double& dta, int& pa, uint32_t& ca, double& dtb,
-                                               int& pb, uint32_t& cb, bool& overlap,
-                                               int32_t* stage) {
-    if (C.cap <= EDMD_STAGE_CAP && (C.cap & 3) == 0)
-        predict_owners_staged<G, W, PF>(C, A, lane, t, nown, a, b, dta, pa, ca, dtb, pb, cb, overlap,
-                                    stage);
-    else
-        predict_owners_gather<G, W>(C, A, lane, t, nown, a, b, dta, pa, ca, dtb, pb, cb, overlap);
-    if (W && C.walls) {
-        /* the wall time starts the reference's minimum: a neighbour
-         * replaces it only when strictly earlier */
-        auto wt = [&](const Owner& o, double& dw, int& xy) {
-            const int typ = (C.walls & 8) ? A.ptype[o.p] : 0;
-            return G ? wall_time_grow(C, o.x, o.y, o.vx, o.vy, o.r, o.vr, o.cx, o.cy, dw, xy, typ)
-                     : wall_time(C, o.x, o.y, o.vx, o.vy, o.r, o.cx, o.cy, dw, xy, typ);
-        };
-        double dw;
-        int xy;
-        if (wt(a, dw, xy) && !(dta < dw)) {
-            dta = dw;
-            pa = EDMD_WALL_CODE(xy);
-            ca = 0;
-        }
-        if (nown == 2 && wt(b, dw, xy) && !(dtb < dw)) {
-            dtb = dw;
-            pb = EDMD_WALL_CODE(xy);
-            cb = 0;
-        }
-    }
 }
 
 /* ------------------------------------------------------------ calendar */
@@ -1433,32 +1081,41 @@ __device__ __forceinline__ void path_prefetch(const EdmdConst& C, const AR& A, i
     }
 }
 
-/* Stores the new leaves of pA (and pB >= 0) with their ranks and recomputes
- * every node on their paths from the prefetched children, substituting the
- * freshly computed path nodes; where the paths meet one node takes both.
- * With `top` (the event loop's LDS copy of the top level) the top-level
- * nodes are written there instead of to HBM. */
+/* Stores leaf p with its rank. */
+template <class AR>
+__device__ __forceinline__ void leaf_store(const AR& A, int lane, int p, const Leaf& L) {
+    if (lane == 0) {
+        EdmdNode n;
+        n.key = L.key;
+        n.idx = p;
+        n.aux = L.aux;
+        A.leaf[p] = n;
+        A.lrank[p] = L.rank;
+    }
+}
+
+/* Recomputes every node on the paths of pA (and pB >= 0), whose new leaves
+ * (keys kA, kB, event codes xA, xB) the caller has stored with their ranks,
+ * from the prefetched children, substituting the freshly computed path
+ * nodes; where the paths meet one node takes both.  With `top` (the event
+ * loop's LDS copy of the top level) the top-level nodes are written there
+ * instead of to HBM. */
 template <int ML, class AR>
 __device__ __forceinline__ void path_update(const EdmdConst& C, const AR& A, int lane,
-                                            const PathCache<ML>& P, int pA, Leaf LA, int pB,
-                                            Leaf LB, EdmdNode* top, double base) {
-    double kA = LA.key, kB = LB.key;
-    int xA = LA.aux, xB = LB.aux;
-    if (lane == 0) {
+                                            const PathCache<ML>& P, int pA, double kA, int xA,
+                                            int pB, double kB, int xB, EdmdNode* top,
+                                            double base) {
+    if (top && C.nlev == 0 && lane == 0) {
         EdmdNode n;
         n.key = kA;
         n.idx = pA;
         n.aux = xA;
-        A.leaf[pA] = n;
-        A.lrank[pA] = LA.rank;
-        if (top && C.nlev == 0) top[pA] = n;
+        top[pA] = n;
         if (pB >= 0) {
             n.key = kB;
             n.idx = pB;
             n.aux = xB;
-            A.leaf[pB] = n;
-            A.lrank[pB] = LB.rank;
-            if (top && C.nlev == 0) top[pB] = n;
+            top[pB] = n;
         }
     }
     WAVE_SYNC();

@@ -86,15 +86,20 @@ __global__ __launch_bounds__(64) void k_repredict(const EdmdSys* __restrict__ sy
     bool ov = false;
     if (which & 2) {
         const bool grow = uni(A.st->growing) != 0;
-        const Owner o{i, pi.x, pi.y, pi.vx, pi.vy, pi.rad, pi.cx, pi.cy, grow ? A.vr[i] : 0.0};
-        double dt, dtb;
-        int pb;
-        uint32_t cpb;
-        if (grow)
-            predict_owners<true>(C, A, lane, t, 1, o, o, dt, e.partner, e.cact, dtb, pb, cpb, ov, stage);
-        else
-            predict_owners<false>(C, A, lane, t, 1, o, o, dt, e.partner, e.cact, dtb, pb, cpb, ov, stage);
-        e.tcoll = t + dt;
+        EvState S;
+        S.own = i;
+        S.x = pi.x; S.y = pi.y; S.vx = pi.vx; S.vy = pi.vy; S.r = pi.rad; S.m = pi.m;
+        S.vr = grow ? A.vr[i] : 0.0;
+        S.coll = pi.coll; S.cx = pi.cx; S.cy = pi.cy;
+        S.kind = EVK_STALE; /* the collision slot alone */
+        S.nown = 1;
+        S.ov = false;
+        if (grow) event_predict<true, true, false>(C, A, lane, t, S, stage);
+        else event_predict<false, true, false>(C, A, lane, t, S, stage);
+        ov = S.ov;
+        e.partner = S.partner;
+        e.cact = S.cact;
+        e.tcoll = S.tk;
         rcoll = rank_of(e.tcoll, paul, C.dtp, C.horizon, ctr++);
     }
     if (lane == 0) {
@@ -102,8 +107,9 @@ __global__ __launch_bounds__(64) void k_repredict(const EdmdSys* __restrict__ sy
         A.erank[2 * i] = rcoll;
         A.erank[2 * i + 1] = rcross;
     }
-    path_update<ML>(C, A, lane, P, i, make_leaf(e.tcoll, rcoll, e.tcross, rcross, e.partner, e.dir),
-                    -1, Leaf{}, nullptr, t);
+    const Leaf L = make_leaf(e.tcoll, rcoll, e.tcross, rcross, e.partner, e.dir);
+    leaf_store(A, lane, i, L);
+    path_update<ML>(C, A, lane, P, i, L.key, L.aux, -1, 0.0, 0, nullptr, t);
     const bool any_ov = __ballot(ov) != 0ull;
     if (lane == 0) {
         A.st->ctr = ctr;
@@ -177,8 +183,9 @@ __global__ __launch_bounds__(64) void k_queue_edit(const EdmdSys* __restrict__ s
         A.erank[2 * i] = rcoll;
         A.erank[2 * i + 1] = rcross;
     }
-    path_update<ML>(C, A, lane, P, i, make_leaf(e.tcoll, rcoll, e.tcross, rcross, e.partner, e.dir),
-                    -1, Leaf{}, nullptr, st->t);
+    const Leaf L = make_leaf(e.tcoll, rcoll, e.tcross, rcross, e.partner, e.dir);
+    leaf_store(A, lane, i, L);
+    path_update<ML>(C, A, lane, P, i, L.key, L.aux, -1, 0.0, 0, nullptr, st->t);
     if (lane == 0) st->ctr = ctr;
 }
 
@@ -360,6 +367,42 @@ hipError_t edmd_launch_run_lds(const EdmdSys* d_sys, int nsys, int max_nlev, int
     else if (walls) EdmdLoopVariant<false, true>::run_lds(d_sys, nsys, max_nlev, dyn_bytes, ra, s);
     else EdmdLoopVariant<false, false>::run_lds(d_sys, nsys, max_nlev, dyn_bytes, ra, s);
     return hipGetLastError();
+}
+
+static const void* wide_kernel(int grow, int walls, int waves, int lds) {
+    if (grow)
+        return walls ? EdmdWideVariant<true, true>::kernel(waves, lds)
+                     : EdmdWideVariant<true, false>::kernel(waves, lds);
+    return walls ? EdmdWideVariant<false, true>::kernel(waves, lds)
+                 : EdmdWideVariant<false, false>::kernel(waves, lds);
+}
+
+hipError_t edmd_wide_occupancy(int grow, int walls, int waves, int lds, size_t dyn_bytes,
+                               int* blocks_per_cu) {
+    *blocks_per_cu = 0;
+    const void* f = wide_kernel(grow, walls, waves, lds);
+    if (!f) return hipErrorInvalidValue;
+    int dev = 0, maxblk = 0;
+    hipFuncAttributes fa;
+    hipError_t e = hipFuncGetAttributes(&fa, f);
+    if (e == hipSuccess) e = hipGetDevice(&dev);
+    if (e == hipSuccess)
+        e = hipDeviceGetAttribute(&maxblk, hipDeviceAttributeMaxSharedMemoryPerBlock, dev);
+    if (e != hipSuccess) return e;
+    if (fa.sharedSizeBytes + dyn_bytes > (size_t)maxblk) return hipSuccess; /* none fits */
+    /* the kernel's own limit, the same whatever the batch */
+    e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize,
+                            maxblk - (int)fa.sharedSizeBytes);
+    if (e != hipSuccess) return e;
+    return hipOccupancyMaxActiveBlocksPerMultiprocessor(blocks_per_cu, f, 64 * waves, dyn_bytes);
+}
+
+hipError_t edmd_launch_run_wide(const EdmdSys* d_sys, int nsys, int grow, int walls, int waves,
+                                int lds, size_t dyn_bytes, EdmdRunArgs ra, hipStream_t s) {
+    if (grow && walls) return EdmdWideVariant<true, true>::run(waves, lds, d_sys, nsys, dyn_bytes, ra, s);
+    if (grow) return EdmdWideVariant<true, false>::run(waves, lds, d_sys, nsys, dyn_bytes, ra, s);
+    if (walls) return EdmdWideVariant<false, true>::run(waves, lds, d_sys, nsys, dyn_bytes, ra, s);
+    return EdmdWideVariant<false, false>::run(waves, lds, d_sys, nsys, dyn_bytes, ra, s);
 }
 
 hipError_t edmd_launch_peek(const EdmdSys* d_sys, int nsys, EdmdPeek* out, hipStream_t s) {

@@ -7,7 +7,7 @@
 #ifndef EDMD_LOOP_H
 #define EDMD_LOOP_H
 
-#include "edmd_device.h"
+#include "edmd_event.h"
 
 /* ------------------------------------------------------------ event loop */
 
@@ -31,6 +31,11 @@ struct QueueState {
      * overflow list (moved != 0) */
     double mkey;
     int32_t mleaf, maux, moved;
+    /* the loop's registers between its inner loop and a scheduled event */
+    double t, paul;
+    int64_t ctr, win;
+    uint64_t ncol, nevents, ncross;
+    int32_t status, err_i, err_j, last_type;
 };
 
 /* Top level of the calendar between HBM and the LDS copy. */
@@ -131,6 +136,30 @@ __device__ __forceinline__ int64_t refiled_rank(const EdmdConst& C, double t_ev,
     return EDMD_RANK_DIRECT - 1 - c;
 }
 
+/* The slots of disk k that wait in the overflow list, filed again at a wrap
+ * of the bucket ring with the counter at now: a slot ranked EDMD_RANK_OVF + c
+ * gets the counter 2 now - 1 - c.  Returns whether its leaf was made again. */
+template <class AR>
+__device__ __forceinline__ bool refile_disk(const EdmdConst& C, const AR& A, int k, double paul,
+                                            int64_t now) {
+    int64_t rk = A.erank[2 * k], rx = A.erank[2 * k + 1];
+    const bool fk = EDMD_RANK_IS_OVF(rk), fx = EDMD_RANK_IS_OVF(rx);
+    if (!fk && !fx) return false;
+    const EdmdEv e = A.e[k];
+    if (fk) rk = refiled_rank(C, e.tcoll, paul, 2 * now - 1 - (rk - EDMD_RANK_OVF));
+    if (fx) rx = refiled_rank(C, e.tcross, paul, 2 * now - 1 - (rx - EDMD_RANK_OVF));
+    A.erank[2 * k] = rk;
+    A.erank[2 * k + 1] = rx;
+    const Leaf Lf = make_leaf(e.tcoll, rk, e.tcross, rx, e.partner, e.dir);
+    EdmdNode nd;
+    nd.key = Lf.key;
+    nd.idx = k;
+    nd.aux = Lf.aux;
+    A.leaf[k] = nd;
+    A.lrank[k] = Lf.rank;
+    return true;
+}
+
 /* The particle events of the overflow list filed again at a wrap
  * (EDMD.c:2292-2302), after its special events, in the order of the list's
  * walk from its head (the newest first): a slot ranked EDMD_RANK_OVF + c
@@ -159,24 +188,7 @@ __device__ __noinline__ void refile_wrap(const EdmdConst& C, const AR& A, QueueS
     refile_specials(C, A.st, paul, win, ctr);
     const int64_t now = ctr;
     bool any = false;
-    for (int k = lane; k < C.n; k += 64) {
-        int64_t rk = A.erank[2 * k], rx = A.erank[2 * k + 1];
-        const bool fk = EDMD_RANK_IS_OVF(rk), fx = EDMD_RANK_IS_OVF(rx);
-        if (!fk && !fx) continue;
-        const EdmdEv e = A.e[k];
-        if (fk) rk = refiled_rank(C, e.tcoll, paul, 2 * now - 1 - (rk - EDMD_RANK_OVF));
-        if (fx) rx = refiled_rank(C, e.tcross, paul, 2 * now - 1 - (rx - EDMD_RANK_OVF));
-        A.erank[2 * k] = rk;
-        A.erank[2 * k + 1] = rx;
-        const Leaf Lf = make_leaf(e.tcoll, rk, e.tcross, rx, e.partner, e.dir);
-        EdmdNode nd;
-        nd.key = Lf.key;
-        nd.idx = k;
-        nd.aux = Lf.aux;
-        A.leaf[k] = nd;
-        A.lrank[k] = Lf.rank;
-        any = true;
-    }
+    for (int k = lane; k < C.n; k += 64) any |= refile_disk(C, A, k, paul, now);
     const bool moved = __ballot(any) != 0ull;
     const int64_t lo = A.st->ovf_lo;
     WAVE_SYNC();
@@ -279,29 +291,51 @@ __device__ __forceinline__ void trace_push(const EdmdConst& C, const AR& A, int 
     }
 }
 
+/* A group of NT threads runs the handlers of scheduled events: one wavefront
+ * (the serial loop) or the whole workgroup (the wide loop). */
+template <int NT>
+__device__ __forceinline__ void group_sync() {
+    if (NT > 64) __syncthreads();
+    else WAVE_SYNC();
+}
+
 /* Ordered sum over all particles of f(q), accumulated in particle order as
- * the reference's serial loops do (physicalQ, EDMD.c:5968-6013). */
-template <class F>
-__device__ __forceinline__ double ordered_sum(int n, int lane, F f) {
+ * the reference's serial loops do (physicalQ, EDMD.c:5968-6013).  The first
+ * wavefront adds; the chain of additions is the bound (n times the latency
+ * of one), so each value comes by readlane, not by an LDS shuffle per
+ * addition, and the next 64 values are read ahead.  red: LDS through which
+ * a group of several wavefronts gets the sum. */
+template <int NT, class F>
+__device__ __forceinline__ double ordered_sum(int n, int tid, double* red, F f) {
     double acc = 0;
-    for (int base = 0; base < n; base += 64) {
-        int q = base + lane;
-        double v = (q < n) ? f(q) : 0.0;
-        int lim = n - base < 64 ? n - base : 64;
-        for (int l = 0; l < lim; ++l) {
-            double vl = __shfl(v, l, 64);
-            acc += vl;
+    if (NT == 64 || tid < 64) {
+        const int lane = tid & 63;
+        double next = lane < n ? f(lane) : 0.0;
+        int base = 0;
+        for (; base + 64 <= n; base += 64) {
+            const double v = next;
+            const int q = base + 64 + lane;
+            next = q < n ? f(q) : 0.0;
+#pragma unroll
+            for (int l = 0; l < 64; ++l) acc += lane_value(v, l);
         }
+        for (int l = 0; l < n - base; ++l) acc += lane_value(next, l);
+        if (NT > 64 && lane == 0) red[0] = acc;
+    }
+    if (NT > 64) {
+        __syncthreads();
+        acc = red[0];
+        __syncthreads();
     }
     return acc;
 }
 
-template <bool G, bool W, class AR>
-__device__ __forceinline__ void ev_screenshot(const EdmdConst& C, const AR& A, int lane,
+template <int NT, bool G, bool W, class AR>
+__device__ __forceinline__ void ev_screenshot(const EdmdConst& C, const AR& A, int tid,
                                               LoopRegs& R) {
     /* takeAScreenshot, EDMD.c:4657-4677: free-fly every particle */
     const double t = R.t;
-    for (int q = lane; q < C.n; q += 64) {
+    for (int q = tid; q < C.n; q += NT) {
         const auto r = A.p + q;
         double x = r->x, y = r->y, tl = r->tl;
         if (G) {
@@ -320,33 +354,34 @@ __device__ __forceinline__ void ev_screenshot(const EdmdConst& C, const AR& A, i
         r->y = y;
         r->tl = tl;
     }
-    WAVE_SYNC();
+    group_sync<NT>();
     const int64_t wk = window_of(t + C.dtime, R.paul, C.dtp, C.nlists, R.win);
     const int64_t rk = take_rank(C, R, t + C.dtime);
-    if (lane == 0) {
+    if (tid == 0) {
         A.st->next_screen = t + C.dtime;
         A.st->rank_screen = rk;
         A.st->win_screen = wk;
     }
-    WAVE_SYNC();
+    group_sync<NT>();
 }
 
-template <class AR>
-__device__ __forceinline__ void ev_thermo(const EdmdConst& C, const AR& A, int lane, LoopRegs& R) {
+template <int NT, class AR>
+__device__ __forceinline__ void ev_thermo(const EdmdConst& C, const AR& A, int tid, LoopRegs& R,
+                                          double* vir, double* red) {
     /* takeAThermo + saveThermo, EDMD.c:4679-4713, 5232-5333 */
     const double t = R.t;
     const uint64_t ncol = R.ncol;
     const int64_t wk = window_of(t + C.dtime_thermo, R.paul, C.dtp, C.nlists, R.win);
     const int64_t rk = take_rank(C, R, t + C.dtime_thermo);
     const auto P = A.p;
-    double E = ordered_sum(C.n, lane, [&](int q) {
+    double E = ordered_sum<NT>(C.n, tid, red, [&](int q) {
         double a = P[q].vx;
         return 0.5 * P[q].m * (a * a + P[q].vy * P[q].vy);
     });
-    double ex = ordered_sum(C.n, lane, [&](int q) { return P[q].m * P[q].vx * P[q].vx; });
-    double ey = ordered_sum(C.n, lane, [&](int q) { return P[q].m * P[q].vy * P[q].vy; });
-    double exy = ordered_sum(C.n, lane, [&](int q) { return P[q].m * P[q].vx * P[q].vy; });
-    double eyx = ordered_sum(C.n, lane, [&](int q) { return P[q].m * P[q].vy * P[q].vx; });
+    double ex = ordered_sum<NT>(C.n, tid, red, [&](int q) { return P[q].m * P[q].vx * P[q].vx; });
+    double ey = ordered_sum<NT>(C.n, tid, red, [&](int q) { return P[q].m * P[q].vy * P[q].vy; });
+    double exy = ordered_sum<NT>(C.n, tid, red, [&](int q) { return P[q].m * P[q].vx * P[q].vy; });
+    double eyx = ordered_sum<NT>(C.n, tid, red, [&](int q) { return P[q].m * P[q].vy * P[q].vx; });
     /* the mid wall's columns (EDMD.c:5453-5477), from the stored disks in
      * particle order; type-0 disks on the other side add +0 */
     double nl = 0, nr = 0, ns = 0, tl = 0, tr = 0, tsol = 0;
@@ -356,20 +391,20 @@ __device__ __forceinline__ void ev_thermo(const EdmdConst& C, const AR& A, int l
         auto temp = [&](int q) {
             return 0.5 * P[q].m * (P[q].vx * P[q].vx + P[q].vy * P[q].vy);
         };
-        nl = ordered_sum(C.n, lane, [&](int q) { return (T[q] == 0 && P[q].x < h) ? 1.0 : 0.0; });
-        nr = ordered_sum(C.n, lane, [&](int q) { return (T[q] == 0 && P[q].x > h) ? 1.0 : 0.0; });
-        ns = ordered_sum(C.n, lane, [&](int q) { return T[q] != 0 ? 1.0 : 0.0; });
-        tl = ordered_sum(C.n, lane, [&](int q) { return (T[q] == 0 && P[q].x < h) ? temp(q) : 0.0; });
-        tr = ordered_sum(C.n, lane, [&](int q) { return (T[q] == 0 && P[q].x > h) ? temp(q) : 0.0; });
-        tsol = ordered_sum(C.n, lane, [&](int q) { return T[q] != 0 ? temp(q) : 0.0; });
+        nl = ordered_sum<NT>(C.n, tid, red, [&](int q) { return (T[q] == 0 && P[q].x < h) ? 1.0 : 0.0; });
+        nr = ordered_sum<NT>(C.n, tid, red, [&](int q) { return (T[q] == 0 && P[q].x > h) ? 1.0 : 0.0; });
+        ns = ordered_sum<NT>(C.n, tid, red, [&](int q) { return T[q] != 0 ? 1.0 : 0.0; });
+        tl = ordered_sum<NT>(C.n, tid, red, [&](int q) { return (T[q] == 0 && P[q].x < h) ? temp(q) : 0.0; });
+        tr = ordered_sum<NT>(C.n, tid, red, [&](int q) { return (T[q] == 0 && P[q].x > h) ? temp(q) : 0.0; });
+        tsol = ordered_sum<NT>(C.n, tid, red, [&](int q) { return T[q] != 0 ? temp(q) : 0.0; });
     }
     EdmdState* st = A.st;
     /* EDMD.c:5253-5256: the disc's area inside a circular wall */
     const double area = (C.walls & 4) ? 3.14159265358979323846 * C.halfLx * C.halfLx : C.Lx * C.Ly;
     const double dT = t - st->last_thermo;
-    const double v0 = R.q->vir[0], v1 = R.q->vir[1], v2 = R.q->vir[2], v3 = R.q->vir[3];
+    const double v0 = vir[0], v1 = vir[1], v2 = vir[2], v3 = vir[3];
     const int k = st->nthermo;
-    if (lane == 0) {
+    if (tid == 0) {
         if (k < C.thermo_cap) {
             EdmdThermoRow row;
             row.t = t;
@@ -412,8 +447,127 @@ __device__ __forceinline__ void ev_thermo(const EdmdConst& C, const AR& A, int l
         st->rank_thermo = rk;
         st->win_thermo = wk;
     }
-    if (lane == 0) R.q->vir[0] = R.q->vir[1] = R.q->vir[2] = R.q->vir[3] = 0;
-    WAVE_SYNC();
+    if (tid == 0) vir[0] = vir[1] = vir[2] = vir[3] = 0;
+    group_sync<NT>();
+}
+
+template <int NT, bool G, bool W, class AR>
+__device__ __forceinline__ bool ev_rescale(const EdmdConst& C, const AR& A, int tid,
+                                           LoopRegs& R, double* red) {
+    const double t = R.t;
+    /* addNoise, velocity-rescale branch (noise == 2): EDMD.c:4828-4832,
+     * 4880-4915, 4922 */
+    const auto P = A.p;
+    double E = ordered_sum<NT>(C.n, tid, red, [&](int q) {
+        double a = P[q].vx;
+        return 0.5 * P[q].m * (a * a + P[q].vy * P[q].vy);
+    });
+    for (int q = tid; q < C.n; q += NT) {
+        EdmdPart r = A.p[q];
+        r.coll = r.coll + 1;
+        if (G) fly_grow(C, t, r.x, r.y, r.vx, r.vy, r.tl, r.rad, A.vr[q]);
+        else fly_v<W>(C, t, r.x, r.y, r.vx, r.vy, r.tl);
+        r.vx /= sqrt(E / C.n / C.temperature);
+        r.vy /= sqrt(E / C.n / C.temperature);
+        A.p[q] = r;
+    }
+    group_sync<NT>();
+    bool ov = false;
+    /* per particle: crossing, then collision (EDMD.c:4909-4915) */
+    for (int q = tid; q < C.n; q += NT)
+        ov |= sweep_one<G, W>(C, A, t, q, R.paul, R.ctr + 2 * (int64_t)q, R.ctr + 2 * (int64_t)q + 1);
+    R.ctr += 2 * (int64_t)C.n;
+    const bool any_ov = __ballot(ov) != 0ull;
+    group_sync<NT>();
+    const int64_t wk = window_of(t + C.dtnoise, R.paul, C.dtp, C.nlists, R.win);
+    const int64_t rk = take_rank(C, R, t + C.dtnoise);
+    if (tid == 0) {
+        A.st->next_noise = t + C.dtnoise;
+        A.st->rank_noise = rk;
+        A.st->win_noise = wk;
+    }
+    group_sync<NT>();
+    return any_ov;
+}
+
+__device__ __forceinline__ void flag_overlap(LoopRegs& R, bool ov, int p) {
+    if (__ballot(ov) != 0ull && R.status == EDMD_DEV_OK) {
+        R.status = EDMD_DEV_OVERLAP;
+        R.err_i = p;
+    }
+}
+
+/* stopGrow, EDMD.c:4740-4785 (2D, no wells): final flight with growth, all
+ * counters and image counters reset, normalizePhysicalQ (EDMD.c:5723-5764:
+ * remove the mean momentum, scale to E/N = Einit), then the Normal
+ * prediction of every disk with stopGrow's partner counters, and a new
+ * calendar.  The caller continues in the Normal loop. */
+template <int NT, bool W, class AR>
+__device__ __forceinline__ bool ev_stop_grow(const EdmdConst& C, const AR& A, int tid,
+                                             LoopRegs& R, double* red) {
+    const double t = R.t;
+    for (int q = tid; q < C.n; q += NT) {
+        EdmdPart r = A.p[q];
+        fly_grow(C, t, r.x, r.y, r.vx, r.vy, r.tl, r.rad, A.vr[q]);
+        r.coll = 0;
+        A.p[q] = r;
+        A.img[2 * q] = 0;
+        A.img[2 * q + 1] = 0;
+    }
+    group_sync<NT>();
+    const auto P = A.p;
+    const int n = C.n;
+    if (!(W && (C.walls & 4))) {
+        const double px = ordered_sum<NT>(n, tid, red, [&](int q) { return P[q].vx * P[q].m; });
+        const double py = ordered_sum<NT>(n, tid, red, [&](int q) { return P[q].vy * P[q].m; });
+        for (int q = tid; q < n; q += NT) {
+            const double m = P[q].m;
+            P[q].vx -= px / (n * m);
+            P[q].vy -= py / (n * m);
+        }
+    } else {
+        /* in a circle, the angular momentum about the centre
+         * (EDMD.c:5730-5749): dvT accumulates -m (x0 vy - y0 vx), dvM m r */
+        const double h = C.halfLx;
+        const double dvT = -ordered_sum<NT>(n, tid, red, [&](int q) {
+            return P[q].m * (-P[q].vx * (P[q].y - h) + P[q].vy * (P[q].x - h));
+        });
+        const double dvM = ordered_sum<NT>(n, tid, red, [&](int q) {
+            return P[q].m * sqrt((P[q].x - h) * (P[q].x - h) + (P[q].y - h) * (P[q].y - h));
+        });
+        const double dv = dvT / dvM;
+        for (int q = tid; q < n; q += NT) {
+            const double x0 = P[q].x - h, y0 = P[q].y - h;
+            const double r = sqrt(x0 * x0 + y0 * y0);
+            P[q].vx += -dv * y0 / r;
+            P[q].vy += dv * x0 / r;
+        }
+    }
+    group_sync<NT>();
+    const double E = ordered_sum<NT>(n, tid, red, [&](int q) {
+        double a = P[q].vx;
+        return 0.5 * P[q].m * (a * a + P[q].vy * P[q].vy);
+    });
+    for (int q = tid; q < n; q += NT) {
+        P[q].vx /= sqrt(E / n / C.einit);
+        P[q].vy /= sqrt(E / n / C.einit);
+        P[q].coll = 1;
+    }
+    group_sync<NT>();
+    bool ov = false;
+    /* per particle: collision, then crossing (EDMD.c:4770-4776) */
+    for (int q = tid; q < n; q += NT)
+        ov |= sweep_one<false, W>(C, A, t, q, R.paul, R.ctr + 2 * (int64_t)q + 1,
+                               R.ctr + 2 * (int64_t)q, true);
+    R.ctr += 2 * (int64_t)n;
+    group_sync<NT>();
+    const bool any_ov = __ballot(ov) != 0ull;
+    if (tid == 0) {
+        A.st->growing = 0;
+        A.st->next_grow = INF_D;
+    }
+    group_sync<NT>();
+    return any_ov;
 }
 
 /* Rebuilds every level of the calendar after a full re-prediction. */
@@ -425,580 +579,30 @@ __device__ void rebuild_tree(const EdmdConst& C, const AR& A, int lane) {
     }
 }
 
-template <bool G, bool W, class AR>
-__device__ __forceinline__ bool ev_rescale(const EdmdConst& C, const AR& A, int lane,
-                                           LoopRegs& R) {
-    const double t = R.t;
-    /* addNoise, velocity-rescale branch (noise == 2): EDMD.c:4828-4832,
-     * 4880-4915, 4922 */
-    const auto P = A.p;
-    double E = ordered_sum(C.n, lane, [&](int q) {
-        double a = P[q].vx;
-        return 0.5 * P[q].m * (a * a + P[q].vy * P[q].vy);
-    });
-    for (int q = lane; q < C.n; q += 64) {
-        EdmdPart r = A.p[q];
-        r.coll = r.coll + 1;
-        if (G) fly_grow(C, t, r.x, r.y, r.vx, r.vy, r.tl, r.rad, A.vr[q]);
-        else fly_v<W>(C, t, r.x, r.y, r.vx, r.vy, r.tl);
-        r.vx /= sqrt(E / C.n / C.temperature);
-        r.vy /= sqrt(E / C.n / C.temperature);
-        A.p[q] = r;
-    }
-    WAVE_SYNC();
-    bool ov = false;
-    /* per particle: crossing, then collision (EDMD.c:4909-4915) */
-    for (int q = lane; q < C.n; q += 64)
-        ov |= sweep_one<G, W>(C, A, t, q, R.paul, R.ctr + 2 * (int64_t)q, R.ctr + 2 * (int64_t)q + 1);
-    R.ctr += 2 * (int64_t)C.n;
-    const bool any_ov = __ballot(ov) != 0ull;
-    WAVE_SYNC();
-    rebuild_tree(C, A, lane);
-    top_load(C, A, lane, R.q->top);
-    const int64_t wk = window_of(t + C.dtnoise, R.paul, C.dtp, C.nlists, R.win);
-    const int64_t rk = take_rank(C, R, t + C.dtnoise);
-    if (lane == 0) {
-        A.st->next_noise = t + C.dtnoise;
-        A.st->rank_noise = rk;
-        A.st->win_noise = wk;
-    }
-    WAVE_SYNC();
-    return any_ov;
-}
-
-__device__ __forceinline__ void flag_overlap(LoopRegs& R, bool ov, int p) {
-    if (__ballot(ov) != 0ull && R.status == EDMD_DEV_OK) {
-        R.status = EDMD_DEV_OVERLAP;
-        R.err_i = p;
-    }
-}
-
-template <int ML, bool W, class AR>
-__device__ __forceinline__ void ev_collision(const EdmdConst& C, const AR& A, int lane, LoopRegs& R, int i,
-                             int j) {
-    /* doTheCollisionNormal, EDMD.c:3542-3562, 3583-3606, 3802-3827, 3869-3879 */
-    const EdmdEv ei = A.e[i];
-    const int64_t rxi_old = A.erank[2 * i + 1]; /* crossing slot kept by a stale pop */
-    const EdmdPart pi = A.p[i];
-    const EdmdPart pj = A.p[j];
-    PathCache<ML> P;
-    path_prefetch<ML>(C, A, lane, i, j, P);
-    const double t = R.t;
-    double xi = uni(pi.x), yi = uni(pi.y), vxi = uni(pi.vx), vyi = uni(pi.vy), tli = uni(pi.tl);
-    const double ri = uni(pi.rad), mi = uni(pi.m);
-    const int cxi = uni((int)pi.cx), cyi = uni((int)pi.cy);
-    const uint32_t colli = (uint32_t)uni((int)pi.coll);
-    const uint32_t collj = (uint32_t)uni((int)pj.coll);
-    const uint32_t ca = (uint32_t)uni((int)ei.cact);
-
-    fly_v<W>(C, t, xi, yi, vxi, vyi, tli);
-    xi = uni(xi);
-    yi = uni(yi);
-    vxi = uni(vxi);
-    vyi = uni(vyi);
-    const bool valid = (ca == collj);
-    trace_push(C, A, lane, t, EDMD_EV_COLLISION, i, j, valid ? 1 : 0);
-    if (!valid) {
-        /* stale prediction: free flight of i and a new collision slot */
-        if (lane == 0) {
-            A.p[i].x = xi;
-            A.p[i].y = yi;
-            A.p[i].vx = vxi;
-            A.p[i].vy = vyi;
-            A.p[i].tl = t;
-        }
-        WAVE_SYNC();
-        const Owner oi{i, xi, yi, vxi, vyi, ri, cxi, cyi};
-        bool ov = false;
-        double dt, dtb;
-        int pa, pb;
-        uint32_t cpa, cpb;
-        predict_owners<false, W, (ML > 2 && !W)>(C, A, lane, t, 1, oi, oi, dt, pa, cpa, dtb, pb, cpb,
-                                                 ov, R.q->cand);
-        flag_overlap(R, ov, i);
-        const double tk = t + dt;
-        const double tci = uni(ei.tcross);
-        const int64_t rci = uni64(rxi_old);
-        const int diri = uni(ei.dir);
-        const int64_t rk = take_rank(C, R, tk);
-        if (lane == 0) {
-            A.e[i].tcoll = tk;
-            A.e[i].partner = pa;
-            A.e[i].cact = cpa;
-            A.erank[2 * i] = rk;
-        }
-        path_update<ML>(C, A, lane, P, i, make_leaf(tk, rk, tci, rci, pa, diri), -1, Leaf{}, R.q->top, R.t);
-        return;
-    }
-    R.ncol++;
-    double xj = uni(pj.x), yj = uni(pj.y), vxj = uni(pj.vx), vyj = uni(pj.vy), tlj = uni(pj.tl);
-    const double rj = uni(pj.rad), mj = uni(pj.m);
-    const int cxj = uni((int)pj.cx), cyj = uni((int)pj.cy);
-    fly_v<W>(C, t, xj, yj, vxj, vyj, tlj);
-    vxj = uni(vxj);
-    vyj = uni(vyj);
-    double dx = xj - xi;
-    double dy = yj - yi;
-    double dvx = vxj - vxi;
-    double dvy = vyj - vyi;
-    double inv_mass = 1 / (mi + mj);
-    min_image(C, dx, dy);
-    double kernel = inv_mass * (1 + C.res) * (dx * dvx + dy * dvy);
-    double ff = kernel / (4 * ri * rj);
-    double w = mi * mj * ff;
-    vxi = uni(vxi + ff * mj * dx);
-    vyi = uni(vyi + ff * mj * dy);
-    vxj = uni(vxj - ff * mi * dx);
-    vyj = uni(vyj - ff * mi * dy);
-    xj = uni(xj);
-    yj = uni(yj);
-    if (lane == 0) {
-        double* vir = R.q->vir;
-        vir[0] += w * dx * dx;
-        vir[1] += w * dy * dy;
-        vir[2] += w * dx * dy;
-        vir[3] += w * dy * dx;
-        EdmdState* st = A.st;
-        auto q = A.p + i;
-        q->x = xi; q->y = yi; q->vx = vxi; q->vy = vyi; q->tl = t; q->coll = colli + 1;
-        q = A.p + j;
-        q->x = xj; q->y = yj; q->vx = vxj; q->vy = vyj; q->tl = t; q->coll = collj + 1;
-        if (C.tape_cap > 0) {
-            const int64_t k = st->ntape;
-            if (k < C.tape_cap) {
-                EdmdTapeRec rec;
-                rec.t = t; rec.ax = dx; rec.ay = dy; rec.cx = dvx; rec.cy = dvy; rec.ff = ff;
-                rec.i = i; rec.j = j; rec.g = 0;
-                A.tape[k] = rec;
-            }
-            st->ntape = k + 1;
-            st->wsum += w * (dx * dx + dy * dy);
-            st->tlast = t;
-        }
-    }
-    WAVE_SYNC();
-    const Owner oi{i, xi, yi, vxi, vyi, ri, cxi, cyi};
-    const Owner oj{j, xj, yj, vxj, vyj, rj, cxj, cyj};
-    bool ov = false;
-    double dti, dtj;
-    int pi_, pj_;
-    uint32_t cpi, cpj;
-    predict_owners<false, W, (ML > 2 && !W)>(C, A, lane, t, 2, oi, oj, dti, pi_, cpi, dtj, pj_, cpj,
-                                             ov, R.q->cand);
-    flag_overlap(R, ov, i);
-    double tci2, tcj2;
-    int di, dj;
-    cross_time<W>(C, t, xi, yi, vxi, vyi, cxi, cyi, tci2, di);
-    cross_time<W>(C, t, xj, yj, vxj, vyj, cxj, cyj, tcj2, dj);
-    const double tki = t + dti, tkj = t + dtj;
-    /* insertion order, EDMD.c:3869-3879: crossings of i and j, then the
-     * collisions of i and j */
-    const int64_t rxi = take_rank(C, R, tci2);
-    const int64_t rxj = take_rank(C, R, tcj2);
-    const int64_t rki = take_rank(C, R, tki);
-    const int64_t rkj = take_rank(C, R, tkj);
-    if (lane == 0) {
-        EdmdEv e;
-        e.tcoll = tki; e.tcross = tci2; e.partner = pi_; e.cact = cpi; e.dir = di; e.pad = 0;
-        A.e[i] = e;
-        e.tcoll = tkj; e.tcross = tcj2; e.partner = pj_; e.cact = cpj; e.dir = dj;
-        A.e[j] = e;
-        A.erank[2 * i] = rki;
-        A.erank[2 * i + 1] = rxi;
-        A.erank[2 * j] = rkj;
-        A.erank[2 * j + 1] = rxj;
-    }
-    path_update<ML>(C, A, lane, P, i, make_leaf(tki, rki, tci2, rxi, pi_, di), j,
-                    make_leaf(tkj, rkj, tcj2, rxj, pj_, dj), R.q->top, R.t);
-}
-
-template <int ML, class AR>
-__device__ __forceinline__ void ev_collision_grow(const EdmdConst& C, const AR& A, int lane, LoopRegs& R,
-                                  int i, int j) {
-    /* doTheCollisionGrow, EDMD.c:3465-3540 (2D): both disks fly with their
-     * radii growing; the unit contact normal and the summed growth speed
-     * enter the impulse; res and delta are the compile-time 1 and 0 of
-     * EDMD.c:3467-3468; no virial. */
-    const double delta = 0.1 * 0;
-    const double res = 0.75 * 0 + 1;
-    const EdmdEv ei = A.e[i];
-    const int64_t rxi_old = A.erank[2 * i + 1]; /* crossing slot kept by a stale pop */
-    const EdmdPart pi = A.p[i];
-    const EdmdPart pj = A.p[j];
-    const double vri = uni(A.vr[i]), vrj = uni(A.vr[j]);
-    PathCache<ML> P;
-    path_prefetch<ML>(C, A, lane, i, j, P);
-    const double t = R.t;
-    double xi = uni(pi.x), yi = uni(pi.y), vxi = uni(pi.vx), vyi = uni(pi.vy), tli = uni(pi.tl);
-    double ri = uni(pi.rad);
-    const double mi = uni(pi.m);
-    const int cxi = uni((int)pi.cx), cyi = uni((int)pi.cy);
-    const uint32_t colli = (uint32_t)uni((int)pi.coll);
-    const uint32_t collj = (uint32_t)uni((int)pj.coll);
-    const uint32_t ca = (uint32_t)uni((int)ei.cact);
-
-    fly_grow(C, t, xi, yi, vxi, vyi, tli, ri, vri);
-    xi = uni(xi);
-    yi = uni(yi);
-    ri = uni(ri);
-    const bool valid = (ca == collj);
-    trace_push(C, A, lane, t, EDMD_EV_COLLISION, i, j, valid ? 1 : 0);
-    if (!valid) {
-        if (lane == 0) {
-            A.p[i].x = xi;
-            A.p[i].y = yi;
-            A.p[i].tl = t;
-            A.p[i].rad = ri;
-        }
-        WAVE_SYNC();
-        const Owner oi{i, xi, yi, vxi, vyi, ri, cxi, cyi, vri};
-        bool ov = false;
-        double dt, dtb;
-        int pa, pb;
-        uint32_t cpa, cpb;
-        predict_owners<true>(C, A, lane, t, 1, oi, oi, dt, pa, cpa, dtb, pb, cpb, ov, R.q->cand);
-        flag_overlap(R, ov, i);
-        const double tk = t + dt;
-        const double tci = uni(ei.tcross);
-        const int64_t rci = uni64(rxi_old);
-        const int diri = uni(ei.dir);
-        const int64_t rk = take_rank(C, R, tk);
-        if (lane == 0) {
-            A.e[i].tcoll = tk;
-            A.e[i].partner = pa;
-            A.e[i].cact = cpa;
-            A.erank[2 * i] = rk;
-        }
-        path_update<ML>(C, A, lane, P, i, make_leaf(tk, rk, tci, rci, pa, diri), -1, Leaf{}, R.q->top, R.t);
-        return;
-    }
-    R.ncol++;
-    double xj = uni(pj.x), yj = uni(pj.y), vxj = uni(pj.vx), vyj = uni(pj.vy), tlj = uni(pj.tl);
-    double rj = uni(pj.rad);
-    const double mj = uni(pj.m);
-    const int cxj = uni((int)pj.cx), cyj = uni((int)pj.cy);
-    fly_grow(C, t, xj, yj, vxj, vyj, tlj, rj, vrj);
-    double dx = xj - xi;
-    double dy = yj - yi;
-    double dvx = vxj - vxi;
-    double dvy = vyj - vyi;
-    double dvr = vri + vrj;
-    min_image(C, dx, dy);
-    double dist = sqrt(dx * dx + dy * dy);
-    double dxr = dx / dist;
-    double dyr = dy / dist;
-    double inv_mass = 1 / (mi + mj);
-    double kernel = inv_mass * (1 + res) * (dxr * dvx + dyr * dvy - dvr);
-    vxi = uni(vxi + (kernel * mj * dxr - 2 * mj * inv_mass * delta * dxr));
-    vyi = uni(vyi + (kernel * mj * dyr - 2 * mj * inv_mass * delta * dyr));
-    vxj = uni(vxj - (kernel * mi * dxr - 2 * mi * inv_mass * delta * dxr));
-    vyj = uni(vyj - (kernel * mi * dyr - 2 * mi * inv_mass * delta * dyr));
-    xj = uni(xj);
-    yj = uni(yj);
-    rj = uni(rj);
-    if (lane == 0) {
-        auto q = A.p + i;
-        q->x = xi; q->y = yi; q->vx = vxi; q->vy = vyi; q->tl = t; q->rad = ri; q->coll = colli + 1;
-        q = A.p + j;
-        q->x = xj; q->y = yj; q->vx = vxj; q->vy = vyj; q->tl = t; q->rad = rj; q->coll = collj + 1;
-    }
-    WAVE_SYNC();
-    const Owner oi{i, xi, yi, vxi, vyi, ri, cxi, cyi, vri};
-    const Owner oj{j, xj, yj, vxj, vyj, rj, cxj, cyj, vrj};
-    bool ov = false;
-    double dti, dtj;
-    int pi_, pj_;
-    uint32_t cpi, cpj;
-    predict_owners<true>(C, A, lane, t, 2, oi, oj, dti, pi_, cpi, dtj, pj_, cpj, ov, R.q->cand);
-    flag_overlap(R, ov, i);
-    double tci2, tcj2;
-    int di, dj;
-    cross_time<false>(C, t, xi, yi, vxi, vyi, cxi, cyi, tci2, di);
-    cross_time<false>(C, t, xj, yj, vxj, vyj, cxj, cyj, tcj2, dj);
-    const double tki = t + dti, tkj = t + dtj;
-    /* insertion order, EDMD.c:3869-3879: crossings of i and j, then the
-     * collisions of i and j */
-    const int64_t rxi = take_rank(C, R, tci2);
-    const int64_t rxj = take_rank(C, R, tcj2);
-    const int64_t rki = take_rank(C, R, tki);
-    const int64_t rkj = take_rank(C, R, tkj);
-    if (lane == 0) {
-        EdmdEv e;
-        e.tcoll = tki; e.tcross = tci2; e.partner = pi_; e.cact = cpi; e.dir = di; e.pad = 0;
-        A.e[i] = e;
-        e.tcoll = tkj; e.tcross = tcj2; e.partner = pj_; e.cact = cpj; e.dir = dj;
-        A.e[j] = e;
-        A.erank[2 * i] = rki;
-        A.erank[2 * i + 1] = rxi;
-        A.erank[2 * j] = rkj;
-        A.erank[2 * j + 1] = rxj;
-    }
-    path_update<ML>(C, A, lane, P, i, make_leaf(tki, rki, tci2, rxi, pi_, di), j,
-                    make_leaf(tkj, rkj, tcj2, rxj, pj_, dj), R.q->top, R.t);
-}
-
-/* stopGrow, EDMD.c:4740-4785 (2D, no wells): final flight with growth, all
- * counters and image counters reset, normalizePhysicalQ (EDMD.c:5723-5764:
- * remove the mean momentum, scale to E/N = Einit), then the Normal
- * prediction of every disk with stopGrow's partner counters, and a new
- * calendar.  The caller continues in the Normal loop. */
-template <bool W, class AR>
-__device__ __forceinline__ bool ev_stop_grow(const EdmdConst& C, const AR& A, int lane,
-                                             LoopRegs& R) {
-    const double t = R.t;
-    for (int q = lane; q < C.n; q += 64) {
-        EdmdPart r = A.p[q];
-        fly_grow(C, t, r.x, r.y, r.vx, r.vy, r.tl, r.rad, A.vr[q]);
-        r.coll = 0;
-        A.p[q] = r;
-        A.img[2 * q] = 0;
-        A.img[2 * q + 1] = 0;
-    }
-    WAVE_SYNC();
-    const auto P = A.p;
-    const int n = C.n;
-    if (!(W && (C.walls & 4))) {
-        const double px = ordered_sum(n, lane, [&](int q) { return P[q].vx * P[q].m; });
-        const double py = ordered_sum(n, lane, [&](int q) { return P[q].vy * P[q].m; });
-        for (int q = lane; q < n; q += 64) {
-            const double m = P[q].m;
-            P[q].vx -= px / (n * m);
-            P[q].vy -= py / (n * m);
-        }
-    } else {
-        /* in a circle, the angular momentum about the centre
-         * (EDMD.c:5730-5749): dvT accumulates -m (x0 vy - y0 vx), dvM m r */
-        const double h = C.halfLx;
-        const double dvT = -ordered_sum(n, lane, [&](int q) {
-            return P[q].m * (-P[q].vx * (P[q].y - h) + P[q].vy * (P[q].x - h));
-        });
-        const double dvM = ordered_sum(n, lane, [&](int q) {
-            return P[q].m * sqrt((P[q].x - h) * (P[q].x - h) + (P[q].y - h) * (P[q].y - h));
-        });
-        const double dv = dvT / dvM;
-        for (int q = lane; q < n; q += 64) {
-            const double x0 = P[q].x - h, y0 = P[q].y - h;
-            const double r = sqrt(x0 * x0 + y0 * y0);
-            P[q].vx += -dv * y0 / r;
-            P[q].vy += dv * x0 / r;
-        }
-    }
-    WAVE_SYNC();
-    const double E = ordered_sum(n, lane, [&](int q) {
-        double a = P[q].vx;
-        return 0.5 * P[q].m * (a * a + P[q].vy * P[q].vy);
-    });
-    for (int q = lane; q < n; q += 64) {
-        P[q].vx /= sqrt(E / n / C.einit);
-        P[q].vy /= sqrt(E / n / C.einit);
-        P[q].coll = 1;
-    }
-    WAVE_SYNC();
-    bool ov = false;
-    /* per particle: collision, then crossing (EDMD.c:4770-4776) */
-    for (int q = lane; q < n; q += 64)
-        ov |= sweep_one<false, W>(C, A, t, q, R.paul, R.ctr + 2 * (int64_t)q + 1,
-                               R.ctr + 2 * (int64_t)q, true);
-    R.ctr += 2 * (int64_t)n;
-    WAVE_SYNC();
-    const bool any_ov = __ballot(ov) != 0ull;
-    rebuild_tree(C, A, lane);
-    top_load(C, A, lane, R.q->top);
-    if (lane == 0) {
-        A.st->growing = 0;
-        A.st->next_grow = INF_D;
-    }
-    WAVE_SYNC();
-    return any_ov;
-}
-
+/* A particle event of the serial loop (doTheCollisionNormal / Grow,
+ * EDMD.c:3465-3915, doTheCrossing, EDMD.c:2501-2590, doTheWallNormal / Grow,
+ * EDMD.c:3333-3460): p's leaf holds the current time and code aux.  Returns
+ * the kind of event handled (EDMD_EV_*). */
 template <int ML, bool G, bool W, class AR>
-__device__ __forceinline__ void ev_single(const EdmdConst& C, const AR& A, int lane, LoopRegs& R, int p,
-                          int d) {
-    /* The events that change one disk.  d = 1-4: a cell crossing in that
-     * direction (doTheCrossing, EDMD.c:2501-2590; its freeFly is the
-     * dispatch pointer, freeFlyGrow while growing).  d = 5 + xy: a wall hit
-     * (doTheWallNormal, EDMD.c:3384-3460, without thermal or shear walls;
-     * doTheWallGrow while growing): counted as a collision, the momentum
-     * given to the wall accumulated for the thermo row, the normal velocity
-     * reversed times resW and the tangential one scaled by resT, a flat
-     * wall's hit written to the tape when taping.  Both then predict the
-     * crossing slot and the collision slot again, in that order. */
-    const bool wall = W && d >= 5;
-    const EdmdPart pp = A.p[p];
-    const double gvr = G ? uni(A.vr[p]) : 0.0;
+__device__ __forceinline__ int ev_particle(const EdmdConst& C, const AR& A, int lane, LoopRegs& R,
+                                           int p, int aux) {
+    /* what follows from the lane alone is made again for each event, not
+     * held in registers through the loop */
+    asm volatile("" : "+v"(lane));
     PathCache<ML> P;
-    path_prefetch<ML>(C, A, lane, p, -1, P);
+    path_prefetch<ML>(C, A, lane, p, aux >= 0 ? aux : -1, P);
     const double t = R.t;
-    double x = uni(pp.x), y = uni(pp.y), tl = uni(pp.tl);
-    double vx = uni(pp.vx), vy = uni(pp.vy);
-    double r = uni(pp.rad);
-    int cx = uni((int)pp.cx), cy = uni((int)pp.cy);
-    trace_push(C, A, lane, t, wall ? EDMD_EV_WALL : EDMD_EV_CELLCROSS, p, wall ? d - 5 : d, 1);
-    if (G) {
-        fly_grow(C, t, x, y, vx, vy, tl, r, gvr);
-        r = uni(r);
-    } else {
-        fly_v<W>(C, t, x, y, vx, vy, tl);
-    }
-    x = uni(x);
-    y = uni(y);
-    vx = uni(vx);
-    vy = uni(vy);
-
-    if (wall && G) {
-        /* doTheWallGrow, EDMD.c:3333-3382: a collision, no momentum to the
-         * wall; the normal velocity turned away with 2 vr added (for y,
-         * which way by the disk's height) */
-        R.ncol++;
-        if (d == 5) {
-            const double sg = vx < 0 ? -1.0 : (vx > 0 ? 1.0 : 0.0);
-            vx = -sg * (fabs(vx) + 2 * gvr);
-        } else if (d == 6) {
-            if (y > C.Ly - 3) vy = -vy - 2 * gvr;
-            else vy = -vy + 2 * gvr;
-        } else {
-            /* the circle: reflected about the normal, 2 vr added along it */
-            double nx, ny;
-            edmd_sincos(edmd_atan2(y - C.halfLx, x - C.halfLx), ny, nx);
-            const double mix = -(1 + C.res_wall) * (vx * nx + vy * ny);
-            vx += (mix - 2 * gvr) * nx;
-            vy += (mix - 2 * gvr) * ny;
-        }
-        vx = uni(vx);
-        vy = uni(vy);
-        if (lane == 0) {
-            const auto q = A.p + p;
-            q->x = x;
-            q->y = y;
-            q->tl = tl;
-            q->vx = vx;
-            q->vy = vy;
-            q->rad = r;
-            q->coll = pp.coll + 1;
-        }
-        WAVE_SYNC();
-    } else if (wall) {
-        R.ncol++;
-        const double m = uni(pp.m);
-        double dp;
-        /* the tangential product is made +0.0 where it is -0.0 (resT = 0
-         * times a negative velocity): the reference's crossing prediction
-         * divides by a -0.0 velocity and flies the disk to t = -inf */
-        double dpl = 0, dpm = 0, dpr = 0;
-        const double vx0 = vx, vy0 = vy; /* before the hit, for the tape */
-        if (d == 5) {
-            dp = fabs((C.res_wall + 1) * m * vx);
-            if (C.walls & 8) {
-                /* EDMD.c:3393-3409: the side walls within 3 of the box's edges */
-                if (vx < 0) {
-                    if (x - 3 < 0) dpl = dp;
-                    else dpm = dp;
-                } else {
-                    if (x + 3 > C.Lx) dpr = dp;
-                    else dpm = dp;
-                }
-            }
-            if (C.thermal_wall) {
-                /* thermoWall (EDMD.c:3411-3413): the normal speed drawn */
-                vx = -ref_sign(vx) * mt_drand0(A, lane, C.temperature / m);
-            } else {
-                vx = -C.res_wall * vx;
-                vy = C.res_tan * vy + 0.0;
-            }
-        } else if (d == 6) {
-            dp = fabs((C.res_wall + 1) * m * vy);
-            if (C.thermal_wall) {
-                vy = -ref_sign(vy) * mt_drand0(A, lane, C.temperature / m);
-            } else {
-                vy = -C.res_wall * vy;
-                vx = C.res_tan * vx + 0.0;
-            }
-            /* addShearWall (EDMD.c:3429-3439, without the delta model's
-             * kick): the top wall drives +0.1 along x, the bottom -0.1 */
-            if (C.shear_wall) vx = (y + 2 * r > C.Ly) ? 0.1 : -0.1;
-        } else {
-            /* the circle (EDMD.c:3441-3454): the normal velocity reversed
-             * times resW (thermal: both components drawn), |m mix| to the
-             * wall */
-            double nx, ny;
-            edmd_sincos(edmd_atan2(y - C.halfLx, x - C.halfLx), ny, nx);
-            const double mix = -(1 + C.res_wall) * (vx * nx + vy * ny);
-            if (C.thermal_wall) {
-                vx = -nx * mt_drand0(A, lane, C.temperature);
-                vy = -ny * mt_drand0(A, lane, C.temperature);
-            } else {
-                vx += mix * nx;
-                vy += mix * ny;
-            }
-            dp = fabs(m * mix);
-        }
-        vx = uni(vx);
-        vy = uni(vy);
-        if (lane == 0) {
-            A.st->dpw += dp;
-            if (C.walls & 8) {
-                A.st->dpl += dpl;
-                A.st->dpm += dpm;
-                A.st->dpr += dpr;
-            }
-            if (C.tape_cap > 0 && d != 7) {
-                /* a flat wall's record: j = -1 - xy, the normal and
-                 * tangential velocities before the hit, resW, resT and the
-                 * contact coordinate */
-                EdmdState* st = A.st;
-                const int64_t k = st->ntape;
-                if (k < C.tape_cap) {
-                    EdmdTapeRec rec;
-                    rec.t = t;
-                    rec.ax = d == 5 ? vx0 : vy0;
-                    rec.ay = d == 5 ? vy0 : vx0;
-                    rec.cx = C.res_wall;
-                    rec.cy = C.res_tan;
-                    rec.ff = d == 5 ? x : y;
-                    rec.i = p;
-                    rec.j = d == 5 ? -1 : -2;
-                    rec.g = C.field_on ? C.field : 0.0;
-                    A.tape[k] = rec;
-                }
-                st->ntape = k + 1;
-            }
-            const auto q = A.p + p;
-            q->x = x;
-            q->y = y;
-            q->tl = tl;
-            q->vx = vx;
-            q->vy = vy;
-            q->coll = pp.coll + 1;
-        }
-        WAVE_SYNC();
-    } else {
-        /* removeFromCell: drop p, keeping the order of the others */
-        const int c0 = cy * C.ncx + cx;
-        const int n0 = A.ccnt[c0];
-        int v = (lane < n0) ? A.cslot[(size_t)c0 * C.cap + lane] : -1;
-        uint64_t hit = __ballot(v == p);
-        int pos = hit ? (int)__builtin_ctzll(hit) : n0;
-        if (lane > pos && lane < n0) A.cslot[(size_t)c0 * C.cap + lane - 1] = v;
-        if (lane == 0) A.ccnt[c0] = n0 - 1;
-
-        int wx = 0, wy = 0; /* periodic image change */
-        switch (d) {
-            case 1:
-                if (cx - 1 == -1) { cx = C.ncx - 1; wx = -1; } else cx -= 1;
-                break;
-            case 2:
-                if (cx + 1 == C.ncx) { cx = 0; wx = 1; } else cx += 1;
-                break;
-            case 3:
-                if (cy - 1 == -1) { cy = C.ncy - 1; wy = -1; } else cy -= 1;
-                break;
-            default:
-                if (cy + 1 == C.ncy) { cy = 0; wy = 1; } else cy += 1;
-                break;
-        }
-        WAVE_SYNC();
-        const int c1 = cy * C.ncx + cx;
+    EvState S;
+    event_open<G, W>(C, A, lane, t, p, aux, S);
+    const bool wall = W && S.kind == EVK_WALL;
+    trace_push(C, A, lane, t,
+               aux >= 0 ? EDMD_EV_COLLISION : (wall ? EDMD_EV_WALL : EDMD_EV_CELLCROSS), p,
+               aux >= 0 ? aux : S.d, S.kind != EVK_STALE);
+    if (S.kind == EVK_COLLISION || wall) R.ncol++;
+    event_store(A, lane, t, S);
+    if (S.kind == EVK_CROSSING) {
+        event_cells(C, A, lane, S);
+        const int c1 = S.cy * C.ncx + S.cx;
         const int n1 = A.ccnt[c1];
         if (n1 >= C.cap) {
             if (R.status == EDMD_DEV_OK) {
@@ -1006,156 +610,204 @@ __device__ __forceinline__ void ev_single(const EdmdConst& C, const AR& A, int l
                 R.err_i = p;
                 R.err_j = c1;
             }
-            return;
+            return EDMD_EV_CELLCROSS;
         }
-        if (lane == 0) {
-            A.cslot[(size_t)c1 * C.cap + n1] = p; /* newest entry: visited first */
-            A.ccnt[c1] = n1 + 1;
-            const auto q = A.p + p;
-            q->x = x;
-            q->y = y;
-            q->tl = tl;
-            if (W) { /* changed by the flight under the field or damping */
-                q->vx = vx;
-                q->vy = vy;
-            }
-            if (G) q->rad = r;
-            q->cx = (int16_t)cx;
-            q->cy = (int16_t)cy;
-            if (wx) A.img[2 * p] += wx;
-            if (wy) A.img[2 * p + 1] += wy;
-        }
-        WAVE_SYNC();
+        event_enter(C, A, lane, S, n1);
+    } else if (S.kind != EVK_STALE) {
+        event_sums<G, W>(C, A, lane, t, S, p, aux, R.q->vir);
     }
-    const Owner o{p, x, y, vx, vy, r, cx, cy, gvr};
+    WAVE_SYNC();
+    event_predict<G, W, false>(C, A, lane, t, S, R.q->cand);
+    flag_overlap(R, S.ov, p);
+    int64_t rk, rx;
+    const Leaf L = event_ranks(C, lane, S, R.paul, R.ctr, rk, rx);
+    R.ctr += event_inserts(S);
+    event_slots(A, lane, S, L, rk, rx);
+    const double kA = lane_value(L.key, 0), kB = lane_value(L.key, 32);
+    const int xA = __builtin_amdgcn_readlane(L.aux, 0), xB = __builtin_amdgcn_readlane(L.aux, 32);
+    path_update<ML>(C, A, lane, P, p, kA, xA, S.nown == 2 ? aux : -1, kB, xB, R.q->top, t);
+    return aux >= 0 ? EDMD_EV_COLLISION : (wall ? EDMD_EV_WALL : EDMD_EV_CELLCROSS);
+}
+
+/* A reference the compiler cannot look through: what it loads through one
+ * is not kept in registers past the next.  The system's record does not
+ * change during a launch: constant memory, read with scalar loads. */
+template <class T>
+__device__ __forceinline__ const T& opaque_const(const T& r) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    typedef const T __attribute__((address_space(4))) * ConstPtr;
+    ConstPtr p = (ConstPtr)&r;
+    asm volatile("" : "+s"(p));
+    return *(const T*)p;
+#else
+    return r;
+#endif
+}
+__device__ __forceinline__ const EdmdConst& opaque(const EdmdConst& r) { return opaque_const(r); }
+__device__ __forceinline__ const EdmdArrays& opaque(const EdmdArrays& r) { return opaque_const(r); }
+template <class AR>
+__device__ __forceinline__ const AR& opaque(const AR& r) { return r; }
+
+/* A scheduled event (screenshot, thermo row, rescale, growth stop), the
+ * loop's registers handed over through its LDS state. */
+template <bool G, bool W, class AR>
+__device__ __forceinline__ void special_event(const EdmdConst& C, const AR& A, int lane,
+                                              QueueState* q, int sp) {
+    LoopRegs R;
+    R.q = q;
+    R.t = q->t;
+    R.paul = q->paul;
+    R.ctr = uni64(q->ctr);
+    R.win = uni64(q->win);
+    R.ncol = q->ncol;
     bool ov = false;
-    double dt, dtb;
-    int pa, pb;
-    uint32_t cpa, cpb;
-    predict_owners<G, W, (ML > 2 && !W)>(C, A, lane, t, 1, o, o, dt, pa, cpa, dtb, pb, cpb, ov,
-                                         R.q->cand);
-    flag_overlap(R, ov, p);
-    double tc;
-    int dir;
-    cross_time<W && !G>(C, t, x, y, vx, vy, cx, cy, tc, dir);
-    const double tk = t + dt;
-    /* crossingEvent(i), then collisionEvent(i), EDMD.c:2587-2589, 3458-3459 */
-    const int64_t rx = take_rank(C, R, tc);
-    const int64_t rk = take_rank(C, R, tk);
-    if (lane == 0) {
-        EdmdEv e;
-        e.tcoll = tk; e.tcross = tc; e.partner = pa; e.cact = cpa; e.dir = dir; e.pad = 0;
-        A.e[p] = e;
-        A.erank[2 * p] = rk;
-        A.erank[2 * p + 1] = rx;
+    if (sp == EDMD_EV_SCREENSHOT) {
+        ev_screenshot<64, G, W>(C, A, lane, R);
+    } else if (sp == EDMD_EV_THERMO) {
+        ev_thermo<64>(C, A, lane, R, q->vir, nullptr);
+    } else {
+        if (sp == EDMD_EV_GROWSTOP) ov = G && ev_stop_grow<64, W>(C, A, lane, R, nullptr);
+        else ov = ev_rescale<64, G, W>(C, A, lane, R, nullptr);
+        rebuild_tree(C, A, lane);
+        top_load(C, A, lane, q->top);
     }
-    path_update<ML>(C, A, lane, P, p, make_leaf(tk, rk, tc, rx, pa, dir), -1, Leaf{}, R.q->top, R.t);
+    WAVE_SYNC();
+    if (lane == 0) {
+        q->ctr = R.ctr;
+        if (ov && q->status == EDMD_DEV_OK) {
+            q->status = EDMD_DEV_OVERLAP;
+            if (sp == EDMD_EV_GROWSTOP) q->err_i = 0;
+        }
+        if (G && sp == EDMD_EV_GROWSTOP) {
+            q->ncol = 0; /* stopGrow resets ncol and ncross, EDMD.c:4745-4746 */
+            q->ncross = 0;
+        }
+    }
+    WAVE_SYNC();
 }
 
 /* Persistent event loop of one system on one wavefront; ML bounds the
  * calendar depth of every system in the launch.  A holds the system's arrays
  * in HBM (EdmdArrays) or in LDS (EdmdArraysL); the caller has checked that
- * the system's growth phase matches G. */
+ * the system's growth phase matches G.
+ *
+ * Particle events run in an inner loop of their own; a scheduled event
+ * leaves it, with the loop's registers and the system's record let go (the
+ * record is read again through an opaque reference), so that the scheduled
+ * events' sweeps and sums cost the inner loop no registers: with them in the
+ * same loop it spilled 61-106 scalar registers into vector ones. */
 template <int ML, bool G, bool W, int WPB = 1, class AR>
-__device__ __forceinline__ void run_loop(const EdmdConst& C, const AR& A, EdmdRunArgs ra) {
+__device__ __forceinline__ void run_loop(const EdmdConst& Cs, const AR& As, EdmdRunArgs ra) {
     /* WPB wavefronts per workgroup, each looping over its own system with
      * its own LDS queue state */
     const int lane = threadIdx.x & 63;
-    EdmdState* st = A.st;
     __shared__ QueueState Qs[WPB];
-    LoopRegs R;
-    R.q = &Qs[WPB > 1 ? wave_in_group() : 0];
-    R.t = uni(st->t);
-    R.ncol = st->ncol;
-    R.nevents = st->nevents;
-    R.status = st->status;
-    R.err_i = st->err_i;
-    R.err_j = st->err_j;
-    R.paul = uni(st->paul);
-    R.ctr = uni64(st->ctr);
-    R.win = uni64(st->win);
-    R.cur = uni((int)(R.win % C.nlists));
-    if (lane == 0)
-        for (int k = 0; k < 4; ++k) R.q->vir[k] = st->vir[k];
-    next_special(st, R);
-    top_load(C, A, lane, R.q->top);
-    uint64_t ncross = st->ncross;
+    QueueState* const q = &Qs[WPB > 1 ? wave_in_group() : 0];
     int reason = EDMD_STOP_NONE;
-    int last_type = st->last_type;
-
-    const int64_t ev_limit = st->ev_limit < ra.max_events ? st->ev_limit : ra.max_events;
-    const uint64_t coll_limit = st->coll_limit < ra.max_coll ? st->coll_limit : ra.max_coll;
-
+    {
+        const EdmdState* st = As.st;
+        if (lane == 0) {
+            q->t = st->t;
+            q->paul = st->paul;
+            q->ctr = st->ctr;
+            q->win = st->win;
+            q->ncol = st->ncol;
+            q->nevents = st->nevents;
+            q->ncross = st->ncross;
+            q->status = st->status;
+            q->err_i = st->err_i;
+            q->err_j = st->err_j;
+            q->last_type = st->last_type;
+            for (int k = 0; k < 4; ++k) q->vir[k] = st->vir[k];
+        }
+        top_load(Cs, As, lane, q->top);
+    }
+    WAVE_SYNC();
     for (;;) {
-        if (R.status != EDMD_DEV_OK) { reason = EDMD_STOP_ERROR; break; }
-        if ((int64_t)R.nevents >= ev_limit) { reason = EDMD_STOP_EVENTS; break; }
-        if (R.ncol >= coll_limit) { reason = EDMD_STOP_COLLISIONS; break; }
-        if (!(R.t <= ra.tmax)) { reason = EDMD_STOP_TIME; break; }
-        double key;
-        int p, aux;
-        top_min(C, A, lane, R.q->top, R.t, key, p, aux);
-        if (!(key < INF_D) && !(R.next_special < INF_D)) { reason = EDMD_STOP_EMPTY; break; }
-        if (pick_next(C, A, st, R, key, p, aux)) {
-            const int sp = R.special;
-            R.t = R.next_special;
-            trace_push(C, A, lane, R.t, sp, 0, 0, 1);
-            if (sp == EDMD_EV_SCREENSHOT) {
-                ev_screenshot<G, W>(C, A, lane, R);
-            } else if (sp == EDMD_EV_THERMO) {
-                ev_thermo(C, A, lane, R);
-            } else if (sp == EDMD_EV_GROWSTOP) {
-                if (G) {
-                    flag_overlap(R, ev_stop_grow<W>(C, A, lane, R), 0);
-                    R.ncol = 0; /* stopGrow resets ncol and ncross, EDMD.c:4745-4746 */
-                    ncross = 0;
-                }
-            } else {
-                if (ev_rescale<G, W>(C, A, lane, R) && R.status == EDMD_DEV_OK)
-                    R.status = EDMD_DEV_OVERLAP;
-            }
+        int sp = -1;
+        {
+            const EdmdConst& C = opaque(Cs);
+            const AR& A = opaque(As);
+            EdmdState* st = A.st;
+            LoopRegs R;
+            R.q = q;
+            R.t = q->t;
+            R.ncol = q->ncol;
+            R.nevents = q->nevents;
+            R.status = q->status;
+            R.err_i = q->err_i;
+            R.err_j = q->err_j;
+            R.paul = q->paul;
+            R.ctr = uni64(q->ctr);
+            R.win = uni64(q->win);
+            R.cur = (int)(R.win % C.nlists);
+            uint64_t ncross = q->ncross;
+            int last_type = q->last_type;
             next_special(st, R);
-            R.nevents++;
-            last_type = sp;
-            if (G && sp == EDMD_EV_GROWSTOP) { reason = EDMD_STOP_GROWN; break; }
-            if (ra.stop_mask & (1 << sp)) { reason = EDMD_STOP_SPECIAL; break; }
-            continue;
-        }
-        R.t = key;
-        if (aux >= 0) {
-            if (G) ev_collision_grow<ML>(C, A, lane, R, p, aux);
-            else ev_collision<ML, W>(C, A, lane, R, p, aux);
-            last_type = EDMD_EV_COLLISION;
-        } else {
-            /* a crossing (code -1..-4) or a wall hit (-5 - xy) */
-            const bool wall = W && aux <= EDMD_WALL_CODE(0);
-            ev_single<ML, G, W>(C, A, lane, R, p, wall ? 5 + EDMD_WALL_CODE(0) - aux : -aux);
-            if (wall) {
-                last_type = EDMD_EV_WALL;
-            } else {
-                ncross++;
-                last_type = EDMD_EV_CELLCROSS;
+            const int64_t ev_limit = st->ev_limit < ra.max_events ? st->ev_limit : ra.max_events;
+            const uint64_t coll_limit = st->coll_limit < ra.max_coll ? st->coll_limit : ra.max_coll;
+            for (;;) {
+                if (R.status != EDMD_DEV_OK) { reason = EDMD_STOP_ERROR; break; }
+                if ((int64_t)R.nevents >= ev_limit) { reason = EDMD_STOP_EVENTS; break; }
+                if (R.ncol >= coll_limit) { reason = EDMD_STOP_COLLISIONS; break; }
+                if (!(R.t <= ra.tmax)) { reason = EDMD_STOP_TIME; break; }
+                double key;
+                int p, aux;
+                top_min(C, A, lane, R.q->top, R.t, key, p, aux);
+                if (!(key < INF_D) && !(R.next_special < INF_D)) { reason = EDMD_STOP_EMPTY; break; }
+                if (pick_next(C, A, st, R, key, p, aux)) {
+                    sp = R.special;
+                    R.t = R.next_special;
+                    trace_push(C, A, lane, R.t, sp, 0, 0, 1);
+                    R.nevents++;
+                    last_type = sp;
+                    break;
+                }
+                R.t = key;
+                last_type = ev_particle<ML, G, W>(C, A, lane, R, p, aux);
+                if (last_type == EDMD_EV_CELLCROSS) ncross++;
+                R.nevents++;
+                if (ra.stop_mask & (1 << last_type)) { reason = EDMD_STOP_SPECIAL; break; }
             }
+            WAVE_SYNC();
+            if (lane == 0) {
+                q->t = R.t;
+                q->ncol = R.ncol;
+                q->nevents = R.nevents;
+                q->ncross = ncross;
+                q->status = R.status;
+                q->err_i = R.err_i;
+                q->err_j = R.err_j;
+                q->paul = R.paul;
+                q->ctr = R.ctr;
+                q->win = R.win;
+                q->last_type = last_type;
+            }
+            WAVE_SYNC();
         }
-        R.nevents++;
-        if (ra.stop_mask & (1 << last_type)) { reason = EDMD_STOP_SPECIAL; break; }
+        if (sp < 0) break;
+        special_event<G, W>(opaque(Cs), opaque(As), lane, q, sp);
+        if (G && sp == EDMD_EV_GROWSTOP) { reason = EDMD_STOP_GROWN; break; }
+        if (ra.stop_mask & (1 << sp)) { reason = EDMD_STOP_SPECIAL; break; }
     }
-
+    const AR& A = opaque(As);
     if (lane == 0) {
-        st->t = R.t;
-        st->ncol = R.ncol;
-        st->ncross = ncross;
-        st->nevents = R.nevents;
-        st->status = R.status;
-        st->err_i = R.err_i;
-        st->err_j = R.err_j;
+        EdmdState* st = A.st;
+        st->t = q->t;
+        st->ncol = q->ncol;
+        st->ncross = q->ncross;
+        st->nevents = q->nevents;
+        st->status = q->status;
+        st->err_i = q->err_i;
+        st->err_j = q->err_j;
         st->stop_reason = reason;
-        st->last_type = last_type;
-        st->paul = R.paul;
-        st->ctr = R.ctr;
-        st->win = R.win;
-        for (int k = 0; k < 4; ++k) st->vir[k] = R.q->vir[k];
+        st->last_type = q->last_type;
+        st->paul = q->paul;
+        st->ctr = q->ctr;
+        st->win = q->win;
+        for (int k = 0; k < 4; ++k) st->vir[k] = q->vir[k];
     }
-    top_store(C, A, lane, R.q->top);
+    top_store(opaque(Cs), A, lane, q->top);
 }
 
 #endif

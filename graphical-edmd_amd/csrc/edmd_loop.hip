@@ -17,6 +17,7 @@
  */
 #define EDMD_DEVICE_ARRAYS 1
 #include "edmd_loop.h"
+#include "edmd_lds.h"
 #include "edmd_variants.h"
 
 /* Systems of up to 64^2 disks (calendar depth <= 2): bounded to 128 VGPRs so
@@ -46,89 +47,6 @@ __global__ __launch_bounds__(64) void k_run(const EdmdSys* __restrict__ systems,
 
 /* ----------------------------------------------------- LDS-resident systems */
 
-#if defined(__HIP_DEVICE_COMPILE__)
-#define EDMD_LDS __attribute__((address_space(3)))
-#else
-#define EDMD_LDS
-#endif
-
-/* The arrays of a system whose event loop runs out of LDS.  Everything the
- * loop reads and writes on each event (particles, event slots, calendar
- * nodes, ranks, image counters, cell lists, growth rates) sits in the
- * workgroup's LDS for the whole launch; the per-system record and the
- * output buffers (trace, thermo rows, tape, derivative state) stay in HBM.
- * Fields mean what the fields of EdmdArrays of the same name mean. */
-struct EdmdArraysL {
-    EdmdPart EDMD_LDS* p;
-    EdmdEv EDMD_LDS* e;
-    EdmdNode EDMD_LDS* leaf;
-    EdmdNode EDMD_LDS* lev[EDMD_MAX_LEVELS];
-    int32_t EDMD_LDS* img;
-    int32_t EDMD_LDS* ccnt;
-    int32_t EDMD_LDS* cslot;
-    EdmdState EDMD_GLOBAL* st;
-    EdmdTraceRec EDMD_GLOBAL* trace;
-    EdmdThermoRow EDMD_GLOBAL* thermo;
-    double EDMD_LDS* vr;
-    int64_t EDMD_LDS* erank;
-    int64_t EDMD_LDS* lrank;
-    EdmdTapeRec EDMD_GLOBAL* tape;
-    double EDMD_GLOBAL* dv;
-    double EDMD_GLOBAL* dtl;
-    double EDMD_GLOBAL* otl;
-    EdmdDeriv EDMD_GLOBAL* dr;
-    int32_t EDMD_GLOBAL* ptype;
-    uint32_t EDMD_GLOBAL* mt;
-};
-
-/* Copies one array between HBM and LDS with the whole wavefront, in 16-,
- * 8- or 4-byte words as the HBM address and the length allow (LDS offsets
- * are 16-byte aligned; every length is a multiple of 4). */
-template <bool IN>
-__device__ __forceinline__ void lds_xfer(unsigned char EDMD_LDS* l, const void EDMD_GLOBAL* gv,
-                                         uint32_t bytes, int lane) {
-    unsigned char EDMD_GLOBAL* g = (unsigned char EDMD_GLOBAL*)gv;
-    const uint32_t al = uni((int)((uint32_t)(uintptr_t)g | bytes));
-    if ((al & 15) == 0) {
-        int4 EDMD_LDS* L = (int4 EDMD_LDS*)l;
-        int4 EDMD_GLOBAL* H = (int4 EDMD_GLOBAL*)g;
-        for (uint32_t i = lane; i < bytes / 16; i += 64) {
-            if (IN) L[i] = H[i]; else H[i] = L[i];
-        }
-    } else if ((al & 7) == 0) {
-        int2 EDMD_LDS* L = (int2 EDMD_LDS*)l;
-        int2 EDMD_GLOBAL* H = (int2 EDMD_GLOBAL*)g;
-        for (uint32_t i = lane; i < bytes / 8; i += 64) {
-            if (IN) L[i] = H[i]; else H[i] = L[i];
-        }
-    } else {
-        int EDMD_LDS* L = (int EDMD_LDS*)l;
-        int EDMD_GLOBAL* H = (int EDMD_GLOBAL*)g;
-        for (uint32_t i = lane; i < bytes / 4; i += 64) {
-            if (IN) L[i] = H[i]; else H[i] = L[i];
-        }
-    }
-}
-
-/* Moves a system's loop arrays into LDS (IN) or back to HBM (!IN); the
- * growth rates are read-only and only come in. */
-template <bool IN, bool G>
-__device__ __forceinline__ void lds_system(const EdmdConst& C, const EdmdArrays& H,
-                                           const EdmdArraysL& A, int lane) {
-    const uint32_t n = (uint32_t)C.n, ncell = (uint32_t)(C.ncx * C.ncy);
-    lds_xfer<IN>((unsigned char EDMD_LDS*)A.p, H.p, n * 64, lane);
-    lds_xfer<IN>((unsigned char EDMD_LDS*)A.e, H.e, n * 32, lane);
-    lds_xfer<IN>((unsigned char EDMD_LDS*)A.leaf, H.leaf, n * 16, lane);
-    for (int l = 0; l < C.nlev; l++)
-        lds_xfer<IN>((unsigned char EDMD_LDS*)A.lev[l], H.lev[l], (uint32_t)C.lsize[l + 1] * 16, lane);
-    lds_xfer<IN>((unsigned char EDMD_LDS*)A.erank, H.erank, n * 16, lane);
-    lds_xfer<IN>((unsigned char EDMD_LDS*)A.lrank, H.lrank, n * 8, lane);
-    lds_xfer<IN>((unsigned char EDMD_LDS*)A.img, H.img, n * 8, lane);
-    lds_xfer<IN>((unsigned char EDMD_LDS*)A.ccnt, H.ccnt, ncell * 4, lane);
-    lds_xfer<IN>((unsigned char EDMD_LDS*)A.cslot, H.cslot, ncell * (uint32_t)C.cap * 4, lane);
-    if (IN && G) lds_xfer<true>((unsigned char EDMD_LDS*)A.vr, H.vr, n * 8, lane);
-}
-
 /* One workgroup (one wavefront) per system with the system's loop arrays
  * resident in LDS: they come in from HBM when the launch starts, the event
  * loop runs on them, and they go back when it stops.  The dynamic LDS of
@@ -142,37 +60,16 @@ __global__ __launch_bounds__(64) void k_run_lds(const EdmdSys* __restrict__ syst
     const EdmdArrays& H = S.a;
     const int lane = threadIdx.x;
     if ((uni(H.st->growing) != 0) != G) return;
-    const EdmdLdsLayout L = edmd_lds_layout(&C, G ? 1 : 0);
-    unsigned char EDMD_LDS* base = (unsigned char EDMD_LDS*)lds_pool;
     /* the pointer table itself lives in LDS: the loop indexes lev[] with
      * run-time levels, which would put a register copy in scratch */
     __shared__ EdmdArraysL A;
-    A.p = (EdmdPart EDMD_LDS*)(base + L.p);
-    A.e = (EdmdEv EDMD_LDS*)(base + L.e);
-    A.leaf = (EdmdNode EDMD_LDS*)(base + L.leaf);
-    for (int l = 0; l < EDMD_MAX_LEVELS; l++) A.lev[l] = (EdmdNode EDMD_LDS*)(base + L.lev[l]);
-    A.img = (int32_t EDMD_LDS*)(base + L.img);
-    A.ccnt = (int32_t EDMD_LDS*)(base + L.ccnt);
-    A.cslot = (int32_t EDMD_LDS*)(base + L.cslot);
-    A.vr = (double EDMD_LDS*)(base + L.vr);
-    A.erank = (int64_t EDMD_LDS*)(base + L.erank);
-    A.lrank = (int64_t EDMD_LDS*)(base + L.lrank);
-    A.st = H.st;
-    A.trace = H.trace;
-    A.thermo = H.thermo;
-    A.tape = H.tape;
-    A.dv = H.dv;
-    A.dtl = H.dtl;
-    A.otl = H.otl;
-    A.dr = H.dr;
-    A.ptype = H.ptype;
-    A.mt = H.mt;
+    lds_carve<G>(C, H, (unsigned char EDMD_LDS*)lds_pool, A);
     WAVE_SYNC();
-    lds_system<true, G>(C, H, A, lane);
+    lds_system<true, G, 64>(C, H, A, lane);
     WAVE_SYNC();
     run_loop<ML, G, W>(C, A, ra);
     WAVE_SYNC();
-    lds_system<false, G>(C, H, A, lane);
+    lds_system<false, G, 64>(C, H, A, lane);
 }
 
 /* ------------------------------------------------------------ launchers */

@@ -193,6 +193,30 @@ static inline EDMD_HD EdmdLdsLayout edmd_lds_layout(const EdmdConst* c, int grow
     return L;
 }
 
+/* The wide loop's window: the calendar level it keeps in LDS.  The leaves
+ * themselves up to EDMD_WIDE_FLAT disks (20 bytes each: 120 KB), above that
+ * the level of 64-leaf or 4096-leaf groups (24 bytes a node); -1: the system
+ * is too large for it. */
+#define EDMD_WIDE_FLAT 6144
+#define EDMD_WIDE_NODES 4096
+#define EDMD_WIDE_PER_CU 2 /* systems a CU takes */
+/* Largest cell capacity the neighbour scan stages in LDS (six 16-byte row
+ * chunks per cell), and the stage: for each of two disks every slot of nine
+ * cells, and before it the room that the rows' unused slots are written to. */
+#define EDMD_STAGE_CAP 24
+#define EDMD_STAGE_HALF (10 * EDMD_STAGE_CAP)
+#define EDMD_STAGE_MAX (2 * EDMD_STAGE_HALF)
+static inline EDMD_HD int edmd_wide_level(const EdmdConst* c) {
+    if (c->n <= EDMD_WIDE_FLAT) return 0;
+    if (c->lsize[1] <= EDMD_WIDE_NODES) return 1;
+    if (c->nlev >= 2 && c->lsize[2] <= EDMD_WIDE_NODES) return 2;
+    return -1;
+}
+static inline EDMD_HD uint64_t edmd_wide_bytes(const EdmdConst* c) {
+    const int l = edmd_wide_level(c);
+    return l < 0 ? 0 : edmd_lds_align((uint64_t)c->lsize[l] * (l == 0 ? 20 : 24));
+}
+
 /* Per-system counters at the end of one epoch of a graph-captured run. */
 typedef struct EdmdEpochRow {
     double t;
