@@ -1740,6 +1740,8 @@ int edmd_internal_fail(int code, const char* msg) { return fail(code, "%s", msg)
 
 /* ------------------------------------------------------------ g(r) */
 
+static size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
+
 /* Histogram of one system or of host arrays, normalised as calculate_pcf
  * (pcf.c:16-75): g = 2 count / (2 pi r dr * (N / (Lx Ly)) * N). */
 static int pcf_common(const double* hx, const double* hy, const EdmdPart* dpart, int n, double t,
@@ -1753,25 +1755,42 @@ static int pcf_common(const double* hx, const double* hy, const EdmdPart* dpart,
         *nbins = nb;
         return fail(EDMD_ERR_ARG, "g(r) output arrays need %d entries", nb);
     }
-    double *dx = nullptr, *dy = nullptr;
-    unsigned long long* dh = nullptr;
-    HIPCHK(hipMalloc(&dh, (size_t)nb * sizeof(unsigned long long)));
-    hipError_t e = hipMemsetAsync(dh, 0, (size_t)nb * sizeof(unsigned long long), stream);
-    if (e == hipSuccess && hx) {
-        e = hipMalloc(&dx, (size_t)n * sizeof(double));
-        if (e == hipSuccess) e = hipMalloc(&dy, (size_t)n * sizeof(double));
-        if (e == hipSuccess) e = hipMemcpy(dx, hx, (size_t)n * sizeof(double), hipMemcpyHostToDevice);
-        if (e == hipSuccess) e = hipMemcpy(dy, hy, (size_t)n * sizeof(double), hipMemcpyHostToDevice);
-    }
-    if (e == hipSuccess)
-        e = edmd_launch_pcf(dx, dy, hx ? nullptr : dpart, n, t, extrap, Lx, Ly, dr, nb, dh, stream);
     std::vector<unsigned long long> cnt(nb);
-    if (e == hipSuccess) e = hipStreamSynchronize(stream);
+    std::vector<double> xy(hx && n <= 8192 ? 2 * (size_t)n : 0);
+    /* one allocation: counts, the host arrays' copies, the sort's scratch; where
+     * the card has no room for that scratch all pairs are taken instead */
+    const size_t cb = cnt.size() * sizeof(cnt[0]), hb = align256(cb);
+    const size_t pb = hx ? (size_t)n * sizeof(double) : 0, db = align256(2 * pb);
+    char* mem = nullptr;
+    bool sort = true;
+    if (hipMalloc(&mem, hb + db + edmd_pcf_scratch(n)) != hipSuccess) {
+        (void)hipGetLastError();
+        sort = false;
+        HIPCHK(hipMalloc(&mem, hb + db));
+    }
+    unsigned long long* dh = (unsigned long long*)mem;
+    double* dx = hx ? (double*)(mem + hb) : nullptr;
+    double* dy = hx ? dx + n : nullptr;
+    hipError_t e = hipSuccess;
+    if (hx && n <= 8192) { /* one copy: a copy's fixed cost passes that of joining the arrays */
+        memcpy(xy.data(), hx, pb);
+        memcpy(xy.data() + n, hy, pb);
+        e = hipMemcpy(dx, xy.data(), 2 * pb, hipMemcpyHostToDevice);
+    } else if (hx) {
+        e = hipMemcpy(dx, hx, pb, hipMemcpyHostToDevice);
+        if (e == hipSuccess) e = hipMemcpy(dy, hy, pb, hipMemcpyHostToDevice);
+    }
+    if (e == hipSuccess && !sort) e = hipMemsetAsync(dh, 0, cb, stream);
+    const EdmdPart* from = hx ? nullptr : dpart;
     if (e == hipSuccess)
-        e = hipMemcpy(cnt.data(), dh, (size_t)nb * sizeof(unsigned long long), hipMemcpyDeviceToHost);
-    (void)hipFree(dh);
-    if (dx) (void)hipFree(dx);
-    if (dy) (void)hipFree(dy);
+        e = sort ? edmd_launch_pcf_pairs(dx, dy, from, n, t, extrap, Lx, Ly, dr, nb, dh,
+                                         mem + hb + db, stream)
+                 : edmd_launch_pcf(dx, dy, from, n, t, extrap, Lx, Ly, dr, nb, dh, stream);
+    if (e == hipSuccess)
+        e = hipMemcpyAsync(cnt.data(), dh, cb, hipMemcpyDeviceToHost, stream);
+    if (e == hipSuccess) e = hipStreamSynchronize(stream);
+    else (void)hipStreamSynchronize(stream);
+    (void)hipFree(mem);
     if (e != hipSuccess) return fail(EDMD_ERR_HIP, "g(r) failed: %s", hipGetErrorString(e));
     const double pi = 3.14159265358979323846;
     const double volume = Lx * Ly;
@@ -1833,8 +1852,6 @@ static std::vector<PoolSpan> state_pools(edmd_batch* b) {
             {b->lrank, b->np * sizeof(int64_t)},
             {b->mt, b->mt ? (size_t)b->nsys * 625 * sizeof(uint32_t) : 0}};
 }
-
-static size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
 static size_t ckpt_bytes(edmd_batch* b) {
     size_t t = 0;

@@ -63,6 +63,12 @@ hipError_t edmd_launch_queue_edit(const EdmdSys* d_sys, int max_nlev, int kind, 
 hipError_t edmd_launch_pcf(const double* x, const double* y, const EdmdPart* part, int n, double t,
                            int extrap, double Lx, double Ly, double dr, int nb,
                            unsigned long long* hist, hipStream_t s);
+/* the same counts, set rather than added, with edmd_pcf_scratch(n) bytes of
+ * device memory for the sorted positions */
+size_t edmd_pcf_scratch(int n);
+hipError_t edmd_launch_pcf_pairs(const double* x, const double* y, const EdmdPart* part, int n,
+                                 double t, int extrap, double Lx, double Ly, double dr, int nb,
+                                 unsigned long long* hist, void* scratch, hipStream_t s);
 hipError_t edmd_launch_fp64_check(int n, const double* a, const double* b, double* q, double* sq,
                                   hipStream_t s);
 

@@ -6,7 +6,7 @@
  *                  per-system bounds and counters of graph-captured epochs
  *   k_peek, k_pair_time, k_repredict, k_queue_edit, k_fly_one
  *                  single steps for the reference-compatible entry points
- *   k_pcf          g(r) (pcf.c:16-75)
+ *   k_pcf          g(r) (pcf.c:16-75) of all pairs, without scratch memory
  *   k_fp64_check   IEEE division / square root probe for the tests
  *
  * Reference line numbers are those of src/EDMD.c.
@@ -213,7 +213,8 @@ __global__ void k_fly_one(const EdmdSys* __restrict__ systems, int i) {
 /* calculate_pcf, pcf.c:16-75: histogram of minimum-image pair distances
  * below rmax = dr * nb, one count per unordered pair (the reference adds
  * 2.0 per pair; the host doubles the counts).  Blocks take 256 x 256 tiles
- * of the upper pair triangle and count into an LDS histogram.  extrap != 0
+ * of the upper pair triangle and count into an LDS histogram.  For callers
+ * without scratch memory; k_pcf_pairs has the others.  extrap != 0
  * uses positions free-flown to time t without storing them. */
 __global__ __launch_bounds__(256) void k_pcf(const double* __restrict__ px,
                                             const double* __restrict__ py,
