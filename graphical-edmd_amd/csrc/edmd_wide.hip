@@ -1123,10 +1123,14 @@ __device__ __forceinline__ void wide_loop(const EdmdConst& Cs, const AR& As, Edm
 }
 
 /* LDS = false: the system's arrays in HBM, the calendar's window level in
- * the dynamic LDS; LDS = true: the arrays in LDS as well (edmd_lds.h). */
+ * the dynamic LDS; LDS = true: the arrays in LDS as well (edmd_lds.h).  Two
+ * wavefronts a SIMD: one workgroup of eight, or two of four; without the bound
+ * the compiler gave four wavefronts every register, and one CU held one
+ * workgroup (512 systems of 400 disks, 300000 events: 18 ms in the loop of one
+ * wavefront that ran instead, 12.3 ms here). */
 template <int NW, bool G, bool W>
-__global__ __launch_bounds__(64 * NW) void k_wide(const EdmdSys* __restrict__ systems,
-                                                  EdmdRunArgs ra) {
+__global__ __launch_bounds__(64 * NW, 2) void k_wide(const EdmdSys* __restrict__ systems,
+                                                     EdmdRunArgs ra) {
     extern __shared__ __align__(64) unsigned char lds_pool[];
     const EdmdSys& S = systems[blockIdx.x];
     if ((uni(S.a.st->growing) != 0) != G) return;
@@ -1134,8 +1138,8 @@ __global__ __launch_bounds__(64 * NW) void k_wide(const EdmdSys* __restrict__ sy
 }
 
 template <int NW, bool G, bool W>
-__global__ __launch_bounds__(64 * NW) void k_wide_lds(const EdmdSys* __restrict__ systems,
-                                                      EdmdRunArgs ra) {
+__global__ __launch_bounds__(64 * NW, 2) void k_wide_lds(const EdmdSys* __restrict__ systems,
+                                                         EdmdRunArgs ra) {
     extern __shared__ __align__(64) unsigned char lds_pool[];
     const EdmdSys& S = systems[blockIdx.x];
     if ((uni(S.a.st->growing) != 0) != G) return;
