@@ -11,6 +11,7 @@
 #include <string.h>
 
 #include <algorithm>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -158,6 +159,13 @@ struct edmd_batch {
     int wide_waves[2] = {0, 0};
     bool wide_lds[2] = {false, false};
     size_t wide_dyn[2] = {0, 0};
+    /* pinned host memory that results come back through (read_rows): two
+     * buffers of stage_half bytes, allocated by the first read */
+    std::mutex stage_lock;
+    char* stage = nullptr;
+    size_t stage_half = 0;
+    /* checkpoint memory that a new taping of the same shape takes over */
+    std::vector<void*> ckpt_free;
 };
 
 struct edmd_ctx {
@@ -183,6 +191,8 @@ static int dalloc(edmd_batch* b, T** p, size_t n) {
 static void deriv_release(edmd_batch* b) {
     for (auto& c : b->ckpts) (void)hipFree(c.mem);
     b->ckpts.clear();
+    for (void* p : b->ckpt_free) (void)hipFree(p);
+    b->ckpt_free.clear();
     if (b->ckpt_end) (void)hipFree(b->ckpt_end);
     b->ckpt_end = nullptr;
     for (void* p : b->dallocs) (void)hipFree(p);
@@ -198,6 +208,7 @@ static void batch_free(edmd_batch* b) {
     if (!b) return;
     deriv_release(b);
     for (void* p : b->allocs) (void)hipFree(p);
+    if (b->stage) (void)hipHostFree(b->stage);
     if (b->d_sys) (void)hipFree(b->d_sys);
     if (b->own_stream && b->stream) (void)hipStreamDestroy(b->stream);
     delete b;
@@ -330,70 +341,112 @@ static int setup_system(const edmd_system_desc* d, HostSys* h, int idx) {
     return EDMD_OK;
 }
 
-static int upload_system(edmd_batch* b, int s, const edmd_system_desc* d) {
+/* One pool's rows of systems in turn, sent in pieces of some 16 MB: a copy per
+ * system and array cost 10 us each. */
+template <class T>
+struct PoolUpload {
+    T* pool;
+    std::vector<T> rows;
+    size_t first = 0;
+    explicit PoolUpload(T* p) : pool(p) {}
+    /* room for rows [at, at + n); rows passed over are zero */
+    int add(size_t at, size_t n, T** out) {
+        if (!rows.empty() && rows.size() * sizeof(T) >= (16u << 20)) {
+            int rc = send();
+            if (rc) return rc;
+        }
+        if (rows.empty()) first = at;
+        rows.resize(at - first + n);
+        *out = rows.data() + (at - first);
+        return EDMD_OK;
+    }
+    int send() {
+        if (!rows.empty())
+            HIPCHK(hipMemcpy(pool + first, rows.data(), rows.size() * sizeof(T), hipMemcpyHostToDevice));
+        rows.clear();
+        return EDMD_OK;
+    }
+};
+
+struct Uploads {
+    PoolUpload<EdmdPart> part;
+    PoolUpload<int32_t> ccnt, cslot, ptype;
+    PoolUpload<uint32_t> mt;
+    PoolUpload<double> vr;
+    PoolUpload<EdmdState> st;
+    explicit Uploads(edmd_batch* b)
+        : part(b->part), ccnt(b->ccnt), cslot(b->cslot), ptype(b->ptype), mt(b->mt), vr(b->vr),
+          st(b->st) {}
+    int send() {
+        int rc = part.send();
+        if (!rc) rc = ccnt.send();
+        if (!rc) rc = cslot.send();
+        if (!rc) rc = ptype.send();
+        if (!rc) rc = mt.send();
+        if (!rc) rc = vr.send();
+        if (!rc) rc = st.send();
+        return rc;
+    }
+};
+
+static int upload_system(edmd_batch* b, int s, const edmd_system_desc* d, Uploads* up) {
     HostSys& h = b->hs[s];
     const EdmdConst& c = h.c;
     const int n = c.n;
     const double cfx = 1 / c.csx, cfy = 1 / c.csy;
-    std::vector<double> x(n), y(n);
-    std::vector<int32_t> cx(n), cy(n);
-    const size_t ncell = (size_t)c.ncx * c.ncy;
-    std::vector<int32_t> cnt(ncell, 0), slot(ncell * c.cap, -1);
+    const size_t ncell = (size_t)c.ncx * c.ncy, p0 = h.p0;
+    EdmdPart* part;
+    int32_t *cnt, *slot;
+    int rc = up->part.add(p0, n, &part);
+    if (!rc) rc = up->ccnt.add(h.cell0, ncell, &cnt);
+    if (!rc) rc = up->cslot.add(h.slot0, ncell * c.cap, &slot);
+    if (rc) return rc;
+    std::fill(cnt, cnt + ncell, 0);
+    std::fill(slot, slot + ncell * c.cap, -1);
     for (int i = 0; i < n; i++) {
         /* load path wraps positions into the box, EDMD.c:1429-1430 */
-        x[i] = wrap_post(d->x[i], c.Lx);
-        y[i] = wrap_post(d->y[i], c.Ly);
-        cx[i] = coord_to_cell(x[i], cfx, c.ncx);
-        cy[i] = coord_to_cell(y[i], cfy, c.ncy);
-        size_t cell = (size_t)cy[i] * c.ncx + cx[i];
+        const double x = wrap_post(d->x[i], c.Lx);
+        const double y = wrap_post(d->y[i], c.Ly);
+        const int32_t cx = coord_to_cell(x, cfx, c.ncx);
+        const int32_t cy = coord_to_cell(y, cfy, c.ncy);
+        size_t cell = (size_t)cy * c.ncx + cx;
         if (cnt[cell] >= c.cap)
             return fail(EDMD_ERR_CELL_OVERFLOW,
                         "system %d: cell (%d,%d) holds more than %d disks; raise cell_capacity",
-                        s, cx[i], cy[i], c.cap);
+                        s, cx, cy, c.cap);
         /* cellListInit adds particles in index order, EDMD.c:1916-1919 */
         slot[cell * c.cap + cnt[cell]++] = i;
-    }
-    const size_t p0 = h.p0;
-    std::vector<EdmdPart> part(n);
-    for (int i = 0; i < n; i++) {
         EdmdPart& r = part[i];
         memset(&r, 0, sizeof r);
-        r.x = x[i];
-        r.y = y[i];
+        r.x = x;
+        r.y = y;
         r.vx = d->vx[i];
         r.vy = d->vy[i];
         r.tl = 0;
         r.rad = d->vr > 0 ? 0.0 : d->rad[i]; /* growth starts from radius 0, EDMD.c:1765 */
         r.m = d->m[i];
         r.coll = 0;
-        r.cx = (int16_t)cx[i];
-        r.cy = (int16_t)cy[i];
+        r.cx = (int16_t)cx;
+        r.cy = (int16_t)cy;
     }
-    HIPCHK(hipMemcpy(b->part + p0, part.data(), (size_t)n * sizeof(EdmdPart), hipMemcpyHostToDevice));
-    HIPCHK(hipMemset(b->img + 2 * p0, 0, (size_t)n * 2 * sizeof(int32_t)));
-    HIPCHK(hipMemcpy(b->ccnt + h.cell0, cnt.data(), ncell * sizeof(int32_t), hipMemcpyHostToDevice));
-    HIPCHK(hipMemcpy(b->cslot + h.slot0, slot.data(), ncell * c.cap * sizeof(int32_t),
-                     hipMemcpyHostToDevice));
     if (b->mt) {
         /* init_genrand(rng_seed) of mersenne.c; the index 624 makes the
          * first draw twist */
-        uint32_t w[625];
+        uint32_t* w;
+        if ((rc = up->mt.add((size_t)s * 625, 625, &w))) return rc;
         w[0] = d->rng_seed;
         for (int k = 1; k < 624; k++) w[k] = 1812433253u * (w[k - 1] ^ (w[k - 1] >> 30)) + (uint32_t)k;
         w[624] = 624;
-        HIPCHK(hipMemcpy(b->mt + (size_t)s * 625, w, sizeof w, hipMemcpyHostToDevice));
     }
     if (b->ptype) {
-        std::vector<int32_t> ty(n, 0);
-        if (d->type)
-            for (int i = 0; i < n; i++) ty[i] = d->type[i];
-        HIPCHK(hipMemcpy(b->ptype + p0, ty.data(), (size_t)n * sizeof(int32_t), hipMemcpyHostToDevice));
+        int32_t* ty;
+        if ((rc = up->ptype.add(p0, n, &ty))) return rc;
+        for (int i = 0; i < n; i++) ty[i] = d->type ? d->type[i] : 0;
     }
     if (b->vr) {
-        std::vector<double> g(n, 0.0);
-        if (d->vr > 0)
-            for (int i = 0; i < n; i++) g[i] = d->vr * d->rad[i]; /* EDMD.c:1772 */
-        HIPCHK(hipMemcpy(b->vr + p0, g.data(), (size_t)n * sizeof(double), hipMemcpyHostToDevice));
+        double* g;
+        if ((rc = up->vr.add(p0, n, &g))) return rc;
+        for (int i = 0; i < n; i++) g[i] = d->vr > 0 ? d->vr * d->rad[i] : 0.0; /* EDMD.c:1772 */
     }
     double first_screen = d->first_screen, first_thermo = d->first_thermo;
     if (d->vr > 0) {
@@ -401,7 +454,9 @@ static int upload_system(edmd_batch* b, int s, const edmd_system_desc* d) {
         if (first_screen < 1 / d->vr) first_screen = 1 / d->vr + first_screen;
         if (first_thermo < 1 / d->vr) first_thermo = 1 / d->vr + first_thermo;
     }
-    EdmdState st;
+    EdmdState* row;
+    if ((rc = up->st.add(s, 1, &row))) return rc;
+    EdmdState& st = *row;
     memset(&st, 0, sizeof st);
     st.t = 0;
     st.next_screen = first_screen;
@@ -438,7 +493,6 @@ static int upload_system(edmd_batch* b, int s, const edmd_system_desc* d) {
     st.last_thermo = 0;
     st.ev_limit = INT64_MAX;
     st.coll_limit = ~(uint64_t)0;
-    HIPCHK(hipMemcpy(b->st + s, &st, sizeof st, hipMemcpyHostToDevice));
     return EDMD_OK;
 }
 
@@ -457,19 +511,77 @@ static int batch_predict_all(edmd_batch* b) {
     return EDMD_OK;
 }
 
-static int check_status(edmd_batch* b) {
-    std::vector<EdmdState> st(b->nsys);
-    HIPCHK(hipMemcpy(st.data(), b->st, b->nsys * sizeof(EdmdState), hipMemcpyDeviceToHost));
-    for (int s = 0; s < b->nsys; s++) {
-        if (st[s].status == EDMD_DEV_OVERLAP)
-            return fail(EDMD_ERR_OVERLAP, "system %d: overlapping disks near particle %d at t=%.17g",
-                        s, st[s].err_i, st[s].t);
-        if (st[s].status == EDMD_DEV_CELL_OVERFLOW)
-            return fail(EDMD_ERR_CELL_OVERFLOW, "system %d: cell %d overflow (particle %d) at t=%.17g",
-                        s, st[s].err_j, st[s].err_i, st[s].t);
-        if (st[s].status != 0) return fail(EDMD_ERR_STATE, "system %d: status %d", s, st[s].status);
+/* Rows [0, n) of device array src, handed to put(first, rows, count) piece by
+ * piece, in order.  They come through pinned memory of the batch's own, the
+ * next piece on its way while put works on one: into ordinary memory a copy of
+ * 4096 disks (256 KB) took 116 us, of 2^20 13.9 ms, into pinned memory 13 us
+ * and 1.2 ms.  Pieces of half a megabyte stay in the caches; without room for
+ * pinned memory the copy goes to ordinary memory as one piece. */
+#define EDMD_STAGE_BYTES (512u << 10)
+template <class R, class F>
+static int read_rows(edmd_batch* b, const R* src, size_t n, F&& put) {
+    if (n == 0) return EDMD_OK;
+    std::lock_guard<std::mutex> only(b->stage_lock);
+    if (!b->stage) {
+        const size_t need = std::max((size_t)b->max_n * sizeof(EdmdPart), b->nsys * sizeof(EdmdState));
+        b->stage_half = std::min((need + 4095) & ~(size_t)4095, (size_t)EDMD_STAGE_BYTES);
+        if (hipHostMalloc((void**)&b->stage, 2 * b->stage_half, 0) != hipSuccess) {
+            (void)hipGetLastError();
+            b->stage = nullptr;
+        }
+    }
+    if (!b->stage) {
+        std::vector<R> rows(n);
+        HIPCHK(hipStreamSynchronize(b->stream));
+        HIPCHK(hipMemcpy(rows.data(), src, n * sizeof(R), hipMemcpyDeviceToHost));
+        put((size_t)0, (const R*)rows.data(), n);
+        return EDMD_OK;
+    }
+    const size_t per = b->stage_half / sizeof(R);
+    auto piece = [&](size_t at) { return std::min(per, n - at); };
+    auto fetch = [&](size_t at, int k) {
+        return hipMemcpyAsync(b->stage + k * b->stage_half, src + at, piece(at) * sizeof(R),
+                              hipMemcpyDeviceToHost, b->stream);
+    };
+    HIPCHK(fetch(0, 0));
+    int k = 0;
+    for (size_t at = 0; at < n; at += per, k ^= 1) {
+        HIPCHK(hipStreamSynchronize(b->stream));
+        if (at + per < n) HIPCHK(fetch(at + per, k ^ 1));
+        put(at, (const R*)(b->stage + k * b->stage_half), piece(at));
     }
     return EDMD_OK;
+}
+
+/* The whole array, into ordinary memory. */
+template <class R>
+static int read_all(edmd_batch* b, R* dst, const R* src, size_t n) {
+    return read_rows(b, src, n, [&](size_t at, const R* r, size_t k) { memcpy((void*)(dst + at), r, k * sizeof(R)); });
+}
+
+/* One member of the rows, into dst (if there is one). */
+template <class R, class M, class T>
+static void column(T* dst, const R* rows, size_t n, M R::*member) {
+    if (dst)
+        for (size_t i = 0; i < n; i++) dst[i] = rows[i].*member;
+}
+
+static int check_status(edmd_batch* b) {
+    int bad = 0;
+    int rc = read_rows(b, b->st, (size_t)b->nsys, [&](size_t s0, const EdmdState* st, size_t k) {
+        for (size_t j = 0; j < k && !bad; j++) {
+            const int s = (int)(s0 + j);
+            if (st[j].status == EDMD_DEV_OVERLAP)
+                bad = fail(EDMD_ERR_OVERLAP, "system %d: overlapping disks near particle %d at t=%.17g",
+                           s, st[j].err_i, st[j].t);
+            else if (st[j].status == EDMD_DEV_CELL_OVERFLOW)
+                bad = fail(EDMD_ERR_CELL_OVERFLOW, "system %d: cell %d overflow (particle %d) at t=%.17g",
+                           s, st[j].err_j, st[j].err_i, st[j].t);
+            else if (st[j].status != 0)
+                bad = fail(EDMD_ERR_STATE, "system %d: status %d", s, st[j].status);
+        }
+    });
+    return rc ? rc : bad;
 }
 
 extern "C" int edmd_batch_create(const edmd_system_desc* descs, int nsys, edmd_batch** out) {
@@ -539,6 +651,7 @@ extern "C" int edmd_batch_create(const edmd_system_desc* descs, int nsys, edmd_b
     }
     b->own_stream = true;
     b->sys.resize(nsys);
+    Uploads up(b);
     for (int s = 0; s < nsys; s++) {
         HostSys& h = b->hs[s];
         EdmdSys& S = b->sys[s];
@@ -561,9 +674,13 @@ extern "C" int edmd_batch_create(const edmd_system_desc* descs, int nsys, edmd_b
         A.mt = b->mt ? b->mt + (size_t)s * 625 : nullptr;
         A.erank = b->erank + 2 * p0;
         A.lrank = b->lrank + p0;
-        rc = upload_system(b, s, descs + s);
+        rc = upload_system(b, s, descs + s, &up);
         if (rc) { batch_free(b); return rc; }
     }
+    rc = up.send();
+    if (!rc && hipMemset(b->img, 0, 2 * np * sizeof(int32_t)) != hipSuccess)
+        rc = fail(EDMD_ERR_HIP, "clearing the image counts failed");
+    if (rc) { batch_free(b); return rc; }
     if (hipMalloc(&b->d_sys, nsys * sizeof(EdmdSys)) != hipSuccess) {
         b->d_sys = nullptr;
         batch_free(b);
@@ -1109,59 +1226,55 @@ static int d2h(T* dst, const T* src, size_t n) {
     return EDMD_OK;
 }
 
+template <class T>
+static T* from(T* p, size_t at) {
+    return p ? p + at : nullptr;
+}
+
 extern "C" int edmd_batch_get_state(edmd_batch* b, int s, double* x, double* y, double* vx,
                                     double* vy, double* t_local, uint32_t* coll, int32_t* cx,
                                     int32_t* cy) {
     int rc = sys_check(b, s);
     if (rc) return rc;
-    HIPCHK(hipStreamSynchronize(b->stream));
     const HostSys& h = b->hs[s];
-    size_t n = h.c.n;
-    std::vector<EdmdPart> part(n);
-    if ((rc = d2h(part.data(), b->part + h.p0, n))) return rc;
-    for (size_t i = 0; i < n; i++) {
-        const EdmdPart& r = part[i];
-        if (x) x[i] = r.x;
-        if (y) y[i] = r.y;
-        if (vx) vx[i] = r.vx;
-        if (vy) vy[i] = r.vy;
-        if (t_local) t_local[i] = r.tl;
-        if (coll) coll[i] = r.coll;
-        if (cx) cx[i] = r.cx;
-        if (cy) cy[i] = r.cy;
-    }
-    return EDMD_OK;
+    return read_rows(b, b->part + h.p0, (size_t)h.c.n, [&](size_t at, const EdmdPart* r, size_t n) {
+        column(from(x, at), r, n, &EdmdPart::x);
+        column(from(y, at), r, n, &EdmdPart::y);
+        column(from(vx, at), r, n, &EdmdPart::vx);
+        column(from(vy, at), r, n, &EdmdPart::vy);
+        column(from(t_local, at), r, n, &EdmdPart::tl);
+        column(from(coll, at), r, n, &EdmdPart::coll);
+        column(from(cx, at), r, n, &EdmdPart::cx);
+        column(from(cy, at), r, n, &EdmdPart::cy);
+    });
 }
 
 extern "C" int edmd_batch_get_radii(edmd_batch* b, int s, double* rad) {
     int rc = sys_check(b, s);
     if (rc) return rc;
     if (!rad) return fail(EDMD_ERR_ARG, "null output");
-    HIPCHK(hipStreamSynchronize(b->stream));
     const HostSys& h = b->hs[s];
-    size_t n = h.c.n;
-    std::vector<EdmdPart> part(n);
-    if ((rc = d2h(part.data(), b->part + h.p0, n))) return rc;
-    for (size_t i = 0; i < n; i++) rad[i] = part[i].rad;
-    return EDMD_OK;
+    return read_rows(b, b->part + h.p0, (size_t)h.c.n, [&](size_t at, const EdmdPart* r, size_t n) {
+        column(rad + at, r, n, &EdmdPart::rad);
+    });
+}
+
+static int read_events(edmd_batch* b, int s, double* t_coll, int32_t* partner, double* t_cross,
+                       int32_t* dir, uint32_t* coll_actual) {
+    const HostSys& h = b->hs[s];
+    return read_rows(b, b->ev + h.p0, (size_t)h.c.n, [&](size_t at, const EdmdEv* r, size_t n) {
+        column(from(t_coll, at), r, n, &EdmdEv::tcoll);
+        column(from(partner, at), r, n, &EdmdEv::partner);
+        column(from(t_cross, at), r, n, &EdmdEv::tcross);
+        column(from(dir, at), r, n, &EdmdEv::dir);
+        column(from(coll_actual, at), r, n, &EdmdEv::cact);
+    });
 }
 
 extern "C" int edmd_batch_get_events(edmd_batch* b, int s, double* t_coll, int32_t* partner,
                                      double* t_cross, int32_t* dir) {
     int rc = sys_check(b, s);
-    if (rc) return rc;
-    HIPCHK(hipStreamSynchronize(b->stream));
-    const HostSys& h = b->hs[s];
-    size_t n = h.c.n;
-    std::vector<EdmdEv> ev(n);
-    if ((rc = d2h(ev.data(), b->ev + h.p0, n))) return rc;
-    for (size_t i = 0; i < n; i++) {
-        if (t_coll) t_coll[i] = ev[i].tcoll;
-        if (partner) partner[i] = ev[i].partner;
-        if (t_cross) t_cross[i] = ev[i].tcross;
-        if (dir) dir[i] = ev[i].dir;
-    }
-    return EDMD_OK;
+    return rc ? rc : read_events(b, s, t_coll, partner, t_cross, dir, nullptr);
 }
 
 extern "C" int edmd_batch_get_calendar(edmd_batch* b, int s, double* key, int32_t* idx,
@@ -1200,22 +1313,21 @@ extern "C" int edmd_batch_get_observables(edmd_batch* b, int s, edmd_observables
     int rc = sys_check(b, s);
     if (rc) return rc;
     if (!o) return fail(EDMD_ERR_ARG, "null output");
-    HIPCHK(hipStreamSynchronize(b->stream));
     const HostSys& h = b->hs[s];
     EdmdState st;
-    HIPCHK(hipMemcpy(&st, b->st + s, sizeof st, hipMemcpyDeviceToHost));
-    size_t n = h.c.n;
-    std::vector<EdmdPart> part(n);
-    if ((rc = d2h(part.data(), b->part + h.p0, n))) return rc;
+    if ((rc = read_all(b, &st, b->st + s, 1))) return rc;
     /* physicalQ, EDMD.c:5968-6013, summed in particle order */
     double E = 0, px = 0, py = 0;
-    for (size_t i = 0; i < n; i++) {
-        const EdmdPart& r = part[i];
-        px += r.vx * r.m;
-        py += r.vy * r.m;
-        double a = r.vx;
-        E += 0.5 * r.m * (a * a + r.vy * r.vy);
-    }
+    rc = read_rows(b, b->part + h.p0, (size_t)h.c.n, [&](size_t, const EdmdPart* part, size_t n) {
+        for (size_t i = 0; i < n; i++) {
+            const EdmdPart& r = part[i];
+            px += r.vx * r.m;
+            py += r.vy * r.m;
+            double a = r.vx;
+            E += 0.5 * r.m * (a * a + r.vy * r.vy);
+        }
+    });
+    if (rc) return rc;
     o->t = st.t;
     o->ncol = st.ncol;
     o->ncross = st.ncross;
@@ -1402,13 +1514,7 @@ extern "C" int edmd_get_radii(edmd_ctx* c, double* rad) {
 extern "C" int edmd_get_events(edmd_ctx* c, double* t_cross, int32_t* dir, double* t_coll,
                                int32_t* partner, uint32_t* coll_actual) {
     if (!c) return fail(EDMD_ERR_ARG, "null context");
-    int rc = edmd_batch_get_events(c->b, 0, t_coll, partner, t_cross, dir);
-    if (rc || !coll_actual) return rc;
-    size_t n = c->b->hs[0].c.n;
-    std::vector<EdmdEv> ev(n);
-    if ((rc = d2h(ev.data(), c->b->ev + c->b->hs[0].p0, n))) return rc;
-    for (size_t i = 0; i < n; i++) coll_actual[i] = ev[i].cact;
-    return EDMD_OK;
+    return read_events(c->b, 0, t_coll, partner, t_cross, dir, coll_actual);
 }
 
 extern "C" int edmd_get_observables(edmd_ctx* c, edmd_observables* o) {
@@ -1887,10 +1993,18 @@ static int deriv_alloc(edmd_batch* b, T** p, size_t n) {
     return EDMD_OK;
 }
 
-extern "C" int edmd_batch_deriv_end(edmd_batch* b) {
-    if (!b) return fail(EDMD_ERR_ARG, "null batch");
+/* Ends the taping; with `keep` its memory stays for the next one, which has
+ * the same tape capacity. */
+static int deriv_stop(edmd_batch* b, bool keep) {
     HIPCHK(hipStreamSynchronize(b->stream));
-    deriv_release(b);
+    if (keep) {
+        for (auto& c : b->ckpts) b->ckpt_free.push_back(c.mem);
+        b->ckpts.clear();
+        b->deriv_on = false;
+        b->seg = 0;
+    } else {
+        deriv_release(b);
+    }
     for (int s = 0; s < b->nsys; s++) {
         EdmdSys& S = b->sys[s];
         S.c.tape_cap = 0;
@@ -1903,6 +2017,10 @@ extern "C" int edmd_batch_deriv_end(edmd_batch* b) {
     HIPCHK(edmd_launch_seg_begin(b->d_sys, b->nsys, 0, 1, b->stream));
     HIPCHK(hipStreamSynchronize(b->stream));
     return EDMD_OK;
+}
+
+extern "C" int edmd_batch_deriv_end(edmd_batch* b) {
+    return b ? deriv_stop(b, false) : fail(EDMD_ERR_ARG, "null batch");
 }
 
 extern "C" int edmd_batch_deriv_begin(edmd_batch* b, int64_t checkpoint_every, int64_t tape_capacity) {
@@ -1924,16 +2042,17 @@ extern "C" int edmd_batch_deriv_begin(edmd_batch* b, int64_t checkpoint_every, i
                         "system %d: derivatives need a system without the circular wall, "
                         "thermal or shear walls, or the field together with damping (flat "
                         "walls, the field and damping are taped)", s);
-    int rc = edmd_batch_deriv_end(b);
+    const bool keep = b->deriv_on && b->tape_cap == cap;
+    int rc = deriv_stop(b, keep);
     if (rc) return rc;
     if ((double)b->nsys * (double)cap * sizeof(EdmdTapeRec) > 1.0e12)
         return fail(EDMD_ERR_NOMEM, "tape of %lld records for %d systems is too large",
                     (long long)cap, b->nsys);
-    if (!rc) rc = deriv_alloc(b, &b->tape, (size_t)b->nsys * (size_t)cap);
-    if (!rc) rc = deriv_alloc(b, &b->dv, 4 * b->np);
-    if (!rc) rc = deriv_alloc(b, &b->dtl, b->np);
-    if (!rc) rc = deriv_alloc(b, &b->otl, b->np);
-    if (!rc) rc = deriv_alloc(b, &b->dr, (size_t)b->nsys);
+    if (!keep) rc = deriv_alloc(b, &b->tape, (size_t)b->nsys * (size_t)cap);
+    if (!rc && !keep) rc = deriv_alloc(b, &b->dv, 4 * b->np);
+    if (!rc && !keep) rc = deriv_alloc(b, &b->dtl, b->np);
+    if (!rc && !keep) rc = deriv_alloc(b, &b->otl, b->np);
+    if (!rc && !keep) rc = deriv_alloc(b, &b->dr, (size_t)b->nsys);
     if (rc) { deriv_release(b); return rc; }
     for (int s = 0; s < b->nsys; s++) {
         EdmdSys& S = b->sys[s];
@@ -1959,7 +2078,8 @@ extern "C" int edmd_batch_deriv_begin(edmd_batch* b, int64_t checkpoint_every, i
 
 static int tape_overflow_check(edmd_batch* b) {
     std::vector<EdmdState> st(b->nsys);
-    HIPCHK(hipMemcpy(st.data(), b->st, b->nsys * sizeof(EdmdState), hipMemcpyDeviceToHost));
+    int rc = read_all(b, st.data(), b->st, (size_t)b->nsys);
+    if (rc) return rc;
     for (int s = 0; s < b->nsys; s++)
         if (st[s].ntape > b->tape_cap)
             return fail(EDMD_ERR_TAPE_FULL, "system %d: %lld collisions exceed the tape capacity %lld",
@@ -1993,15 +2113,21 @@ extern "C" int edmd_batch_deriv_run(edmd_batch* b, int64_t max_events, uint64_t 
     std::vector<EdmdState> st(b->nsys);
     for (;;) {
         void* mem = nullptr;
-        hipError_t e = hipMalloc(&mem, bytes);
+        hipError_t e = hipSuccess;
+        if (b->ckpt_free.empty()) {
+            e = hipMalloc(&mem, bytes);
+        } else {
+            mem = b->ckpt_free.back();
+            b->ckpt_free.pop_back();
+        }
         if (e != hipSuccess)
             return fail(EDMD_ERR_NOMEM, "checkpoint %zu (%zu bytes): %s", b->ckpts.size(), bytes,
                         hipGetErrorString(e));
         b->ckpts.push_back({mem, ra});
         int rc = ckpt_copy(b, mem, true);
         if (!rc) rc = run_segment(b, ra);
+        if (!rc) rc = read_all(b, st.data(), b->st, (size_t)b->nsys);
         if (rc) return rc;
-        HIPCHK(hipMemcpy(st.data(), b->st, b->nsys * sizeof(EdmdState), hipMemcpyDeviceToHost));
         bool more = false;
         for (int s = 0; s < b->nsys; s++)
             if (st[s].stop_reason == EDMD_STOP_EVENTS && (int64_t)st[s].nevents < max_events)
@@ -2059,10 +2185,9 @@ extern "C" int edmd_batch_tangent(edmd_batch* b, const double* tan_in, double* t
         if (rc) return rc;
     }
     HIPCHK(edmd_launch_deriv_flush(b->d_sys, b->nsys, b->max_n, 0, b->stream));
-    HIPCHK(hipStreamSynchronize(b->stream));
-    HIPCHK(hipMemcpy(tan_out, b->dv, 4 * b->np * sizeof(double), hipMemcpyDeviceToHost));
+    if ((rc = read_all(b, tan_out, (const double*)b->dv, 4 * b->np))) return rc;
     std::vector<EdmdDeriv> d(b->nsys);
-    HIPCHK(hipMemcpy(d.data(), b->dr, b->nsys * sizeof(EdmdDeriv), hipMemcpyDeviceToHost));
+    if ((rc = read_all(b, d.data(), b->dr, (size_t)b->nsys))) return rc;
     for (int s = 0; s < b->nsys; s++) {
         if (dw) dw[s] = d[s].dsum;
         if (dtlast) dtlast[s] = d[s].dtlast;
@@ -2099,9 +2224,7 @@ extern "C" int edmd_batch_adjoint(edmd_batch* b, const double* lw, const double*
         if (rc) return rc;
     }
     HIPCHK(edmd_launch_deriv_flush(b->d_sys, b->nsys, b->max_n, 1, b->stream));
-    HIPCHK(hipStreamSynchronize(b->stream));
-    HIPCHK(hipMemcpy(grad, b->dv, 4 * b->np * sizeof(double), hipMemcpyDeviceToHost));
-    return EDMD_OK;
+    return read_all(b, grad, (const double*)b->dv, 4 * b->np);
 }
 
 extern "C" int edmd_batch_deriv_values(edmd_batch* b, int sys, double* w, double* tlast,

@@ -1126,8 +1126,8 @@ __device__ __forceinline__ void wide_loop(const EdmdConst& Cs, const AR& As, Edm
  * the dynamic LDS; LDS = true: the arrays in LDS as well (edmd_lds.h).  Two
  * wavefronts a SIMD: one workgroup of eight, or two of four; without the bound
  * the compiler gave four wavefronts every register, and one CU held one
- * workgroup (512 systems of 400 disks, 300000 events: 18 ms in the loop of one
- * wavefront that ran instead, 12.3 ms here). */
+ * workgroup (512 systems of 400 disks, 4000 collisions each: 18 ms in the loop
+ * of one wavefront that ran instead, 12.3 ms here). */
 template <int NW, bool G, bool W>
 __global__ __launch_bounds__(64 * NW, 2) void k_wide(const EdmdSys* __restrict__ systems,
                                                      EdmdRunArgs ra) {
