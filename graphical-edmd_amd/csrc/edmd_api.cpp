@@ -1967,13 +1967,18 @@ static size_t ckpt_bytes(edmd_batch* b) {
 
 static int ckpt_copy(edmd_batch* b, void* mem, bool save) {
     char* c = (char*)mem;
+    EdmdSpans sp;
+    sp.n = 0;
     for (auto& q : state_pools(b)) {
         if (q.bytes) {
-            if (save) HIPCHK(hipMemcpyAsync(c, q.p, q.bytes, hipMemcpyDeviceToDevice, b->stream));
-            else HIPCHK(hipMemcpyAsync(q.p, c, q.bytes, hipMemcpyDeviceToDevice, b->stream));
+            sp.src[sp.n] = save ? q.p : c;
+            sp.dst[sp.n] = save ? c : q.p;
+            sp.bytes[sp.n] = q.bytes;
+            sp.n++;
         }
         c += align256(q.bytes);
     }
+    HIPCHK(edmd_launch_copy_spans(sp, b->stream));
     return EDMD_OK;
 }
 

@@ -79,6 +79,16 @@ hipError_t edmd_launch_deriv_init(const EdmdSys* d_sys, int nsys, int max_n, int
                                   hipStream_t s);
 hipError_t edmd_launch_deriv_flush(const EdmdSys* d_sys, int nsys, int max_n, int mode,
                                    hipStream_t s);
+/* Spans of device memory copied together; sizes are multiples of 4 bytes,
+ * addresses of 16. */
+#define EDMD_SPANS 11
+struct EdmdSpans {
+    int n;
+    const void* src[EDMD_SPANS];
+    void* dst[EDMD_SPANS];
+    uint64_t bytes[EDMD_SPANS];
+};
+hipError_t edmd_launch_copy_spans(const EdmdSpans& sp, hipStream_t s);
 hipError_t edmd_launch_deriv_origin(const EdmdSys* d_sys, int nsys, int max_n, hipStream_t s);
 hipError_t edmd_launch_seg_begin(const EdmdSys* d_sys, int nsys, int64_t seg, int clear,
                                  hipStream_t s);
