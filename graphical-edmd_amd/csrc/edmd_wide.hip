@@ -12,11 +12,13 @@
  *
  * A round, between barriers:
  *   scan     the keys of the calendar nodes below a moving time limit are
- *            gathered from LDS
- *   leader   the first wavefront orders them, leaves out those that an
- *            earlier one takes away (a collision re-predicts its partner,
- *            whose own event, often the same collision seen from the other
- *            disk, then never pops) and gives wavefront w the w-th of the rest
+ *            gathered from LDS, while the first wavefront brings the loop's
+ *            state up to date
+ *   order    every wavefront places its share of them among the others, and
+ *            marks those that an earlier one takes away (a collision
+ *            re-predicts its partner, whose own event, often the same
+ *            collision seen from the other disk, then never pops); wavefront w
+ *            picks the w-th of the rest
  *   compute  every wavefront works out its event without writing
  *            (event_open, event_predict<SPEC>)
  *   check    every wavefront tests its event against the ones before it: it
@@ -28,9 +30,14 @@
  *            positions follow from the events' order in it
  * The first event of a round always commits, so the loop advances whatever
  * the limit or the spatial distribution; scheduled events and ring wraps are
- * handled between rounds by the whole workgroup.  The ordering is the first
- * wavefront's alone: done by all eight alike it took twice as long, two
- * wavefronts sharing each SIMD's issue.
+ * handled between rounds by the whole workgroup.
+ *
+ * Each round has a fixed cost beside its events: of 19000 cycles (2000 disks)
+ * the scan took 2600 and the ordering 4250 while the first wavefront alone did
+ * it, a chain of some thirty dependent LDS accesses.  Spread over the
+ * wavefronts, one comparison of 64 lanes per entry, and with one count for a
+ * scan's four nodes a lane, the round takes 17400 (2000 disks, 4000
+ * collisions: 6.76 ms to 6.20).
  *
  * The calendar's window level lives in LDS: the leaves themselves up to
  * EDMD_WIDE_FLAT disks, else the first level of at most EDMD_WIDE_NODES
@@ -52,9 +59,19 @@ struct WideEntry {
     int64_t rank;
     int32_t p, aux; /* leaf and event code */
 };
-constexpr int WIDE_LIST = 32; /* entries an order takes */
+template <int NW>
+constexpr int WIDE_LIST = NW > 8 ? 64 : 32; /* entries an order takes: a lane each */
 
-/* An event as the leader hands it to a wavefront. */
+/* An entry in the order of (time, rank). */
+struct WideOrder {
+    double key;
+    int32_t p, aux;
+    int32_t flags; /* WO_*, and from bit 2 the place of the one that takes it away */
+    int32_t pad;
+};
+enum { WO_SHADOWED = 1, WO_STOP = 2 };
+
+/* An event as a wavefront takes it. */
 struct WidePick {
     double key, paul; /* its time; bucket start when it is handled */
     int32_t p, aux;
@@ -79,9 +96,11 @@ struct WideSlot {
 
 enum { WS_COLL = 1, WS_WALL = 2, WS_OV = 4, WS_FULL = 8 };
 
-/* A wavefront's byte of the round's verdict. */
-enum { WB_OK = 1, WB_LAST = 2, WB_COUNTED = 4, WB_TAPED = 8, WB_INS = 16, WB_SHARE = 128 };
-constexpr uint64_t WB_EACH = 0x0101010101010101ull;
+/* A wavefront's word of the round's verdict. */
+enum {
+    WB_OK = 1, WB_LAST = 2, WB_COUNTED = 4, WB_TAPED = 8, WB_INS = 16, WB_SHARE = 128,
+    WB_CROSS = 256
+};
 
 /* The nodes above an event's new leaves up to the window level (in LDS
  * until the event commits). */
@@ -102,7 +121,6 @@ struct WideState {
     int64_t ntape, ntrace;
     double width; /* of the window */
     int32_t last_type, guard, tries, reason;
-    int32_t solo; /* the next round handles the earliest event alone */
     int32_t halt; /* a kind of event that stops the run was handled */
 };
 
@@ -113,10 +131,11 @@ struct WideShared {
     WidePick pick[NW];
     WideSlot slot[NW];
     PathNodes nodes[NW];
-    WideEntry list[WIDE_LIST];
-    int32_t shad[WIDE_LIST];
-    uint64_t verdict; /* a byte per wavefront */
+    WideEntry list[WIDE_LIST<NW>];
+    WideOrder sorted[WIDE_LIST<NW>];
+    int32_t verdict[NW];
     int32_t lcount, todo, cut, sums, moved; /* cut: events the last round committed */
+    int32_t stop; /* why the loop stops, EDMD_STOP_NONE: it goes on */
     int32_t room, croom; /* events and counted events that the bounds leave */
     double lim;          /* the scan's time limit */
     double vir[4];
@@ -415,154 +434,158 @@ __device__ __forceinline__ void fly_neighbours(const EdmdConst& C, const AR& A, 
     }
 }
 
-/* The leader's part of a round: orders the gathered nodes, leaves out what an
- * earlier one takes away and fills the picks; the buckets up to each event
- * (pick_next) are counted in plain steps, an event behind a ring wrap or a
- * scheduled event is not plain.  Returns WT_ROUND, or what must happen before
- * the earliest event. */
-template <int NW, bool W, class AR>
-__device__ __forceinline__ int wide_order(const EdmdConst& C, const AR& A, int lane,
-                                          const WideCal& Wc, WideShared<NW>& Sh) {
-    WideState& Z = Sh.state;
-    LoopRegs& R = Z.R;
-    double width = Z.width;
-    int n = Sh.lcount;
-    if (n < 1 || n > WIDE_LIST) {
-        if (Z.tries < 12) {
-            /* no usable window: another limit */
-            ++Z.tries;
-            width *= n > WIDE_LIST ? 0.5 : 4.0;
-            if (!(width > 0)) width = 1e-300;
-            Z.width = width;
-            if (lane == 0) {
-                Sh.lcount = 0;
-                Sh.lim = R.t + width;
+/* This wavefront's share of the n gathered nodes, entries wave, wave + NW, ...:
+ * each one's place by (time, rank) and whether an earlier one takes it away.
+ * Every lane holds an entry, so one comparison a lane places one of them. */
+template <int NW>
+__device__ __forceinline__ void wide_rank(WideShared<NW>& Sh, int lane, int wave, int n) {
+    const bool in = lane < n;
+    const WideEntry me = Sh.list[in ? lane : 0];
+    const double key = in ? me.key : INF_D;
+    const int p = in ? me.p : -1, aux = in ? me.aux : -1;
+    const int64_t rank = me.rank;
+    /* the entries before e, and those whose partner e's disk is */
+    auto look = [&](int e, uint64_t& sooner, uint64_t& hit) {
+        const double ke = lane_value(key, e);
+        const int64_t re = lane_value64(rank, e);
+        sooner = __ballot((key < ke) | (in & (key == ke) & (rank < re)));
+        hit = __ballot(aux == __builtin_amdgcn_readlane(p, e));
+    };
+    for (int e = wave; e < n; e += NW) {
+        uint64_t sooner, hit;
+        look(e, sooner, hit);
+        const int place = (int)__popcll(sooner);
+        int flags = 0;
+        if (hit) {
+            /* taken away by entry `by`, if that comes earlier; where it is
+             * itself taken away, or several name this disk, the window ends
+             * here */
+            const int by = 63 - (int)__builtin_clzll(hit);
+            const bool shadowed = ((sooner >> by) & 1) != 0;
+            bool stop = __popcll(hit) > 1 && place > 0;
+            if (shadowed) {
+                uint64_t bsooner, bhit;
+                look(by, bsooner, bhit);
+                if (bhit) stop |= ((bsooner >> (63 - (int)__builtin_clzll(bhit))) & 1) != 0;
+                flags = WO_SHADOWED | ((int)__popcll(bsooner) << 2);
             }
-            return WT_SCAN;
+            if (stop) flags |= WO_STOP;
         }
-        n = -1;
-    }
-    /* the next window: about two events a wavefront */
-    if (n >= 0 && n < NW + NW / 2) width = width * 1.2 + 1e-300;
-    else if (n > 2 * NW + NW / 4) width = width * 0.85;
-    Z.width = width;
-    double key;
-    int p, aux;
-    bool shadowed = false, stop = false;
-    if (n > 0) {
-        /* lanes e and 32 + e: entry e of the list, against every other one
-         * (even ones on the lower half, odd ones on the upper): its place by
-         * (time, rank), and the one whose partner it is */
-        const int e = lane & 31, h = lane >> 5;
-        const bool in = e < n;
-        const WideEntry me = Sh.list[in ? e : 0];
-        p = me.p;
-        int place = 0, by = -1, count = 0;
-        for (int i = 0; i < n; i += 8) {
-            WideEntry o[4];
-#pragma unroll
-            for (int c = 0; c < 4; ++c) o[c] = Sh.list[(i + 2 * c + h) & (WIDE_LIST - 1)];
-#pragma unroll
-            for (int c = 0; c < 4; ++c) {
-                const int k = i + 2 * c + h;
-                const bool real = k < n;
-                const bool sooner = (o[c].key < me.key) | ((o[c].key == me.key) & (o[c].rank < me.rank));
-                const bool hit = real & (o[c].aux == p);
-                place += (real & sooner) ? 1 : 0;
-                by = hit ? k : by;
-                count += hit ? 1 : 0;
-            }
+        if (lane == e) {
+            WideOrder& o = Sh.sorted[place];
+            o.key = key;
+            o.p = p;
+            o.aux = aux;
+            o.flags = flags;
         }
-        int u, v;
-        halves(place, u, v);
-        place = in ? u + v : e;
-        halves(by, u, v);
-        by = u > v ? u : v;
-        halves(count, u, v);
-        count = u + v;
-        /* taken away by entry `by`, if that comes earlier; where it is itself
-         * taken away, or several name this disk, the window ends here */
-        const int bat = 4 * (by < 0 ? 0 : by);
-        const int bplace = __builtin_amdgcn_ds_bpermute(bat, place);
-        shadowed = in && by >= 0 && bplace < place;
-        const int bshadowed = __builtin_amdgcn_ds_bpermute(bat, shadowed ? 1 : 0);
-        stop = in && by >= 0 && ((count > 1 && place > 0) || (shadowed && bshadowed));
-        /* by place, on lanes 0 .. n - 1 */
-        const int from = 4 * (__builtin_amdgcn_ds_permute(4 * place, lane) & 31);
-        const int flag = (shadowed ? 1 : 0) | (stop ? 2 : 0) | (bplace << 2);
-        const int sflag = __builtin_amdgcn_ds_bpermute(from, flag);
-        const long long kb = __double_as_longlong(me.key);
-        const int klo = __builtin_amdgcn_ds_bpermute(from, (int)kb);
-        const int khi = __builtin_amdgcn_ds_bpermute(from, (int)(kb >> 32));
-        key = __longlong_as_double(((long long)khi << 32) | (unsigned int)klo);
-        p = __builtin_amdgcn_ds_bpermute(from, p);
-        aux = __builtin_amdgcn_ds_bpermute(from, me.aux);
-        shadowed = (sflag & 1) != 0;
-        stop = (sflag & 2) != 0 && lane < n;
-        if (lane < WIDE_LIST) Sh.shad[lane] = 64;
-        WAVE_SYNC();
-        if (lane < n && shadowed) atomicMin(&Sh.shad[sflag >> 2], lane);
-        WAVE_SYNC();
-    } else {
-        /* many equal times, or none pending: the earliest event alone */
-        key = INF_D;
-        int64_t rank = 0;
-        int node = 0;
-        for (int g = lane; g < Wc.m; g += 64) {
-            const double k = Wc.key[g];
-            if (k < key || (k == key && k < INF_D && Wc.rank[g] < rank)) {
-                key = k;
-                rank = Wc.rank[g];
-                node = g;
-            }
-        }
-        int leaf = Wc.ls > 0 ? Wc.idx[node] : node, who = lane;
-        double kk = key;
-        wave_argmin(A, R.t, kk, leaf, who);
-        key = kk;
-        node = __builtin_amdgcn_readlane(node, who);
-        p = Wc.ls > 0 ? Wc.idx[node] : node;
-        aux = Wc.aux[node];
-        n = 1;
-        if (lane < WIDE_LIST) Sh.shad[lane] = 64;
-        WAVE_SYNC();
     }
-    Z.tries = 0;
-    const double k0 = lane_value(key, 0);
-    const int p0 = __builtin_amdgcn_readlane(p, 0);
-    if (lane == 0) {
-        Sh.lcount = 0;
-        Sh.lim = k0 + width; /* of the next scan, unless the time moves on */
-    }
-    if (!(k0 < INF_D) && !(R.next_special < INF_D)) return WT_STOP;
-    /* the buckets up to each event */
-    uint64_t use = __ballot(lane < n && !shadowed);
-    const uint64_t end = __ballot(stop);
-    if (end) use &= ((uint64_t)1 << __builtin_ctzll(end)) - 1;
-    if (Z.solo) use = 1;
-    const int pos = (int)__popcll(use & (((uint64_t)1 << lane) - 1));
-    const bool mine = ((use >> lane) & 1) != 0 && pos < NW;
-    double paul = R.paul;
-    int steps = 0;
-    bool plain = mine && key < INF_D && key < R.next_special && !(R.swin >= 0 && R.swin <= R.win);
+}
+
+/* The buckets up to an event at `key` (pick_next): paul and steps; whether it
+ * is a plain one, not behind a ring wrap or a scheduled event. */
+__device__ __forceinline__ bool wide_buckets(const EdmdConst& C, const LoopRegs& R, bool on,
+                                             double key, double& paul, int& steps) {
+    paul = R.paul;
+    steps = 0;
+    const int cur = R.cur;
+    const int64_t win = R.win, swin = R.swin;
+    bool plain = on && key < INF_D && key < R.next_special && !(swin >= 0 && swin <= win);
     while (plain && !(key - paul < C.dtp)) {
         paul = paul + C.dtp;
         ++steps;
-        if (R.cur + steps >= C.nlists || steps > 4096 || (R.swin >= 0 && R.swin <= R.win + steps))
+        if (cur + steps >= C.nlists || steps > 4096 || (swin >= 0 && swin <= win + steps))
             plain = false;
     }
-    if (W && C.thermal_wall && pos > 0 && aux <= EDMD_WALL_CODE(0)) plain = false;
-    if (Z.solo && lane == 0) {
-        plain = true;
-        paul = R.paul;
-        steps = 0;
+    return plain;
+}
+
+/* This wavefront's event of the n ordered ones, into its pick and k; false
+ * where the earliest one is not plain. */
+template <int NW, bool W>
+__device__ __forceinline__ bool wide_pick(const EdmdConst& C, WideShared<NW>& Sh, int lane,
+                                          int wave, int n, WidePick& k) {
+    const WideOrder me = Sh.sorted[lane < n ? lane : 0];
+    const int flags = lane < n ? me.flags : 0;
+    uint64_t use = __ballot(lane < n && !(flags & WO_SHADOWED));
+    const uint64_t end = __ballot((flags & WO_STOP) != 0);
+    if (end) use &= ((uint64_t)1 << __builtin_ctzll(end)) - 1;
+    const int pos = (int)__popcll(use & (((uint64_t)1 << lane) - 1));
+    const uint64_t mine = __ballot(pos == wave && ((use >> lane) & 1) != 0);
+    const int ord = mine ? (int)__builtin_ctzll(mine) : 0;
+    double paul;
+    int steps;
+    const bool plain = wide_buckets(C, Sh.state.R, lane == 0 || lane == ord, me.key, paul, steps);
+    const uint64_t plains = __ballot(plain);
+    k.key = lane_value(me.key, ord);
+    k.paul = lane_value(paul, ord);
+    k.p = __builtin_amdgcn_readlane(me.p, ord);
+    k.aux = __builtin_amdgcn_readlane(me.aux, ord);
+    k.steps = __builtin_amdgcn_readlane(steps, ord);
+    k.ord = ord;
+    const uint64_t takes = __ballot((flags & WO_SHADOWED) != 0 && (flags >> 2) == ord);
+    k.shad = takes ? (int)__builtin_ctzll(takes) : 64;
+    k.plain = mine && ((plains >> ord) & 1) ? 1 : 0;
+    if (W && C.thermal_wall && wave > 0 && k.aux <= EDMD_WALL_CODE(0)) k.plain = 0;
+    if (lane == 0) Sh.pick[wave] = k;
+    return (plains & 1) != 0;
+}
+
+/* The leader's decision where a round cannot start from the gathered nodes:
+ * too many of them or none (another limit, WT_SCAN; the earliest event alone
+ * after twelve), or the earliest one is not plain (what findNextEvent does
+ * next, EDMD.c:2313-2327, one ring wrap at a time). */
+template <int NW, class AR>
+__device__ __forceinline__ int wide_decide(const EdmdConst& C, const AR& A, int lane,
+                                           const WideCal& Wc, WideShared<NW>& Sh, bool ordered) {
+    WideState& Z = Sh.state;
+    LoopRegs& R = Z.R;
+    double width = Z.width;
+    if (!ordered && Z.tries < 12) {
+        width *= Sh.lcount > WIDE_LIST<NW> ? 0.5 : 4.0;
+        if (!(width > 0)) width = 1e-300;
+        WAVE_SYNC();
+        if (lane == 0) {
+            ++Z.tries;
+            Z.width = width;
+            Sh.lcount = 0;
+            Sh.lim = R.t + width;
+        }
+        return WT_SCAN;
     }
-    if (__ballot(lane == 0 && plain) == 0) {
-        /* the earliest event is not a plain one: findNextEvent's decision
-         * (EDMD.c:2313-2327), one ring wrap at a time */
-        for (;; ++Z.guard) {
-            const bool part_in = k0 - R.paul < C.dtp;
-            const bool spec_in = R.swin >= 0 && R.swin <= R.win;
+    double k0 = INF_D;
+    int64_t rank = 0;
+    int node = 0;
+    for (int g = lane; g < Wc.m; g += 64) {
+        const double k = Wc.key[g];
+        if (k < k0 || (k == k0 && k < INF_D && Wc.rank[g] < rank)) {
+            k0 = k;
+            rank = Wc.rank[g];
+            node = g;
+        }
+    }
+    int leaf = Wc.ls > 0 ? Wc.idx[node] : node, who = lane;
+    wave_argmin(A, R.t, k0, leaf, who);
+    node = __builtin_amdgcn_readlane(node, who);
+    const int p0 = Wc.ls > 0 ? Wc.idx[node] : node, aux0 = Wc.aux[node];
+    if (lane == 0) {
+        Z.tries = 0;
+        Sh.lcount = 0;
+        Sh.lim = k0 + width;
+    }
+    WAVE_SYNC();
+    if (!(k0 < INF_D) && !(R.next_special < INF_D)) {
+        if (lane == 0) Z.reason = EDMD_STOP_EMPTY;
+        return WT_STOP;
+    }
+    double paul;
+    int steps;
+    if (!wide_buckets(C, R, true, k0, paul, steps)) {
+        double rpaul = R.paul;
+        int64_t win = R.win;
+        int cur = R.cur, guard = Z.guard, todo = -1;
+        for (;; ++guard) {
+            const bool part_in = k0 - rpaul < C.dtp;
+            const bool spec_in = R.swin >= 0 && R.swin <= win;
             auto sooner = [&]() {
                 return before(R.next_special, R.srank, k0,
                               k0 == R.next_special ? uni64(A.lrank[p0]) : (int64_t)0);
@@ -572,142 +595,172 @@ __device__ __forceinline__ int wide_order(const EdmdConst& C, const AR& A, int l
                 special = spec_in && (!part_in || sooner());
             } else if (!(k0 < 1e25) && !(R.next_special < 1e25)) {
                 special = R.next_special <= k0;
-            } else if (Z.guard >= (1 << 24)) {
+            } else if (guard >= (1 << 24)) {
                 const double tn = k0 < R.next_special ? k0 : R.next_special;
-                while (!(tn - R.paul < C.dtp)) {
-                    R.paul = R.paul + C.dtp;
-                    R.win++;
+                while (!(tn - rpaul < C.dtp)) {
+                    rpaul = rpaul + C.dtp;
+                    win++;
                 }
                 special = sooner();
             } else {
-                R.paul = R.paul + C.dtp;
-                R.win++;
-                if (++R.cur >= C.nlists) {
-                    R.cur = 0;
-                    ++Z.guard;
-                    return WT_WRAP;
+                rpaul = rpaul + C.dtp;
+                win++;
+                if (++cur >= C.nlists) {
+                    cur = 0;
+                    ++guard;
+                    todo = WT_WRAP;
+                    break;
                 }
                 continue;
             }
-            if (special) return WT_SPECIAL;
-            /* a particle event after all: alone in a round of its own */
-            Z.solo = 1;
-            if (lane == 0) Sh.lim = k0 + width;
-            return WT_SCAN;
+            if (special) todo = WT_SPECIAL;
+            break;
         }
+        WAVE_SYNC();
+        if (lane == 0) {
+            R.paul = rpaul;
+            R.win = win;
+            R.cur = cur;
+            Z.guard = guard;
+        }
+        if (todo >= 0) return todo;
+        /* a particle event after all, alone */
+        paul = rpaul;
+        steps = 0;
     }
-    if (lane < NW) Sh.pick[lane].plain = 0;
-    WAVE_SYNC();
-    if (mine) {
-        WidePick& k = Sh.pick[pos];
-        k.key = key;
+    if (lane < NW) {
+        WidePick k;
+        k.key = k0;
         k.paul = paul;
-        k.p = p;
-        k.aux = aux;
+        k.p = p0;
+        k.aux = aux0;
         k.steps = steps;
-        k.plain = plain ? 1 : 0;
-        k.ord = lane;
-        k.shad = Sh.shad[lane & (WIDE_LIST - 1)];
+        k.plain = lane == 0 ? 1 : 0;
+        k.ord = 0;
+        k.shad = 64;
+        Sh.pick[lane] = k;
     }
     return WT_ROUND;
 }
 
-/* The events of a round that commit, from its verdict: up to the first one
- * that failed its test, the first after which the loop stops, the bounds. */
+/* The round's verdict: one bit a wavefront each. */
+struct WideVerdict {
+    uint32_t ok, last, counted, taped, one, two, four, share, cross;
+};
+
 template <int NW>
-__device__ __forceinline__ int wide_cut(uint64_t verdict, int room, int croom) {
-    const uint64_t all = NW == 8 ? ~(uint64_t)0 : ((uint64_t)1 << (8 * (NW & 7))) - 1;
-    const uint64_t fail = ~verdict & WB_EACH & all, last = (verdict >> 1) & WB_EACH;
-    int cut = NW;
-    if (fail) cut = (int)__builtin_ctzll(fail) >> 3;
-    if (last) {
-        const int c = ((int)__builtin_ctzll(last) >> 3) + 1;
+__device__ __forceinline__ WideVerdict wide_verdict(const WideShared<NW>& Sh, int lane) {
+    const int v = lane < NW ? Sh.verdict[lane] : 0;
+    WideVerdict V;
+    V.ok = (uint32_t)__ballot((v & WB_OK) != 0);
+    V.last = (uint32_t)__ballot((v & WB_LAST) != 0);
+    V.counted = (uint32_t)__ballot((v & WB_COUNTED) != 0);
+    V.taped = (uint32_t)__ballot((v & WB_TAPED) != 0);
+    V.one = (uint32_t)__ballot((v & WB_INS) != 0);
+    V.two = (uint32_t)__ballot((v & (2 * WB_INS)) != 0);
+    V.four = (uint32_t)__ballot((v & (4 * WB_INS)) != 0);
+    V.share = (uint32_t)__ballot((v & WB_SHARE) != 0);
+    V.cross = (uint32_t)__ballot((v & WB_CROSS) != 0);
+    return V;
+}
+
+/* The events of a round that commit: up to the first one that failed its
+ * test, the first after which the loop stops, the bounds. */
+template <int NW>
+__device__ __forceinline__ int wide_cut(const WideVerdict& V, int room, int croom) {
+    int cut = (int)__builtin_ctz(~V.ok | (1u << NW));
+    if (V.last) {
+        const int c = (int)__builtin_ctz(V.last) + 1;
         cut = c < cut ? c : cut;
     }
     cut = room < cut ? room : cut;
     if (croom <= NW) {
         int c = 0, m = 0;
-        for (; m < cut && c < croom; ++m) c += (int)(verdict >> (8 * m + 2)) & 1;
+        for (; m < cut && c < croom; ++m) c += (int)(V.counted >> m) & 1;
         cut = m;
     }
     return cut;
 }
 
-/* The verdict's bytes below wavefront m. */
-__device__ __forceinline__ uint64_t wide_below(uint64_t verdict, int m) {
-    return m >= 8 ? verdict : verdict & (((uint64_t)1 << (8 * m)) - 1);
+/* Insertions of the events below m. */
+__device__ __forceinline__ int wide_inserts(const WideVerdict& V, int m) {
+    const uint32_t below = (1u << m) - 1;
+    return __popc(V.one & below) + 2 * __popc(V.two & below) + 4 * __popc(V.four & below);
 }
 
-__device__ __forceinline__ int wide_inserts(uint64_t v) {
-    return (int)(__popcll((v >> 4) & WB_EACH) + 2 * __popcll((v >> 5) & WB_EACH) +
-                 4 * __popcll((v >> 6) & WB_EACH));
-}
-
-/* The loop's state after a round of `cut` events (the leader's first lane),
- * and what the next round needs of it. */
+/* The loop's state after a round of `cut` events (the leader), what the next
+ * round needs of it, and whether there is one. */
 template <int NW>
-__device__ __forceinline__ void wide_advance(const EdmdConst& C, WideShared<NW>& Sh, int cut,
-                                             int stop_mask, int64_t ev_limit, uint64_t coll_limit) {
+__device__ __forceinline__ void wide_advance(const EdmdConst& C, WideShared<NW>& Sh, int lane,
+                                             const EdmdRunArgs& ra, int64_t ev_limit,
+                                             uint64_t coll_limit) {
     WideState& Z = Sh.state;
     LoopRegs& R = Z.R;
-    if (cut == 0) {
-        /* no round since the state was read or a scheduled event */
-        const int64_t er = ev_limit - (int64_t)R.nevents;
-        const uint64_t cr = coll_limit - R.ncol;
-        Sh.room = er < NW ? (int)er : NW;
-        Sh.croom = cr <= NW ? (int)cr : NW + 1;
-        Sh.ctr = R.ctr;
-        Sh.ntape = Z.ntape;
-        Sh.ntrace = Z.ntrace;
-        return;
+    const int cut = __builtin_amdgcn_readfirstlane(Sh.cut); /* 0: no round since */
+    const WideVerdict V = wide_verdict<NW>(Sh, lane);
+    if (lane != 0) return;
+    double t = R.t;
+    int64_t ctr = R.ctr, ntape = Z.ntape, ntrace = Z.ntrace, nevents = (int64_t)R.nevents;
+    uint64_t ncol = R.ncol;
+    int status = R.status, halt = Z.halt;
+    if (cut > 0) {
+        const uint32_t done = (1u << cut) - 1;
+        const WideSlot& last = Sh.slot[cut - 1];
+        const WidePick& lp = Sh.pick[cut - 1];
+        const int type = last.type, flags = last.flags;
+        t = lp.key;
+        ctr += wide_inserts(V, cut);
+        ncol += (uint64_t)__popc(V.counted & done);
+        nevents += cut;
+        if (C.trace_cap > 0) ntrace += cut;
+        ntape += __popc(V.taped & done);
+        if (ra.stop_mask & (1 << type)) halt = 1;
+        if (flags & WS_FULL) {
+            status = EDMD_DEV_CELL_OVERFLOW;
+            R.err_i = last.p;
+            R.err_j = (last.ca >> 16) * C.ncx + (last.ca & 0xffff);
+            ctr -= 2; /* the crossing stops before its insertions */
+        } else if (flags & WS_OV) {
+            status = EDMD_DEV_OVERLAP;
+            R.err_i = last.p;
+        }
+        R.t = t;
+        R.paul = lp.paul;
+        R.win += lp.steps;
+        R.cur += lp.steps;
+        R.ncol = ncol;
+        R.nevents = (uint64_t)nevents;
+        R.status = status;
+        R.ctr = ctr;
+        Z.last_type = type;
+        Z.ntape = ntape;
+        Z.ntrace = ntrace;
+        Z.ncross += (uint64_t)__popc(V.cross & done);
+        Z.guard = 0;
+        Z.halt = halt;
     }
-    const uint64_t done = wide_below(Sh.verdict, cut);
-    const WideSlot& last = Sh.slot[cut - 1];
-    const WidePick& lp = Sh.pick[cut - 1];
-    const int type = last.type, flags = last.flags, nins = wide_inserts(done);
-    int ncr = 0;
-#pragma unroll
-    for (int m = 0; m < NW; ++m) ncr += (m < cut && Sh.slot[m].type == EDMD_EV_CELLCROSS) ? 1 : 0;
-    const double t = lp.key;
-    int64_t ctr = R.ctr + nins;
-    R.t = t;
-    R.paul = lp.paul;
-    R.win += lp.steps;
-    R.cur += lp.steps;
-    R.ncol += __popcll((done >> 2) & WB_EACH);
-    R.nevents += cut;
-    Z.last_type = type;
-    if (C.trace_cap > 0) Z.ntrace += cut;
-    Z.ntape += __popcll((done >> 3) & WB_EACH);
-    Z.ncross += ncr;
-    Z.guard = 0;
-    Z.solo = 0;
-    if (stop_mask & (1 << type)) Z.halt = 1;
-    if (flags & WS_FULL) {
-        R.status = EDMD_DEV_CELL_OVERFLOW;
-        R.err_i = last.p;
-        R.err_j = (last.ca >> 16) * C.ncx + (last.ca & 0xffff);
-        ctr -= 2; /* the crossing stops before its insertions */
-    } else if (flags & WS_OV) {
-        R.status = EDMD_DEV_OVERLAP;
-        R.err_i = last.p;
-    }
-    R.ctr = ctr;
-    /* for the round that follows */
-    const int64_t er = ev_limit - (int64_t)R.nevents;
-    const uint64_t cr = coll_limit - R.ncol;
+    const int64_t er = ev_limit - nevents;
+    const uint64_t cr = coll_limit - ncol;
     Sh.room = er < NW ? (int)er : NW;
     Sh.croom = cr <= NW ? (int)cr : NW + 1;
     Sh.ctr = ctr;
-    Sh.ntape = Z.ntape;
-    Sh.ntrace = Z.ntrace;
+    Sh.ntape = ntape;
+    Sh.ntrace = ntrace;
+    int why = EDMD_STOP_NONE;
+    if (halt) why = EDMD_STOP_SPECIAL;
+    else if (status != EDMD_DEV_OK) why = EDMD_STOP_ERROR;
+    else if (nevents >= ev_limit) why = EDMD_STOP_EVENTS;
+    else if (ncol >= coll_limit) why = EDMD_STOP_COLLISIONS;
+    else if (!(t <= ra.tmax)) why = EDMD_STOP_TIME;
+    Sh.stop = why;
+    if (why != EDMD_STOP_NONE) Z.reason = why;
 }
 
 template <int NW, bool G, bool W, class AR>
 __device__ __forceinline__ void wide_loop(const EdmdConst& Cs, const AR& As, EdmdRunArgs ra,
                                           unsigned char EDMD_LDS* pool) {
     constexpr int NT = 64 * NW;
-    static_assert(NW <= 8, "a byte of the verdict per wavefront");
+    static_assert(NW <= 16, "a bit of the verdict's masks per wavefront");
     __shared__ WideShared<NW> Sh;
     const int tid = threadIdx.x, lane = tid & 63, wave = wave_in_group();
     WideCal Wc;
@@ -740,15 +793,15 @@ __device__ __forceinline__ void wide_loop(const EdmdConst& Cs, const AR& As, Edm
         Z.ntape = st->ntape;
         Z.ntrace = st->ntrace;
         Z.width = 0.25 / C.n; /* about a window's events; it adapts */
-        Z.guard = Z.tries = Z.solo = Z.halt = 0;
+        Z.guard = Z.tries = Z.halt = 0;
         Z.reason = EDMD_STOP_NONE;
         if (tid < 4) Sh.vir[tid] = st->vir[tid];
+        if (tid < NW) Sh.verdict[tid] = 0;
         if (tid == 0) {
             Sh.state = Z;
             Sh.cut = 0;
             Sh.lcount = 0;
             Sh.sums = 0;
-            Sh.verdict = 0;
             Sh.lim = R.t + Z.width;
         }
         cal_build<NT>(C, A, Wc, tid);
@@ -764,10 +817,9 @@ __device__ __forceinline__ void wide_loop(const EdmdConst& Cs, const AR& As, Edm
             const int reach = (W && !G && (C.field_on || C.damping)) ? 2 : 1;
             for (;;) {
                 /* scan (the others), the state after the last round (the
-                 * leader's first lane) */
+                 * leader) */
                 if (wave == 0) {
-                    if (lane == 0)
-                        wide_advance<NW>(C, Sh, Sh.cut, ra.stop_mask, ev_limit, coll_limit);
+                    wide_advance<NW>(C, Sh, lane, ra, ev_limit, coll_limit);
                 } else {
                     const double lim = Sh.lim;
                     for (int g0 = tid - 64; g0 - lane < Wc.m; g0 += 4 * (NT - 64)) {
@@ -779,50 +831,46 @@ __device__ __forceinline__ void wide_loop(const EdmdConst& Cs, const AR& As, Edm
                         }
                         const double least = min_f64(min_f64(k[0], k[1]), min_f64(k[2], k[3]));
                         if (!__ballot(least < lim)) continue;
+                        /* one count for the four */
+                        int all = 0;
+#pragma unroll
+                        for (int u = 0; u < 4; ++u) all += (int)__popcll(__ballot(k[u] < lim));
+                        int at = 0;
+                        if (lane == 0) at = atomicAdd(&Sh.lcount, all);
+                        at = __builtin_amdgcn_readfirstlane(at);
 #pragma unroll
                         for (int u = 0; u < 4; ++u) {
                             const uint64_t in = __ballot(k[u] < lim);
-                            if (!in) continue;
-                            int at = 0;
-                            if (lane == 0) at = atomicAdd(&Sh.lcount, (int)__popcll(in));
-                            at = __builtin_amdgcn_readfirstlane(at) +
-                                 (int)__popcll(in & (((uint64_t)1 << lane) - 1));
-                            if (k[u] < lim && at < WIDE_LIST) {
+                            const int to = at + (int)__popcll(in & (((uint64_t)1 << lane) - 1));
+                            at += (int)__popcll(in);
+                            if (k[u] < lim && to < WIDE_LIST<NW>) {
                                 const int g = g0 + u * (NT - 64);
                                 WideEntry e;
                                 e.key = k[u];
                                 e.rank = Wc.rank[g];
                                 e.p = Wc.ls > 0 ? Wc.idx[g] : g;
                                 e.aux = Wc.aux[g];
-                                Sh.list[at] = e;
+                                Sh.list[to] = e;
                             }
                         }
                     }
                 }
                 __syncthreads();
-                if (wave == 0) {
-                    WideState& Z = Sh.state;
-                    const LoopRegs& R = Z.R;
-                    int td = WT_STOP;
-                    if (Z.halt) Z.reason = EDMD_STOP_SPECIAL;
-                    else if (R.status != EDMD_DEV_OK) Z.reason = EDMD_STOP_ERROR;
-                    else if ((int64_t)R.nevents >= ev_limit) Z.reason = EDMD_STOP_EVENTS;
-                    else if (R.ncol >= coll_limit) Z.reason = EDMD_STOP_COLLISIONS;
-                    else if (!(R.t <= ra.tmax)) Z.reason = EDMD_STOP_TIME;
-                    else {
-                        td = wide_order<NW, W>(C, A, lane, Wc, Sh);
-                        if (td == WT_STOP) Z.reason = EDMD_STOP_EMPTY;
-                    }
-                    if (lane == 0) Sh.todo = td;
-                } else if (wave == 1 && !G) {
+                if (wave == NW - 1 && !G) {
                     /* the last round's sums, in its events' order */
                     const int cut = Sh.sums;
                     if (lane < 4) {
-                        double v = Sh.vir[lane];
-                        for (int m = 0; m < cut; ++m) {
-                            const double u = Sh.slot[m].vir[lane];
-                            if (Sh.slot[m].flags & WS_COLL) v += u;
+                        double u[NW];
+                        int f[NW];
+#pragma unroll
+                        for (int m = 0; m < NW; ++m) {
+                            u[m] = Sh.slot[m].vir[lane];
+                            f[m] = Sh.slot[m].flags;
                         }
+                        double v = Sh.vir[lane];
+#pragma unroll
+                        for (int m = 0; m < NW; ++m)
+                            if (m < cut && (f[m] & WS_COLL)) v += u[m];
                         Sh.vir[lane] = v;
                     }
                     if (lane == 0) {
@@ -847,17 +895,45 @@ __device__ __forceinline__ void wide_loop(const EdmdConst& Cs, const AR& As, Edm
                         Sh.sums = 0;
                     }
                 }
-                lds_barrier();
-                todo = Sh.todo;
-                if (todo == WT_SCAN) {
-                    if (tid == 0) Sh.cut = 0;
-                    lds_barrier(); /* read by all before the leader writes it again */
-                    continue;
+                if (__builtin_amdgcn_readfirstlane(Sh.stop) != EDMD_STOP_NONE) {
+                    todo = WT_STOP;
+                    break;
                 }
-                if (todo != WT_ROUND) break;
+                /* order */
+                const int n = __builtin_amdgcn_readfirstlane(Sh.lcount);
+                const bool listed = n >= 1 && n <= WIDE_LIST<NW>;
+                WidePick my;
+                bool plain0 = false;
+                if (listed) {
+                    wide_rank<NW>(Sh, lane, wave, n);
+                    lds_barrier();
+                    plain0 = wide_pick<NW, W>(C, Sh, lane, wave, n, my);
+                    if (tid == 0) {
+                        /* the next window: about two nodes a wavefront */
+                        const double width = Sh.state.width;
+                        if (n < NW + NW / 2) Sh.state.width = width * 1.2 + 1e-300;
+                        else if (n > 2 * NW + NW / 4) Sh.state.width = width * 0.85;
+                        Sh.state.tries = 0;
+                        Sh.lcount = 0;
+                    }
+                }
+                if (!plain0) {
+                    lds_barrier(); /* the picks and the count read by all */
+                    if (wave == 0) {
+                        const int td = wide_decide<NW>(C, A, lane, Wc, Sh, listed);
+                        if (lane == 0) Sh.todo = td;
+                    }
+                    lds_barrier();
+                    todo = __builtin_amdgcn_readfirstlane(Sh.todo);
+                    if (todo == WT_SCAN) {
+                        if (tid == 0) Sh.cut = 0;
+                        continue;
+                    }
+                    if (todo != WT_ROUND) break;
+                    my = Sh.pick[wave];
+                }
 
                 /* compute */
-                const WidePick& my = Sh.pick[wave];
                 EvState S;
                 int brief = 0, cellA = 0, cellB = 0, pj2 = -1;
                 if (my.plain) {
@@ -900,6 +976,7 @@ __device__ __forceinline__ void wide_loop(const EdmdConst& Cs, const AR& As, Edm
                     }
                     const int type = aux >= 0 ? EDMD_EV_COLLISION : (wall ? EDMD_EV_WALL : EDMD_EV_CELLCROSS);
                     brief = WB_INS * event_inserts(S);
+                    if (type == EDMD_EV_CELLCROSS) brief |= WB_CROSS;
                     if ((flags & (WS_OV | WS_FULL)) || !(t <= ra.tmax) || (ra.stop_mask & (1 << type)))
                         brief |= WB_LAST;
                     if (coll || wall) brief |= WB_COUNTED;
@@ -957,15 +1034,14 @@ __device__ __forceinline__ void wide_loop(const EdmdConst& Cs, const AR& As, Edm
                     if (!__ballot(on && (same || near || zero || back || late))) brief |= WB_OK;
                     if (Wc.ls > 0 && __ballot(on && share)) brief |= WB_SHARE;
                 }
-                if (lane == 0) ((unsigned char*)&Sh.verdict)[wave] = (unsigned char)brief;
+                if (lane == 0) Sh.verdict[wave] = brief;
                 lds_barrier();
 
                 /* commit */
-                const uint64_t verdict = (uint64_t)uni64((int64_t)Sh.verdict);
-                const int cut = wide_cut<NW>(verdict, __builtin_amdgcn_readfirstlane(Sh.room),
+                const WideVerdict V = wide_verdict<NW>(Sh, lane);
+                const int cut = wide_cut<NW>(V, __builtin_amdgcn_readfirstlane(Sh.room),
                                              __builtin_amdgcn_readfirstlane(Sh.croom));
-                const uint64_t done = wide_below(verdict, cut);
-                const bool share = Wc.ls > 0 && ((done >> 7) & WB_EACH) != 0;
+                const bool share = Wc.ls > 0 && (V.share & ((1u << cut) - 1)) != 0;
                 if (tid == 0) {
                     Sh.cut = cut;
                     Sh.sums = cut;
@@ -974,10 +1050,9 @@ __device__ __forceinline__ void wide_loop(const EdmdConst& Cs, const AR& As, Edm
                 if (wave < cut) {
                     const double t = my.key;
                     const int p = my.p, aux = my.aux;
-                    const uint64_t prior = wide_below(done, wave);
                     const int64_t trace = Sh.ntrace + wave;
                     int64_t rk, rx;
-                    const Leaf L = event_ranks(C, lane, S, my.paul, Sh.ctr + wide_inserts(prior), rk, rx);
+                    const Leaf L = event_ranks(C, lane, S, my.paul, Sh.ctr + wide_inserts(V, wave), rk, rx);
                     if (C.trace_cap > 0 && lane == 0 && trace < C.trace_cap) {
                         EdmdTraceRec rec;
                         rec.type = Sh.slot[wave].type;
@@ -997,7 +1072,7 @@ __device__ __forceinline__ void wide_loop(const EdmdConst& Cs, const AR& As, Edm
                         if (S.kind == EVK_CROSSING) event_enter(C, A, lane, S, S.n1);
                         if (!G && (brief & WB_TAPED) && lane == 0)
                             tape_store<W>(C, A, t, S, p, aux,
-                                          Sh.ntape + __popcll((prior >> 3) & WB_EACH));
+                                          Sh.ntape + __popc(V.taped & ((1u << wave) - 1)));
                         event_slots(A, lane, S, L, rk, rx);
                         if (Wc.ls == 0) {
                             if ((lane & 31) == 0 && (lane == 0 || S.nown == 2)) {
