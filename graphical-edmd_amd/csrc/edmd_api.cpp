@@ -157,7 +157,7 @@ struct edmd_batch {
      * Normal [0] and growing [1] launches: its wavefronts (0: not used),
      * whether its arrays are in LDS, and its dynamic LDS */
     int wide_waves[2] = {0, 0};
-    bool wide_lds[2] = {false, false};
+    int wide_place[2] = {EDMD_WIDE_GROUPS, EDMD_WIDE_GROUPS};
     size_t wide_dyn[2] = {0, 0};
     /* pinned host memory that results come back through (read_rows): two
      * buffers of stage_half bytes, allocated by the first read */
@@ -804,6 +804,22 @@ static int choose_residency(edmd_batch* b) {
     return choose_wide(b);
 }
 
+/* Wavefronts a system of so many disks (the batch's mean) gets of the 16 a CU
+ * has at the loop's registers (128), which per_cu systems share.  A round commits the events up to the first two
+ * that lie near each other, so what more wavefronts give depends on the disks:
+ * of 16 events 12 commit at 2000 disks, of 8 there 7.3, at 400 disks 3.4,
+ * while every wavefront adds to the round's length.  us a collision with 4, 8,
+ * 16 wavefronts: one system of 200 disks 3.18, 3.45, 4.25; 400 2.67, 2.52,
+ * 3.17; 1500 2.50, 1.65, 1.75; 2000 2.54, 1.57, 1.49; 4000 2.82, 1.61, 1.25;
+ * 2^18 3.85, 2.05, 1.45.  512 systems with 4, 8: 400 disks 3.38, 3.54; 1000
+ * 3.23, 2.51.  1024 systems with 4, and in the loop of one wavefront: 400
+ * disks 4.25, 6.55; 1000 3.83, 6.72. */
+static int wide_width(int per_cu, int64_t disks) {
+    if (per_cu > 2) return 4;
+    if (per_cu > 1) return disks < 500 ? 4 : 8;
+    return disks < 300 ? 4 : (disks < 1800 ? 8 : 16);
+}
+
 /* Whether the loop runs each system on a workgroup of several wavefronts
  * (edmd_wide.hip): while the device has wavefront slots to spare, i.e. for
  * batches of at most EDMD_WIDE_PER_CU systems a CU, all of them resident at
@@ -817,28 +833,36 @@ static int choose_wide(edmd_batch* b) {
     const int per_cu = (b->nsys + ncu - 1) / ncu;
     if (per_cu > EDMD_WIDE_PER_CU) return EDMD_OK;
     size_t cal = 0, both[2] = {0, 0};
+    bool flat = true;
+    int64_t disks = 0;
     for (int s = 0; s < b->nsys; s++) {
         const EdmdConst& c = b->hs[s].c;
         /* the scan of cells in LDS takes rows of whole 16-byte chunks */
         if (edmd_wide_level(&c) < 0 || c.cap > EDMD_STAGE_CAP || (c.cap & 3) != 0) return EDMD_OK;
+        flat &= edmd_wide_level(&c) == 0;
+        disks += c.n;
         const size_t w = (size_t)edmd_wide_bytes(&c);
         cal = std::max(cal, w);
         for (int g = 0; g < 2; g++)
             both[g] = std::max(both[g], (size_t)edmd_lds_layout(&c, g).total + w);
     }
-    const int waves = per_cu <= 1 ? 8 : 4;
-    for (int g = 0; g < (b->any_grow ? 2 : 1); g++) {
-        int fit = 0;
-        b->wide_lds[g] = b->use_lds;
-        b->wide_dyn[g] = b->use_lds ? both[g] : cal;
-        HIPCHK(edmd_wide_occupancy(g, b->any_walls ? 1 : 0, waves, b->wide_lds[g], b->wide_dyn[g], &fit));
-        if (fit < per_cu && b->use_lds && b->residency != EDMD_RES_LDS) {
-            b->wide_lds[g] = false;
+    const int most = wide_width(per_cu, disks / b->nsys);
+    for (int g = 0; g < (b->any_grow ? 2 : 1); g++)
+        for (int waves = most; waves >= 4 && !b->wide_waves[g]; waves /= 2) {
+            int fit = 0;
+            b->wide_place[g] = flat ? EDMD_WIDE_LEAVES : EDMD_WIDE_GROUPS;
             b->wide_dyn[g] = cal;
-            HIPCHK(edmd_wide_occupancy(g, b->any_walls ? 1 : 0, waves, 0, cal, &fit));
+            if (b->use_lds && flat) {
+                HIPCHK(edmd_wide_occupancy(g, b->any_walls ? 1 : 0, waves, EDMD_WIDE_LDS, both[g], &fit));
+                if (fit >= per_cu || b->residency == EDMD_RES_LDS) {
+                    b->wide_place[g] = EDMD_WIDE_LDS;
+                    b->wide_dyn[g] = both[g];
+                }
+            }
+            if (b->wide_place[g] != EDMD_WIDE_LDS)
+                HIPCHK(edmd_wide_occupancy(g, b->any_walls ? 1 : 0, waves, b->wide_place[g], cal, &fit));
+            if (fit >= per_cu) b->wide_waves[g] = waves;
         }
-        if (fit >= per_cu) b->wide_waves[g] = waves;
-    }
     return EDMD_OK;
 }
 
@@ -852,7 +876,7 @@ static hipError_t launch_loop(edmd_batch* b, int grow, const EdmdRunArgs& ra) {
     /* (several systems per workgroup, where asked for, is the other loop's) */
     if (b->wide_waves[g] && (grow || b->loop_wpb == 1))
         return edmd_launch_run_wide(b->d_sys, b->nsys, grow, walls, b->wide_waves[g],
-                                    b->wide_lds[g] ? 1 : 0, b->wide_dyn[g], ra, b->stream);
+                                    b->wide_place[g], b->wide_dyn[g], ra, b->stream);
     if (b->use_lds)
         return edmd_launch_run_lds(b->d_sys, b->nsys, b->max_nlev, grow, walls,
                                    b->lds_dyn[grow ? 1 : 0], ra, b->stream);

@@ -370,18 +370,18 @@ hipError_t edmd_launch_run_lds(const EdmdSys* d_sys, int nsys, int max_nlev, int
     return hipGetLastError();
 }
 
-static const void* wide_kernel(int grow, int walls, int waves, int lds) {
+static const void* wide_kernel(int grow, int walls, int waves, int place) {
     if (grow)
-        return walls ? EdmdWideVariant<true, true>::kernel(waves, lds)
-                     : EdmdWideVariant<true, false>::kernel(waves, lds);
-    return walls ? EdmdWideVariant<false, true>::kernel(waves, lds)
-                 : EdmdWideVariant<false, false>::kernel(waves, lds);
+        return walls ? EdmdWideVariant<true, true>::kernel(waves, place)
+                     : EdmdWideVariant<true, false>::kernel(waves, place);
+    return walls ? EdmdWideVariant<false, true>::kernel(waves, place)
+                 : EdmdWideVariant<false, false>::kernel(waves, place);
 }
 
-hipError_t edmd_wide_occupancy(int grow, int walls, int waves, int lds, size_t dyn_bytes,
+hipError_t edmd_wide_occupancy(int grow, int walls, int waves, int place, size_t dyn_bytes,
                                int* blocks_per_cu) {
     *blocks_per_cu = 0;
-    const void* f = wide_kernel(grow, walls, waves, lds);
+    const void* f = wide_kernel(grow, walls, waves, place);
     if (!f) return hipErrorInvalidValue;
     int dev = 0, maxblk = 0;
     hipFuncAttributes fa;
@@ -399,11 +399,11 @@ hipError_t edmd_wide_occupancy(int grow, int walls, int waves, int lds, size_t d
 }
 
 hipError_t edmd_launch_run_wide(const EdmdSys* d_sys, int nsys, int grow, int walls, int waves,
-                                int lds, size_t dyn_bytes, EdmdRunArgs ra, hipStream_t s) {
-    if (grow && walls) return EdmdWideVariant<true, true>::run(waves, lds, d_sys, nsys, dyn_bytes, ra, s);
-    if (grow) return EdmdWideVariant<true, false>::run(waves, lds, d_sys, nsys, dyn_bytes, ra, s);
-    if (walls) return EdmdWideVariant<false, true>::run(waves, lds, d_sys, nsys, dyn_bytes, ra, s);
-    return EdmdWideVariant<false, false>::run(waves, lds, d_sys, nsys, dyn_bytes, ra, s);
+                                int place, size_t dyn_bytes, EdmdRunArgs ra, hipStream_t s) {
+    if (grow && walls) return EdmdWideVariant<true, true>::run(waves, place, d_sys, nsys, dyn_bytes, ra, s);
+    if (grow) return EdmdWideVariant<true, false>::run(waves, place, d_sys, nsys, dyn_bytes, ra, s);
+    if (walls) return EdmdWideVariant<false, true>::run(waves, place, d_sys, nsys, dyn_bytes, ra, s);
+    return EdmdWideVariant<false, false>::run(waves, place, d_sys, nsys, dyn_bytes, ra, s);
 }
 
 hipError_t edmd_launch_peek(const EdmdSys* d_sys, int nsys, EdmdPeek* out, hipStream_t s) {

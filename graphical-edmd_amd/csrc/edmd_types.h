@@ -199,7 +199,11 @@ static inline EDMD_HD EdmdLdsLayout edmd_lds_layout(const EdmdConst* c, int grow
  * is too large for it. */
 #define EDMD_WIDE_FLAT 6144
 #define EDMD_WIDE_NODES 4096
-#define EDMD_WIDE_PER_CU 2 /* systems a CU takes */
+#define EDMD_WIDE_PER_CU 4 /* systems a CU takes */
+/* Where the wide loop's systems are: arrays in HBM and a window of groups (any
+ * level), arrays in LDS and a window of leaves, arrays in HBM and a window of
+ * leaves. */
+enum { EDMD_WIDE_GROUPS, EDMD_WIDE_LDS, EDMD_WIDE_LEAVES };
 /* Largest cell capacity the neighbour scan stages in LDS (six 16-byte row
  * chunks per cell), and the stage: for each of two disks every slot of nine
  * cells, and before it the room that the rows' unused slots are written to. */

@@ -20,12 +20,12 @@ struct EdmdLoopVariant {
                         EdmdRunArgs ra, hipStream_t s);
 };
 
-/* The wide loop (edmd_wide.hip): one system per workgroup of 4 or 8
- * wavefronts, its arrays in HBM or (lds) in LDS. */
+/* The wide loop (edmd_wide.hip): one system per workgroup of 4, 8 or
+ * 16 wavefronts; place: EDMD_WIDE_*. */
 template <bool G, bool W>
 struct EdmdWideVariant {
-    static const void* kernel(int waves, int lds);
-    static hipError_t run(int waves, int lds, const EdmdSys* d_sys, int nsys, size_t dyn_bytes,
+    static const void* kernel(int waves, int place);
+    static hipError_t run(int waves, int place, const EdmdSys* d_sys, int nsys, size_t dyn_bytes,
                           EdmdRunArgs ra, hipStream_t s);
 };
 

@@ -91,6 +91,7 @@ struct WideSlot {
     int32_t gp, gj;  /* window nodes of its leaves */
     double vir[4];   /* its virial terms */
     double wsum;     /* its term of the tape's virial sum */
+    double ax, ay, cx, cy, ff; /* its tape record's */
     double dp[4];    /* its momentum to the walls */
 };
 
@@ -141,6 +142,8 @@ struct WideShared {
     double vir[4];
     double red[2];
     int64_t ctr, ntape, ntrace;
+    int64_t ev_limit; /* the run's */
+    uint64_t coll_limit;
 };
 
 /* The calendar's window level in LDS (SoA: the search reads keys alone). */
@@ -692,8 +695,7 @@ __device__ __forceinline__ int wide_inserts(const WideVerdict& V, int m) {
  * round needs of it, and whether there is one. */
 template <int NW>
 __device__ __forceinline__ void wide_advance(const EdmdConst& C, WideShared<NW>& Sh, int lane,
-                                             const EdmdRunArgs& ra, int64_t ev_limit,
-                                             uint64_t coll_limit) {
+                                             const EdmdRunArgs& ra) {
     WideState& Z = Sh.state;
     LoopRegs& R = Z.R;
     const int cut = __builtin_amdgcn_readfirstlane(Sh.cut); /* 0: no round since */
@@ -739,7 +741,8 @@ __device__ __forceinline__ void wide_advance(const EdmdConst& C, WideShared<NW>&
         Z.guard = 0;
         Z.halt = halt;
     }
-    const int64_t er = ev_limit - nevents;
+    const int64_t ev_limit = Sh.ev_limit, er = ev_limit - nevents;
+    const uint64_t coll_limit = Sh.coll_limit;
     const uint64_t cr = coll_limit - ncol;
     Sh.room = er < NW ? (int)er : NW;
     Sh.croom = cr <= NW ? (int)cr : NW + 1;
@@ -756,19 +759,20 @@ __device__ __forceinline__ void wide_advance(const EdmdConst& C, WideShared<NW>&
     if (why != EDMD_STOP_NONE) Z.reason = why;
 }
 
-template <int NW, bool G, bool W, class AR>
+template <int NW, bool FLAT, bool G, bool W, class AR>
 __device__ __forceinline__ void wide_loop(const EdmdConst& Cs, const AR& As, EdmdRunArgs ra,
                                           unsigned char EDMD_LDS* pool) {
     constexpr int NT = 64 * NW;
     static_assert(NW <= 16, "a bit of the verdict's masks per wavefront");
     __shared__ WideShared<NW> Sh;
-    const int tid = threadIdx.x, lane = tid & 63, wave = wave_in_group();
+    const int tid0 = threadIdx.x;
+    int tid = tid0, lane = tid & 63, wave = wave_in_group();
     WideCal Wc;
     {
         const EdmdConst& C = opaque(Cs);
         const AR& A = opaque(As);
         const EdmdState* st = A.st;
-        Wc.ls = edmd_wide_level(&C);
+        Wc.ls = FLAT ? 0 : edmd_wide_level(&C);
         Wc.m = C.lsize[Wc.ls];
         Wc.key = (double EDMD_LDS*)pool;
         Wc.rank = (int64_t EDMD_LDS*)(pool + (size_t)Wc.m * 8);
@@ -799,6 +803,8 @@ __device__ __forceinline__ void wide_loop(const EdmdConst& Cs, const AR& As, Edm
         if (tid < NW) Sh.verdict[tid] = 0;
         if (tid == 0) {
             Sh.state = Z;
+            Sh.ev_limit = st->ev_limit < ra.max_events ? st->ev_limit : ra.max_events;
+            Sh.coll_limit = st->coll_limit < ra.max_coll ? st->coll_limit : ra.max_coll;
             Sh.cut = 0;
             Sh.lcount = 0;
             Sh.sums = 0;
@@ -809,17 +815,16 @@ __device__ __forceinline__ void wide_loop(const EdmdConst& Cs, const AR& As, Edm
     for (;;) {
         int todo;
         {
-            const EdmdConst& C = opaque(Cs);
-            const AR& A = opaque(As);
-            EdmdState* st = A.st;
-            const int64_t ev_limit = st->ev_limit < ra.max_events ? st->ev_limit : ra.max_events;
-            const uint64_t coll_limit = st->coll_limit < ra.max_coll ? st->coll_limit : ra.max_coll;
-            const int reach = (W && !G && (C.field_on || C.damping)) ? 2 : 1;
             for (;;) {
+                const EdmdConst& C = opaque(Cs);
+                const AR& A = opaque(As);
+                /* what follows from the thread or the system's record alone is
+                 * made or read again each round, not held in registers */
+                asm volatile("" : "+v"(tid), "+v"(lane), "+s"(wave));
                 /* scan (the others), the state after the last round (the
                  * leader) */
                 if (wave == 0) {
-                    wide_advance<NW>(C, Sh, lane, ra, ev_limit, coll_limit);
+                    wide_advance<NW>(C, Sh, lane, ra);
                 } else {
                     const double lim = Sh.lim;
                     for (int g0 = tid - 64; g0 - lane < Wc.m; g0 += 4 * (NT - 64)) {
@@ -857,6 +862,7 @@ __device__ __forceinline__ void wide_loop(const EdmdConst& Cs, const AR& As, Edm
                 }
                 __syncthreads();
                 if (wave == NW - 1 && !G) {
+                    EdmdState* st = A.st;
                     /* the last round's sums, in its events' order */
                     const int cut = Sh.sums;
                     if (lane < 4) {
@@ -940,10 +946,29 @@ __device__ __forceinline__ void wide_loop(const EdmdConst& Cs, const AR& As, Edm
                     const double t = my.key;
                     const int p = my.p, aux = my.aux;
                     event_open<G, W>(C, A, lane, t, p, aux, S);
+                    if (!G && S.kind == EVK_COLLISION) {
+                        /* what only the sums and the tape need waits in LDS */
+                        WideSlot& me = Sh.slot[wave];
+                        if (lane < 4) {
+                            const double u = (lane & 1) == 0 ? S.dx : S.dy;
+                            const double v = (lane == 0 || lane == 3) ? S.dx : S.dy;
+                            me.vir[lane] = S.w * u * v;
+                        }
+                        if (lane == 0 && C.tape_cap > 0) {
+                            me.wsum = S.w * (S.dx * S.dx + S.dy * S.dy);
+                            me.ax = S.dx;
+                            me.ay = S.dy;
+                            me.cx = S.dvx;
+                            me.cy = S.dvy;
+                            me.ff = S.ff;
+                        }
+                    }
                     PathWindow P;
                     const int pj = S.nown == 2 ? aux : -1;
-                    if (Wc.ls > 0) path_window(C, A, lane, Wc.ls, p, pj, P);
+                    if (NW <= 8 && Wc.ls > 0) path_window(C, A, lane, Wc.ls, p, pj, P);
                     event_predict<G, W, true>(C, A, lane, t, S, Sh.cand[wave]);
+                    /* (16 wavefronts hide its latency and have no registers for it) */
+                    if (NW > 8 && Wc.ls > 0) path_window(C, A, lane, Wc.ls, p, pj, P);
                     /* the leaf's key and code do not depend on the counter:
                      * the ranks of this disk's slots compare alike for any */
                     int64_t rk, rx;
@@ -983,16 +1008,9 @@ __device__ __forceinline__ void wide_loop(const EdmdConst& Cs, const AR& As, Edm
                     if (C.tape_cap > 0 && !G && (coll || (wall && S.d != 2))) brief |= WB_TAPED;
                     pj2 = pj;
                     WideSlot& me = Sh.slot[wave];
-                    if (coll && !G && lane < 4) {
-                        const double u = (lane & 1) == 0 ? S.dx : S.dy;
-                        const double v = (lane == 0 || lane == 3) ? S.dx : S.dy;
-                        me.vir[lane] = S.w * u * v;
-                    }
                     if (lane == 0) {
                         me.key = t;
                         me.lim = lim;
-                        if (coll && !G && C.tape_cap > 0)
-                            me.wsum = S.w * (S.dx * S.dx + S.dy * S.dy);
                         if (wall) {
                             me.dp[0] = S.dp;
                             me.dp[1] = S.dpl;
@@ -1013,6 +1031,7 @@ __device__ __forceinline__ void wide_loop(const EdmdConst& Cs, const AR& As, Edm
 
                 /* check: lane k tests the event of wavefront k < this one's */
                 if (my.plain) {
+                    const int reach = (W && !G && (C.field_on || C.damping)) ? 2 : 1;
                     const int k = lane < wave ? lane : 0;
                     const WideSlot& o = Sh.slot[k];
                     const WidePick& ok = Sh.pick[k];
@@ -1070,9 +1089,18 @@ __device__ __forceinline__ void wide_loop(const EdmdConst& Cs, const AR& As, Edm
                             fly_neighbours(C, A, lane, t, S, Sh.cand[wave]);
                         }
                         if (S.kind == EVK_CROSSING) event_enter(C, A, lane, S, S.n1);
-                        if (!G && (brief & WB_TAPED) && lane == 0)
+                        if (!G && (brief & WB_TAPED) && lane == 0) {
+                            if (S.kind == EVK_COLLISION) {
+                                const WideSlot& me = Sh.slot[wave];
+                                S.dx = me.ax;
+                                S.dy = me.ay;
+                                S.dvx = me.cx;
+                                S.dvy = me.cy;
+                                S.ff = me.ff;
+                            }
                             tape_store<W>(C, A, t, S, p, aux,
                                           Sh.ntape + __popc(V.taped & ((1u << wave) - 1)));
+                        }
                         event_slots(A, lane, S, L, rk, rx);
                         if (Wc.ls == 0) {
                             if ((lane & 31) == 0 && (lane == 0 || S.nown == 2)) {
@@ -1197,23 +1225,21 @@ __device__ __forceinline__ void wide_loop(const EdmdConst& Cs, const AR& As, Edm
     cal_close<NT>(C, A, Wc, tid);
 }
 
-/* LDS = false: the system's arrays in HBM, the calendar's window level in
- * the dynamic LDS; LDS = true: the arrays in LDS as well (edmd_lds.h).  Two
- * wavefronts a SIMD: one workgroup of eight, or two of four; without the bound
- * the compiler gave four wavefronts every register, and one CU held one
- * workgroup (512 systems of 400 disks, 4000 collisions each: 18 ms in the loop
- * of one wavefront that ran instead, 12.3 ms here). */
-template <int NW, bool G, bool W>
-__global__ __launch_bounds__(64 * NW, 2) void k_wide(const EdmdSys* __restrict__ systems,
-                                                     EdmdRunArgs ra) {
+/* The arrays in HBM, the calendar's window level in the dynamic LDS.  FLAT:
+ * the window is of leaves for every system, so none of the code for the
+ * levels between, whose path of nodes took 30 registers.  REGNOTE */
+template <int NW, bool FLAT, bool G, bool W>
+__global__ __launch_bounds__(64 * NW, (FLAT || NW > 8) ? 4 : 2) void k_wide(
+    const EdmdSys* __restrict__ systems, EdmdRunArgs ra) {
     extern __shared__ __align__(64) unsigned char lds_pool[];
     const EdmdSys& S = systems[blockIdx.x];
     if ((uni(S.a.st->growing) != 0) != G) return;
-    wide_loop<NW, G, W>(S.c, S.a, ra, (unsigned char EDMD_LDS*)lds_pool);
+    wide_loop<NW, FLAT, G, W>(S.c, S.a, ra, (unsigned char EDMD_LDS*)lds_pool);
 }
 
+/* The arrays in LDS as well (edmd_lds.h). */
 template <int NW, bool G, bool W>
-__global__ __launch_bounds__(64 * NW, 2) void k_wide_lds(const EdmdSys* __restrict__ systems,
+__global__ __launch_bounds__(64 * NW, 4) void k_wide_lds(const EdmdSys* __restrict__ systems,
                                                          EdmdRunArgs ra) {
     extern __shared__ __align__(64) unsigned char lds_pool[];
     const EdmdSys& S = systems[blockIdx.x];
@@ -1224,24 +1250,32 @@ __global__ __launch_bounds__(64 * NW, 2) void k_wide_lds(const EdmdSys* __restri
     __syncthreads();
     lds_system<true, G, 64 * NW>(S.c, S.a, A, threadIdx.x);
     __syncthreads();
-    wide_loop<NW, G, W>(S.c, A, ra, base + used);
+    wide_loop<NW, true, G, W>(S.c, A, ra, base + used);
     __syncthreads();
     lds_system<false, G, 64 * NW>(S.c, S.a, A, threadIdx.x);
+}
+
+template <int NW, bool G, bool W>
+const void* kernel_of(int place) {
+    if (place == EDMD_WIDE_LDS) return (const void*)k_wide_lds<NW, G, W>;
+    if (place == EDMD_WIDE_LEAVES) return (const void*)k_wide<NW, true, G, W>;
+    return (const void*)k_wide<NW, false, G, W>;
 }
 
 } // namespace
 
 template <bool G, bool W>
-const void* EdmdWideVariant<G, W>::kernel(int waves, int lds) {
-    if (waves == 8) return lds ? (const void*)k_wide_lds<8, G, W> : (const void*)k_wide<8, G, W>;
-    if (waves == 4) return lds ? (const void*)k_wide_lds<4, G, W> : (const void*)k_wide<4, G, W>;
+const void* EdmdWideVariant<G, W>::kernel(int waves, int place) {
+    if (waves == 16) return kernel_of<16, G, W>(place);
+    if (waves == 8) return kernel_of<8, G, W>(place);
+    if (waves == 4) return kernel_of<4, G, W>(place);
     return nullptr;
 }
 
 template <bool G, bool W>
-hipError_t EdmdWideVariant<G, W>::run(int waves, int lds, const EdmdSys* d_sys, int nsys,
+hipError_t EdmdWideVariant<G, W>::run(int waves, int place, const EdmdSys* d_sys, int nsys,
                                       size_t dyn_bytes, EdmdRunArgs ra, hipStream_t s) {
-    const void* f = kernel(waves, lds);
+    const void* f = kernel(waves, place);
     if (!f) return hipErrorInvalidValue;
     ra.nsys = nsys;
     void* args[] = {(void*)&d_sys, (void*)&ra};
