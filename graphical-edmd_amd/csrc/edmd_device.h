@@ -195,12 +195,18 @@ __device__ __forceinline__ void min_image(const EdmdConst& C, double& dx, double
     else if (dy < -C.mihy) dy += C.Ly;
 }
 
-/* edmd_exp (e^x, the library's own) is in edmd_math.h. */
+/* edmd_exp (e^x, the library's own) is in edmd_math.h.  The event loops call
+ * the functions below, which only damping and the circular wall need: inlined
+ * at each of their places, their constants alone filled the scalar registers,
+ * and the loops for walls spilled 300 of them, run or not: one wavefront a system, 2048
+ * systems of 500 disks between walls under the field, 11.2 us a collision
+ * inlined, 10.5 called. */
+__device__ __noinline__ double edmd_exp_call(double x) { return edmd_exp(x); }
 
 /* log x from log m = 2 atanh s = 2(s + s^3/3 + ... + s^23/23),
  * s = (m - 1)/(m + 1), x = m 2^e with m in [sqrt(1/2), sqrt(2)), plus
  * e ln2 in two parts; within 4 ulp, the oracle's steps. */
-__device__ __forceinline__ double edmd_log(double x) {
+__device__ __noinline__ double edmd_log(double x) {
     if (x != x || x < 0) return __builtin_nan("");
     if (x == 0) return -__builtin_huge_val();
     if (x == __builtin_huge_val()) return x;
@@ -273,6 +279,13 @@ __device__ __forceinline__ double edmd_atan2(double y, double x) {
     return __builtin_signbit(y) ? -a : a;
 }
 
+/* The unit vector (x: cos, y: sin) along (x, y), by its angle. */
+__device__ __noinline__ double2 circle_normal(double y, double x) {
+    double2 n;
+    edmd_sincos(edmd_atan2(y, x), n.y, n.x);
+    return n;
+}
+
 /* The quartic of the circular wall under the field (quartic.c:27-158):
  * Ferrari's method through the cubic resolvent, step for step as there,
  * with this library's own acos (atan2 of sqrt((1 - t)(1 + t)) and t), cos
@@ -319,8 +332,8 @@ __device__ __forceinline__ unsigned edmd_solve_p3(double* x, double a, double b,
 
 /* The smallest real root above 1e-9 of a t^4 + b t^3 + c t^2 + d t + e,
  * 1e10 when there is none (smallestRoot, quartic.c:143-157). */
-__device__ __forceinline__ double edmd_smallest_root(double a, double b, double c, double d,
-                                                     double e) {
+__device__ __noinline__ double edmd_smallest_root(double a, double b, double c, double d,
+                                                  double e) {
     const double qa = b / a, qb = c / a, qc = d / a, qd = e / a;
     const double a3 = -qb;
     const double b3 = qa * qc - 4. * qd;
@@ -687,7 +700,7 @@ __device__ __forceinline__ void fly_v(const EdmdConst& C, double t, double& x, d
         const double dt = t - tl;
         tl = t;
         const double g = C.gamma;
-        const double ex = edmd_exp(-g * dt);
+        const double ex = edmd_exp_call(-g * dt);
         x += vx / g * (1 - ex);
         y += vy / g * (1 - ex);
         vx *= ex;

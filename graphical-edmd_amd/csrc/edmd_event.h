@@ -225,8 +225,8 @@ __device__ __forceinline__ void event_open(const EdmdConst& C, const AR& A, int 
                 else vy = -vy + 2 * S.vr;
             } else {
                 /* the circle: reflected about the normal, 2 vr added along it */
-                double nx, ny;
-                edmd_sincos(edmd_atan2(y - C.halfLx, x - C.halfLx), ny, nx);
+                const double2 nrm = circle_normal(y - C.halfLx, x - C.halfLx);
+                const double nx = nrm.x, ny = nrm.y;
                 const double mix = -(1 + C.res_wall) * (vx * nx + vy * ny);
                 vx += (mix - 2 * S.vr) * nx;
                 vy += (mix - 2 * S.vr) * ny;
@@ -271,8 +271,8 @@ __device__ __forceinline__ void event_open(const EdmdConst& C, const AR& A, int 
                 /* the circle (EDMD.c:3441-3454): the normal velocity reversed
                  * times resW (thermal: both components drawn), |m mix| to the
                  * wall */
-                double nx, ny;
-                edmd_sincos(edmd_atan2(y - C.halfLx, x - C.halfLx), ny, nx);
+                const double2 nrm = circle_normal(y - C.halfLx, x - C.halfLx);
+                const double nx = nrm.x, ny = nrm.y;
                 const double mix = -(1 + C.res_wall) * (vx * nx + vy * ny);
                 if (C.thermal_wall) {
                     vx = -nx * mt_drand0(A, lane, C.temperature);
