@@ -5,14 +5,17 @@
 #include <hip/hip_runtime.h>
 
 #include <math.h>
+#include <stddef.h>
 #include <stdarg.h>
 #include <stdio.h>
 #include <stdlib.h>
 #include <string.h>
 
 #include <algorithm>
+#include <initializer_list>
 #include <mutex>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "../../include/edmd.h"
@@ -511,25 +514,30 @@ static int batch_predict_all(edmd_batch* b) {
     return EDMD_OK;
 }
 
+#define EDMD_STAGE_BYTES (512u << 10)
+
+/* The batch's pinned memory, two halves, where there is room for it. */
+static void stage_open(edmd_batch* b) {
+    if (b->stage) return;
+    const size_t need = std::max((size_t)b->max_n * sizeof(EdmdPart), b->nsys * sizeof(EdmdState));
+    b->stage_half = std::min((need + 4095) & ~(size_t)4095, (size_t)EDMD_STAGE_BYTES);
+    if (hipHostMalloc((void**)&b->stage, 2 * b->stage_half, 0) != hipSuccess) {
+        (void)hipGetLastError();
+        b->stage = nullptr;
+    }
+}
+
 /* Rows [0, n) of device array src, handed to put(first, rows, count) piece by
  * piece, in order.  They come through pinned memory of the batch's own, the
  * next piece on its way while put works on one: into ordinary memory a copy of
  * 4096 disks (256 KB) took 116 us, of 2^20 13.9 ms, into pinned memory 13 us
  * and 1.2 ms.  Pieces of half a megabyte stay in the caches; without room for
  * pinned memory the copy goes to ordinary memory as one piece. */
-#define EDMD_STAGE_BYTES (512u << 10)
 template <class R, class F>
 static int read_rows(edmd_batch* b, const R* src, size_t n, F&& put) {
     if (n == 0) return EDMD_OK;
     std::lock_guard<std::mutex> only(b->stage_lock);
-    if (!b->stage) {
-        const size_t need = std::max((size_t)b->max_n * sizeof(EdmdPart), b->nsys * sizeof(EdmdState));
-        b->stage_half = std::min((need + 4095) & ~(size_t)4095, (size_t)EDMD_STAGE_BYTES);
-        if (hipHostMalloc((void**)&b->stage, 2 * b->stage_half, 0) != hipSuccess) {
-            (void)hipGetLastError();
-            b->stage = nullptr;
-        }
-    }
+    stage_open(b);
     if (!b->stage) {
         std::vector<R> rows(n);
         HIPCHK(hipStreamSynchronize(b->stream));
@@ -559,11 +567,96 @@ static int read_all(edmd_batch* b, R* dst, const R* src, size_t n) {
     return read_rows(b, src, n, [&](size_t at, const R* r, size_t k) { memcpy((void*)(dst + at), r, k * sizeof(R)); });
 }
 
-/* One member of the rows, into dst (if there is one). */
-template <class R, class M, class T>
-static void column(T* dst, const R* rows, size_t n, M R::*member) {
-    if (dst)
-        for (size_t i = 0; i < n; i++) dst[i] = rows[i].*member;
+/* A member of rows: its place, width (EdmdColumns) and the caller's array, or
+ * none. */
+struct Column {
+    size_t src;
+    int kind;
+    void* out;
+};
+
+/* A member of n rows of type R, from its place in the first, as an array. */
+template <class R, class T>
+static void pick(char* out, const char* at, size_t n) {
+    using O = typename std::conditional<sizeof(T) == 2, int32_t, T>::type;
+    O* const to = (O*)out;
+    for (size_t i = 0; i < n; i++, at += sizeof(R)) to[i] = *(const T*)at;
+}
+
+/* Members of rows [0, n) of device array src, into the caller's arrays.  From
+ * EDMD_COLUMNS_FROM rows on the card lays them out as arrays (k_columns), in
+ * pieces through the batch's pinned memory, the next on its way while one is
+ * copied; fewer rows come as they are.  us for the state of 1000 disks 16.6
+ * as rows and 19.0 as arrays, of 2000 20.7 and 21.3, 4000 29.9 and 25.3, 65536
+ * 243 and 178, 300000 1046 and 734; for the events 13.3 and 16.7 (2000), 17.0
+ * and 18.5 (4000), 22.2 and 20.7 (7000), 425 and 347 (300000). */
+#define EDMD_COLUMNS_FROM 4096
+template <class R>
+static int read_columns(edmd_batch* b, const R* src, size_t n, std::initializer_list<Column> all) {
+    EdmdColumns cols;
+    memset(&cols, 0, sizeof cols);
+    cols.row = (int)sizeof(R);
+    char* out[EDMD_COLUMNS];
+    size_t wide[EDMD_COLUMNS], each = 0;
+    for (const Column& c : all) {
+        if (!c.out) continue;
+        cols.src[cols.n] = (int)c.src;
+        cols.kind[cols.n] = c.kind;
+        out[cols.n] = (char*)c.out;
+        wide[cols.n] = c.kind == 8 ? 8 : 4;
+        each += wide[cols.n++];
+    }
+    if (n == 0 || cols.n == 0) return EDMD_OK;
+    std::lock_guard<std::mutex> only(b->stage_lock);
+    stage_open(b);
+    if (!b->stage || n < EDMD_COLUMNS_FROM) {
+        /* picked out here, a member at a time */
+        std::vector<R> own;
+        const char* rows = b->stage;
+        if (!b->stage) {
+            own.resize(n);
+            rows = (const char*)own.data();
+            HIPCHK(hipStreamSynchronize(b->stream));
+            HIPCHK(hipMemcpy(own.data(), src, n * sizeof(R), hipMemcpyDeviceToHost));
+        } else {
+            HIPCHK(hipMemcpyAsync(b->stage, src, n * sizeof(R), hipMemcpyDeviceToHost, b->stream));
+            HIPCHK(hipStreamSynchronize(b->stream));
+        }
+        for (int c = 0; c < cols.n; c++) {
+            const char* at = rows + cols.src[c];
+            if (cols.kind[c] == 8) pick<R, double>(out[c], at, n);
+            else if (cols.kind[c] == 4) pick<R, int32_t>(out[c], at, n);
+            else pick<R, int16_t>(out[c], at, n);
+        }
+        return EDMD_OK;
+    }
+    /* whole lines of every array: at least 64 rows of 56 bytes and the arrays'
+     * starts in the smallest stage */
+    const size_t per = (b->stage_half - 64 * EDMD_COLUMNS) / each & ~(size_t)15;
+    auto place = [&](size_t k) {
+        size_t at = 0;
+        for (int c = 0; c < cols.n; c++) {
+            cols.dst[c] = (uint32_t)at;
+            at += (k * wide[c] + 63) & ~(size_t)63;
+        }
+    };
+    auto piece = [&](size_t at) { return std::min(per, n - at); };
+    auto fetch = [&](size_t at, int k) {
+        place(piece(at));
+        return edmd_launch_columns(src + at, (int64_t)piece(at), b->stage + k * b->stage_half, cols,
+                                   b->stream);
+    };
+    HIPCHK(fetch(0, 0));
+    int k = 0;
+    for (size_t at = 0; at < n; at += per, k ^= 1) {
+        HIPCHK(hipStreamSynchronize(b->stream));
+        if (at + per < n) HIPCHK(fetch(at + per, k ^ 1));
+        place(piece(at));
+        for (int c = 0; c < cols.n; c++)
+            memcpy(out[c] + at * wide[c], b->stage + k * b->stage_half + cols.dst[c],
+                   piece(at) * wide[c]);
+    }
+    return EDMD_OK;
 }
 
 static int check_status(edmd_batch* b) {
@@ -1250,27 +1343,21 @@ static int d2h(T* dst, const T* src, size_t n) {
     return EDMD_OK;
 }
 
-template <class T>
-static T* from(T* p, size_t at) {
-    return p ? p + at : nullptr;
-}
-
 extern "C" int edmd_batch_get_state(edmd_batch* b, int s, double* x, double* y, double* vx,
                                     double* vy, double* t_local, uint32_t* coll, int32_t* cx,
                                     int32_t* cy) {
     int rc = sys_check(b, s);
     if (rc) return rc;
     const HostSys& h = b->hs[s];
-    return read_rows(b, b->part + h.p0, (size_t)h.c.n, [&](size_t at, const EdmdPart* r, size_t n) {
-        column(from(x, at), r, n, &EdmdPart::x);
-        column(from(y, at), r, n, &EdmdPart::y);
-        column(from(vx, at), r, n, &EdmdPart::vx);
-        column(from(vy, at), r, n, &EdmdPart::vy);
-        column(from(t_local, at), r, n, &EdmdPart::tl);
-        column(from(coll, at), r, n, &EdmdPart::coll);
-        column(from(cx, at), r, n, &EdmdPart::cx);
-        column(from(cy, at), r, n, &EdmdPart::cy);
-    });
+    return read_columns(b, b->part + h.p0, (size_t)h.c.n,
+                        {{offsetof(EdmdPart, x), 8, x},
+                         {offsetof(EdmdPart, y), 8, y},
+                         {offsetof(EdmdPart, vx), 8, vx},
+                         {offsetof(EdmdPart, vy), 8, vy},
+                         {offsetof(EdmdPart, tl), 8, t_local},
+                         {offsetof(EdmdPart, coll), 4, coll},
+                         {offsetof(EdmdPart, cx), 2, cx},
+                         {offsetof(EdmdPart, cy), 2, cy}});
 }
 
 extern "C" int edmd_batch_get_radii(edmd_batch* b, int s, double* rad) {
@@ -1278,21 +1365,18 @@ extern "C" int edmd_batch_get_radii(edmd_batch* b, int s, double* rad) {
     if (rc) return rc;
     if (!rad) return fail(EDMD_ERR_ARG, "null output");
     const HostSys& h = b->hs[s];
-    return read_rows(b, b->part + h.p0, (size_t)h.c.n, [&](size_t at, const EdmdPart* r, size_t n) {
-        column(rad + at, r, n, &EdmdPart::rad);
-    });
+    return read_columns(b, b->part + h.p0, (size_t)h.c.n, {{offsetof(EdmdPart, rad), 8, rad}});
 }
 
 static int read_events(edmd_batch* b, int s, double* t_coll, int32_t* partner, double* t_cross,
                        int32_t* dir, uint32_t* coll_actual) {
     const HostSys& h = b->hs[s];
-    return read_rows(b, b->ev + h.p0, (size_t)h.c.n, [&](size_t at, const EdmdEv* r, size_t n) {
-        column(from(t_coll, at), r, n, &EdmdEv::tcoll);
-        column(from(partner, at), r, n, &EdmdEv::partner);
-        column(from(t_cross, at), r, n, &EdmdEv::tcross);
-        column(from(dir, at), r, n, &EdmdEv::dir);
-        column(from(coll_actual, at), r, n, &EdmdEv::cact);
-    });
+    return read_columns(b, b->ev + h.p0, (size_t)h.c.n,
+                        {{offsetof(EdmdEv, tcoll), 8, t_coll},
+                         {offsetof(EdmdEv, partner), 4, partner},
+                         {offsetof(EdmdEv, tcross), 8, t_cross},
+                         {offsetof(EdmdEv, dir), 4, dir},
+                         {offsetof(EdmdEv, cact), 4, coll_actual}});
 }
 
 extern "C" int edmd_batch_get_events(edmd_batch* b, int s, double* t_coll, int32_t* partner,

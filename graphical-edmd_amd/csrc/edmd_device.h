@@ -198,9 +198,9 @@ __device__ __forceinline__ void min_image(const EdmdConst& C, double& dx, double
 /* edmd_exp (e^x, the library's own) is in edmd_math.h.  The event loops call
  * the functions below, which only damping and the circular wall need: inlined
  * at each of their places, their constants alone filled the scalar registers,
- * and the loops for walls spilled 300 of them, run or not: one wavefront a system, 2048
- * systems of 500 disks between walls under the field, 11.2 us a collision
- * inlined, 10.5 called. */
+ * and the loops for walls spilled 300 of them, run or not: 2048 systems of 500
+ * disks between walls under the field took 11.2 us a collision with them
+ * inlined, 10.5 with calls. */
 __device__ __noinline__ double edmd_exp_call(double x) { return edmd_exp(x); }
 
 /* log x from log m = 2 atanh s = 2(s + s^3/3 + ... + s^23/23),

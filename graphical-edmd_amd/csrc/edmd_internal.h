@@ -79,6 +79,17 @@ hipError_t edmd_launch_deriv_init(const EdmdSys* d_sys, int nsys, int max_n, int
                                   hipStream_t s);
 hipError_t edmd_launch_deriv_flush(const EdmdSys* d_sys, int nsys, int max_n, int mode,
                                    hipStream_t s);
+/* Members of rows of `row` bytes, to be laid out as arrays: member c is at
+ * src[c] of its row, of `kind` 8 or 4 bytes (2: two, written as four with its
+ * sign), and its array starts dst[c] bytes into the output. */
+#define EDMD_COLUMNS 8
+struct EdmdColumns {
+    int row, n;
+    int src[EDMD_COLUMNS], kind[EDMD_COLUMNS];
+    uint32_t dst[EDMD_COLUMNS];
+};
+hipError_t edmd_launch_columns(const void* rows, int64_t n, void* out, const EdmdColumns& cols,
+                               hipStream_t s);
 /* Spans of device memory copied together; sizes are multiples of 4 bytes,
  * addresses of 16. */
 #define EDMD_SPANS 11
