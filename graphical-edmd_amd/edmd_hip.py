@@ -401,7 +401,7 @@ class System:
 
 
 class Batch:
-    """Many independent systems, one wavefront each."""
+    """Many independent systems in one launch."""
 
     def __init__(self, states, per_system=None, **kw):
         """kw: descriptor fields for every system; per_system: field -> list

@@ -286,8 +286,9 @@ int edmd_queue_remove(edmd_ctx* ctx, int kind, int i);
 /* ---- batched replicas ---------------------------------------------------- */
 typedef struct edmd_batch edmd_batch;
 
-/* nsys independent systems of any sizes, one wavefront each in one
- * persistent launch. */
+/* nsys independent systems of any sizes, in one persistent launch: each on
+ * 4 to 16 wavefronts in batches of up to four systems per compute unit, on
+ * one in larger ones. */
 int edmd_batch_create(const edmd_system_desc* descs, int nsys, edmd_batch** out);
 int edmd_batch_destroy(edmd_batch* b);
 /* Every system runs until its own event counter reaches max_events or its
@@ -333,7 +334,7 @@ int edmd_batch_set_stream(edmd_batch* b, void* stream);
 /* Where the event loop keeps each system's arrays while it runs.  No
  * counterpart in the reference (one system in host memory): the batched
  * form of its step loop, mainLoop (EDMD.c:5595-5630).  EDMD_RES_HBM: in
- * device memory, one wavefront per system.  EDMD_RES_LDS: each system's
+ * device memory.  EDMD_RES_LDS: each system's
  * particles, event slots, calendar, ranks and cell lists are copied into
  * its workgroup's LDS when a run launches and back when it stops (calendar
  * depth <= 2 and the largest system's arrays within one workgroup's LDS,
@@ -373,8 +374,8 @@ int edmd_batch_set_screen(edmd_batch* b, int mode);
 int edmd_batch_screen_stats(edmd_batch* b, uint64_t* marks, uint64_t* solved, uint64_t* misses);
 
 /* Systems per workgroup of the event loop with arrays in HBM, no
- * counterpart in the reference: 1 (default), 2 or 4, one wavefront per
- * system either way.  More than one only for calendars of depth <= 2 (up to
+ * counterpart in the reference: 1 (default), 2 or 4; with more than one each
+ * system runs on one wavefront.  More than one only for calendars of depth <= 2 (up to
  * 4096 disks) without walls, field or damping; the growing systems' launch
  * always takes one.  Results do not depend on it. */
 int edmd_batch_set_loop_waves(edmd_batch* b, int systems_per_group);

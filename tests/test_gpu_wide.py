@@ -1,9 +1,10 @@
 """The event loop of one system on a workgroup of several wavefronts against
 the oracle and against the loop of one wavefront, bit for bit.
 
-A batch of at most one system per compute unit runs eight wavefronts a
-system, of at most two four, larger ones the loop of one wavefront; the
-results may not depend on it.  The reference runs one event at a time
+Small disk counts here run four wavefronts a system in batches of up to four
+systems per compute unit; the other widths, and those batches against the loop
+of one wavefront, are in test_gpu_wide_widths.py.  The results may not depend
+on it.  The reference runs one event at a time
 (mainLoop, EDMD.c:5595-5630)."""
 import numpy as np
 import pytest
@@ -68,7 +69,7 @@ def test_cell_capacities_match_oracle(gpu, oracle, cap):
 def test_equal_times_agree(gpu):
     """Columns of a square grid closing on one another at one speed: hundreds
     of collisions and crossings at exactly equal times, more than a round
-    takes; against the loop of one wavefront (a batch of 600)."""
+    takes; in batches of 1, 300 and 600."""
     side = 20
     k = np.arange(side * side)
     L = 32.0
@@ -109,8 +110,7 @@ VARIANTS = {
 
 @pytest.mark.parametrize("name", list(VARIANTS))
 def test_loop_widths_agree(gpu, name):
-    """The same systems in batches of 3 (eight wavefronts a system), 300 (four)
-    and 600 (one): states, counters, sums and thermo rows alike."""
+    """The same systems in batches of 3, 300 and 600: states, counters, sums and thermo rows alike."""
     kw = VARIANTS[name]
     if "vr" in kw:
         base = [gpu.init_random(n, 0.4, seed=n) for n in (70, 120, 200)]
