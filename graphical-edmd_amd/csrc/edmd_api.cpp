@@ -898,14 +898,15 @@ static int choose_residency(edmd_batch* b) {
 }
 
 /* Wavefronts a system of so many disks (the batch's mean) gets of the 16 a CU
- * has at the loop's registers (128), which per_cu systems share.  A round commits the events up to the first two
- * that lie near each other, so what more wavefronts give depends on the disks:
+ * has at the loop's registers (128), which per_cu systems share.  A round
+ * commits the events up to the first two that lie near each other, so what
+ * more wavefronts give depends on the disks:
  * of 16 events 12 commit at 2000 disks, of 8 there 7.3, at 400 disks 3.4,
  * while every wavefront adds to the round's length.  us a collision with 4, 8,
  * 16 wavefronts: one system of 200 disks 3.18, 3.45, 4.25; 400 2.67, 2.52,
  * 3.17; 1500 2.50, 1.65, 1.75; 2000 2.54, 1.57, 1.49; 4000 2.82, 1.61, 1.25;
- * 2^18 3.85, 2.05, 1.45.  512 systems with 4, 8: 400 disks 3.38, 3.54; 1000
- * 3.23, 2.51.  1024 systems with 4, and in the loop of one wavefront: 400
+ * 2^18 3.85, 2.05, 1.45.  512 systems with 4, 8, arrays in HBM: 400 disks
+ * 3.38, 3.54; 1000 3.23, 2.51.  1024 systems with 4, and in the loop of one wavefront: 400
  * disks 4.25, 6.55; 1000 3.83, 6.72. */
 static int wide_width(int per_cu, int64_t disks) {
     if (per_cu > 2) return 4;
@@ -934,10 +935,9 @@ static int choose_wide(edmd_batch* b) {
         if (edmd_wide_level(&c) < 0 || c.cap > EDMD_STAGE_CAP || (c.cap & 3) != 0) return EDMD_OK;
         flat &= edmd_wide_level(&c) == 0;
         disks += c.n;
-        const size_t w = (size_t)edmd_wide_bytes(&c);
-        cal = std::max(cal, w);
+        cal = std::max(cal, (size_t)edmd_wide_bytes(&c, 0));
         for (int g = 0; g < 2; g++)
-            both[g] = std::max(both[g], (size_t)edmd_lds_layout(&c, g).total + w);
+            both[g] = std::max(both[g], (size_t)edmd_lds_layout(&c, g).total + (size_t)edmd_wide_bytes(&c, 1));
     }
     const int most = wide_width(per_cu, disks / b->nsys);
     for (int g = 0; g < (b->any_grow ? 2 : 1); g++)

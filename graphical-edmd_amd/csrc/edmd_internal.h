@@ -41,9 +41,9 @@ hipError_t edmd_lds_occupancy(int max_nlev, int grow, int walls, size_t dyn_byte
                               int* blocks_per_cu, size_t* static_bytes);
 /* The loop of one system on a workgroup of `waves` wavefronts (4, 8 or 16;
  * every system has edmd_wide_level >= 0, 0 unless place is EDMD_WIDE_GROUPS,
- * and a cell capacity that the staged neighbour scan takes): dyn_bytes of dynamic LDS, at least edmd_wide_bytes
- * for every system, after edmd_lds_layout's total when the arrays are in LDS
- * too.  Workgroups one CU holds of it, 0 when none fits. */
+ * and a cell capacity that the staged neighbour scan takes): dyn_bytes of dynamic LDS, at least
+ * edmd_wide_bytes for every system, after edmd_lds_layout's total when the
+ * arrays are in LDS too.  Workgroups one CU holds of it, 0 when none fits. */
 hipError_t edmd_launch_run_wide(const EdmdSys* d_sys, int nsys, int grow, int walls, int waves,
                                 int place, size_t dyn_bytes, EdmdRunArgs ra, hipStream_t s);
 hipError_t edmd_wide_occupancy(int grow, int walls, int waves, int place, size_t dyn_bytes,

@@ -216,9 +216,12 @@ static inline EDMD_HD int edmd_wide_level(const EdmdConst* c) {
     if (c->nlev >= 2 && c->lsize[2] <= EDMD_WIDE_NODES) return 2;
     return -1;
 }
-static inline EDMD_HD uint64_t edmd_wide_bytes(const EdmdConst* c) {
+/* The window's bytes; in_lds: of a system whose arrays are in LDS too, whose
+ * window of leaves takes the leaves' ranks from there. */
+static inline EDMD_HD uint64_t edmd_wide_bytes(const EdmdConst* c, int in_lds) {
     const int l = edmd_wide_level(c);
-    return l < 0 ? 0 : edmd_lds_align((uint64_t)c->lsize[l] * (l == 0 ? 20 : 24));
+    const uint64_t node = l > 0 ? 24 : (in_lds ? 12 : 20);
+    return l < 0 ? 0 : edmd_lds_align((uint64_t)c->lsize[l] * node);
 }
 
 /* Per-system counters at the end of one epoch of a graph-captured run. */

@@ -87,3 +87,29 @@ def test_equal_times_in_wide_rounds(gpu, n):
         b.close()
     same_trace(got[1][0], got[0][0])
     same_state(got[1][1], got[0][1])
+
+
+@pytest.mark.parametrize("n", [350, 400, 430])
+@pytest.mark.parametrize("name", ["plain", "thermostat", "grow", "walls"])
+def test_two_systems_a_unit_in_lds_agree(gpu, name, n):
+    """300 systems, two a compute unit, with their arrays in LDS where two of
+    them fit it beside their windows (about 410 disks) and in HBM above that;
+    against the loop of one wavefront (1200)."""
+    base = systems(gpu, name, (n, n - 1, n - 50))
+    got = []
+    for size in (300, 1200):
+        b = gpu.Batch(base * (size // 3), **VARIANTS[name])
+        b.set_residency(gpu.RES_AUTO if size == 300 else gpu.RES_HBM)
+        b.run(max_events=900)
+        b.run(max_events=3000)
+        at = size - 3
+        got.append([(b.state(at + k), b.observables(at + k), b.thermo(at + k), b.calendar(at + k))
+                    for k in range(3)])
+        b.close()
+    for (sa, oa, ta, ca), (sb, ob, tb, cb) in zip(*got):
+        same_state(sa, sb)
+        assert oa == ob
+        assert np.array_equal(ta.view(np.uint8), tb.view(np.uint8))
+        for k in ca:
+            assert np.array_equal(np.asarray(ca[k]).view(np.uint8),
+                                  np.asarray(cb[k]).view(np.uint8)), k
