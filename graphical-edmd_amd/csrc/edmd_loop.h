@@ -599,8 +599,8 @@ __device__ __forceinline__ int ev_particle(const EdmdConst& C, const AR& A, int 
                aux >= 0 ? EDMD_EV_COLLISION : (wall ? EDMD_EV_WALL : EDMD_EV_CELLCROSS), p,
                aux >= 0 ? aux : S.d, S.kind != EVK_STALE);
     if (S.kind == EVK_COLLISION || wall) R.ncol++;
-    event_store(A, lane, t, S);
     if (S.kind == EVK_CROSSING) {
+        /* into a full cell: the disk's record stays as it was */
         event_cells(C, A, lane, S);
         const int c1 = S.cy * C.ncx + S.cx;
         const int n1 = A.ccnt[c1];
@@ -612,9 +612,11 @@ __device__ __forceinline__ int ev_particle(const EdmdConst& C, const AR& A, int 
             }
             return EDMD_EV_CELLCROSS;
         }
+        event_store(A, lane, t, S);
         event_enter(C, A, lane, S, n1);
-    } else if (S.kind != EVK_STALE) {
-        event_sums<G, W>(C, A, lane, t, S, p, aux, R.q->vir);
+    } else {
+        event_store(A, lane, t, S);
+        if (S.kind != EVK_STALE) event_sums<G, W>(C, A, lane, t, S, p, aux, R.q->vir);
     }
     WAVE_SYNC();
     event_predict<G, W, false>(C, A, lane, t, S, R.q->cand);
