@@ -158,10 +158,12 @@ struct edmd_batch {
     int loop_wpb = 1;
     /* the wide loop (one system per workgroup of several wavefronts), of the
      * Normal [0] and growing [1] launches: its wavefronts (0: not used),
-     * whether its arrays are in LDS, and its dynamic LDS */
+     * whether its arrays are in LDS, its dynamic LDS and how many of its
+     * workgroups the device holds */
     int wide_waves[2] = {0, 0};
     int wide_place[2] = {EDMD_WIDE_GROUPS, EDMD_WIDE_GROUPS};
     size_t wide_dyn[2] = {0, 0};
+    int64_t wide_slots[2] = {0, 0};
     /* pinned host memory that results come back through (read_rows): two
      * buffers of stage_half bytes, allocated by the first read */
     std::mutex stage_lock;
@@ -954,7 +956,10 @@ static int choose_wide(edmd_batch* b) {
             }
             if (b->wide_place[g] != EDMD_WIDE_LDS)
                 HIPCHK(edmd_wide_occupancy(g, b->any_walls ? 1 : 0, waves, b->wide_place[g], cal, &fit));
-            if (fit >= per_cu) b->wide_waves[g] = waves;
+            if (fit >= per_cu) {
+                b->wide_waves[g] = waves;
+                b->wide_slots[g] = (int64_t)fit * ncu;
+            }
         }
     return EDMD_OK;
 }
@@ -962,12 +967,22 @@ static int choose_wide(edmd_batch* b) {
 /* Whether the HBM-resident loop may hold several systems per workgroup. */
 static bool packable(const edmd_batch* b) { return !b->any_walls && b->max_nlev <= 2; }
 
+/* Whether a launch of the Normal (g = 0) or growing (1) systems takes the wide
+ * loop; several systems per workgroup, where asked for, is the other loop's. */
+static bool runs_wide(const edmd_batch* b, int g) {
+    return b->wide_waves[g] && (g || b->loop_wpb == 1);
+}
+
+/* Whether the loop that such a launch runs has its arrays in LDS. */
+static bool runs_in_lds(const edmd_batch* b, int g) {
+    return runs_wide(b, g) ? b->wide_place[g] == EDMD_WIDE_LDS : b->use_lds;
+}
+
 /* One launch of the event loop over every system (grow: the growing ones). */
 static hipError_t launch_loop(edmd_batch* b, int grow, const EdmdRunArgs& ra) {
     const int walls = b->any_walls ? 1 : 0;
     const int g = grow ? 1 : 0;
-    /* (several systems per workgroup, where asked for, is the other loop's) */
-    if (b->wide_waves[g] && (grow || b->loop_wpb == 1))
+    if (runs_wide(b, g))
         return edmd_launch_run_wide(b->d_sys, b->nsys, grow, walls, b->wide_waves[g],
                                     b->wide_place[g], b->wide_dyn[g], ra, b->stream);
     if (b->use_lds)
@@ -1013,9 +1028,18 @@ extern "C" int edmd_batch_set_residency(edmd_batch* b, int mode) {
 extern "C" int edmd_batch_get_residency(edmd_batch* b, int* in_lds, int64_t* lds_bytes,
                                         int64_t* lds_slots) {
     if (!b) return fail(EDMD_ERR_ARG, "null batch");
-    if (in_lds) *in_lds = b->use_lds ? 1 : 0;
-    if (lds_bytes) *lds_bytes = (int64_t)(b->any_grow ? b->lds_dyn[1] : b->lds_dyn[0]);
-    if (lds_slots) *lds_slots = b->lds_fit ? b->lds_slots : 0;
+    const int g = b->any_grow ? 1 : 0;
+    const bool lds = runs_in_lds(b, g), wide = lds && runs_wide(b, g);
+    if (in_lds) *in_lds = lds ? 1 : 0;
+    if (lds_bytes) *lds_bytes = (int64_t)(wide ? b->wide_dyn[g] : b->lds_dyn[g]);
+    if (lds_slots) *lds_slots = wide ? b->wide_slots[g] : (b->lds_fit ? b->lds_slots : 0);
+    return EDMD_OK;
+}
+
+extern "C" int edmd_batch_get_wavefronts(edmd_batch* b, int* per_system) {
+    if (!b) return fail(EDMD_ERR_ARG, "null batch");
+    const int g = b->any_grow ? 1 : 0;
+    if (per_system) *per_system = runs_wide(b, g) ? b->wide_waves[g] : 1;
     return EDMD_OK;
 }
 
@@ -1187,7 +1211,7 @@ extern "C" int edmd_batch_autotune(edmd_batch* b, int sweep_reps, int64_t trial_
     if (e1) (void)hipEventDestroy(e1);
     (void)hipFree(snap);
     r.sweep_shape = b->sweep_variant;
-    r.in_lds = b->use_lds ? 1 : 0;
+    r.in_lds = runs_in_lds(b, b->any_grow ? 1 : 0) ? 1 : 0;
     r.loop_systems_per_group = b->loop_wpb;
     if (out) *out = r;
     return rc;

@@ -135,6 +135,7 @@ def lib():
             "edmd_batch_set_stream": (i32, [vp, vp]),
             "edmd_batch_set_residency": (i32, [vp, i32]),
             "edmd_batch_get_residency": (i32, [vp, vp, vp, vp]),
+            "edmd_batch_get_wavefronts": (i32, [vp, vp]),
             "edmd_batch_set_sweep_shape": (i32, [vp, i32]),
             "edmd_batch_get_sweep_shape": (i32, [vp, vp, vp, vp, vp]),
             "edmd_batch_set_screen": (i32, [vp, i32]),
@@ -561,11 +562,17 @@ class Batch:
         return v.value
 
     def residency(self):
-        """{'lds': mode in use is LDS, 'lds_bytes': dynamic LDS per workgroup
-        in LDS mode, 'lds_slots': workgroups resident at once in LDS mode}"""
+        """{'lds': the next run's loop has its arrays in LDS, 'lds_bytes':
+        dynamic LDS per workgroup, 'lds_slots': workgroups resident at once}"""
         a, b, c = C.c_int(), C.c_int64(), C.c_int64()
         check(lib().edmd_batch_get_residency(self.h, C.byref(a), C.byref(b), C.byref(c)))
         return {"lds": bool(a.value), "lds_bytes": b.value, "lds_slots": c.value}
+
+    def wavefronts(self):
+        """Wavefronts that the next run's loop gives each system."""
+        v = C.c_int()
+        check(lib().edmd_batch_get_wavefronts(self.h, C.byref(v)))
+        return v.value
 
     # ---- derivatives of the event map
 

@@ -345,11 +345,15 @@ int edmd_batch_set_stream(edmd_batch* b, void* stream);
 #define EDMD_RES_HBM 1
 #define EDMD_RES_LDS 2
 int edmd_batch_set_residency(edmd_batch* b, int mode);
-/* The mode in use (*in_lds 1 = LDS), the dynamic LDS per workgroup the LDS
- * mode takes, and the workgroups the device holds at once in that mode
- * (0 when the systems do not fit).  Any output may be NULL. */
+/* Where the loop of the next run has its arrays (*in_lds 1 = LDS); the dynamic
+ * LDS per workgroup of that loop, and the workgroups the device holds of it at
+ * once; where it runs from device memory, those of the loop of one wavefront
+ * in LDS (0 workgroups when the systems do not fit).  Any output may be NULL. */
 int edmd_batch_get_residency(edmd_batch* b, int* in_lds, int64_t* lds_bytes,
                              int64_t* lds_slots);
+/* Wavefronts that the loop of the next run gives each system: 16, 8, 4 or 1.
+ * No counterpart in the reference; results do not depend on it. */
+int edmd_batch_get_wavefronts(edmd_batch* b, int* per_system);
 
 /* Tile shape of the prediction sweep (collisionEventNormal and
  * crossingEventNormal for every disk, as eventListInit runs them,

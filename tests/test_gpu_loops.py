@@ -1,6 +1,6 @@
-"""The event loops against one another where they part: the state that a full
-cell leaves behind (addToCell, EDMD.c:2576-2585, has no bound; the capacity is
-this library's)."""
+"""The event loops where they part: what a full cell leaves behind (addToCell,
+EDMD.c:2576-2585, has no bound; the capacity is this library's), and which loop
+a batch gets (the reference has one, mainLoop, EDMD.c:5595-5630)."""
 import numpy as np
 import pytest
 
@@ -38,3 +38,32 @@ def test_state_after_a_full_cell(gpu, size, waves, res):
     same_trace(tr[:-1], c.trace(0))
     for k, v in b.events(0).items():
         np.testing.assert_array_equal(v, c.events(0)[k], err_msg=k)
+
+
+def test_residency_names_the_loop_that_runs(gpu):
+    """300 systems, two a compute unit: their arrays lie in LDS only where two
+    of them fit it beside their windows (about 410 disks; one of 600 would)."""
+    for n, lds in ((350, True), (450, False), (600, False)):
+        st = F.lattice_state(n, 0.55, seed=n, lattice="fit")
+        two = gpu.Batch([st] * 300)
+        r = two.residency()
+        assert r["lds"] == lds, (n, r)
+        assert two.wavefronts() == (4 if n < 500 else 8)
+        one = gpu.Batch([st])
+        r1 = one.residency()
+        assert r1["lds"] and one.wavefronts() == 8
+        if lds:  # the wide loop's own: the arrays and the window
+            assert r["lds_slots"] >= 300 and r["lds_bytes"] > n * 64 + 12 * n
+        one.set_residency(gpu.RES_HBM)
+        assert not one.residency()["lds"]
+        rep = two.autotune(sweep_reps=0, trial_events=0)
+        assert rep["in_lds"] == lds
+        two.close()
+        one.close()
+    st = F.lattice_state(600, 0.55, seed=1, lattice="fit")
+    b = gpu.Batch([st] * 300)
+    b.set_loop_waves(2)
+    assert b.wavefronts() == 1
+    b.set_loop_waves(1)
+    b.set_residency(gpu.RES_LDS)
+    assert b.residency()["lds"]
