@@ -342,9 +342,9 @@ __device__ __forceinline__ bool staged_cap(const EdmdConst& C) {
  * candidates f, f + 32, ...; one disk: all 64 lanes its f, f + 64, ....
  * Each lane keeps its first strictly least time, and the least over the
  * half, the lowest position among equal times, is the reference's
- * strict-less first minimum.  Cell capacities that the stage cannot take
- * (over EDMD_STAGE_CAP, or rows that are not whole 16-byte chunks) are
- * scanned cell by cell from memory.
+ * strict-less first minimum.  Of cell capacities that the stage cannot take
+ * (over EDMD_STAGE_CAP, or rows that are not whole 16-byte chunks) each lane
+ * reads its candidate's slot from memory: one round trip more a pass.
  *
  * SPEC = false: the event's records are stored already (event_store), and
  * the field's or the damping's flights of the neighbours (EDMD.c:2664-2666)
@@ -363,16 +363,18 @@ __device__ __forceinline__ void predict_halves(const EdmdConst& C, const AR& A, 
     const int sub = lane & 31;
     const bool two = S.nown == 2;
     const bool staged = SPEC || staged_cap(C);
-    const bool ent = sub < 9 && (two || !hi) && staged;
+    const bool ent = sub < 9 && (two || !hi);
     int cnt = 0;
     int4 row[EDMD_STAGE_CAP / 4];
     if (ent) {
         const int cell = near_cell(C, S.cx, S.cy, sub);
         const int4* src = (const int4*)(A.cslot + (int64_t)cell * C.cap);
         cnt = A.ccnt[cell];
+        if (staged) {
 #pragma unroll
-        for (int c = 0; c < EDMD_STAGE_CAP / 4; ++c)
-            if (4 * c < C.cap) row[c] = src[c];
+            for (int c = 0; c < EDMD_STAGE_CAP / 4; ++c)
+                if (4 * c < C.cap) row[c] = src[c];
+        }
     }
     /* the other disk's state, for its place among the candidates */
     int oth = -1;
@@ -399,7 +401,16 @@ __device__ __forceinline__ void predict_halves(const EdmdConst& C, const AR& A, 
     S.n1 = __builtin_amdgcn_readlane(cnt, 4); /* the disk's own cell */
     int32_t* const half_stage =
         stage + ((two && hi) ? EDMD_STAGE_HALF : 0) + EDMD_STAGE_CAP;
-    if (ent && cnt > 0) {
+    if (!staged) {
+        if (ent) {
+            /* what the fetch below needs of this cell: the candidates up to
+             * its last, and the slot that candidate 0 would have */
+            const int64_t at = (int64_t)near_cell(C, S.cx, S.cy, sub) * C.cap + incl - 1;
+            half_stage[sub] = incl;
+            half_stage[16 + 2 * sub] = (int)at;
+            half_stage[17 + 2 * sub] = (int)(at >> 32);
+        }
+    } else if (ent && cnt > 0) {
         /* slot k (k-th oldest) goes to incl - 1 - k.  The row is written
          * whole, its last slot first: an unused slot (k >= cnt) falls on the
          * slot k - cnt, or a lower one, of a cell before, which is written
@@ -421,22 +432,24 @@ __device__ __forceinline__ void predict_halves(const EdmdConst& C, const AR& A, 
     const int most = totA > totB ? totA : totB;
     const int mine = (two && hi) ? totB : totA;
     const int li = two ? sub : lane, step = two ? 32 : 64;
-    const int chunks = staged ? 1 : (C.cap + step - 1) / step; /* passes per cell */
-    const int passes = staged ? (most + step - 1) / step : 9 * chunks;
+    const int passes = (most + step - 1) / step;
     double bt = INF_D;
     int bq = 0, bf = 0;
     uint32_t bc = 0;
     for (int pass = 0; pass < passes; ++pass) {
-        int f, q = -1;
-        if (staged) {
-            f = pass * step + li;
-            if (f < mine) q = half_stage[f];
-        } else {
-            const int e = pass / chunks, k = (pass - e * chunks) * step + li;
-            const int cell = near_cell(C, S.cx, S.cy, e);
-            const int n = A.ccnt[cell];
-            f = e * 64 + k;
-            if (k < n) q = A.cslot[(size_t)cell * C.cap + n - 1 - k];
+        const int f = pass * step + li;
+        int q = -1;
+        if (f < mine) {
+            if (staged) {
+                q = half_stage[f];
+            } else {
+                int e = 0; /* the candidate's cell */
+#pragma unroll
+                for (int s = 0; s < 8; ++s) e += f >= half_stage[s] ? 1 : 0;
+                const int64_t at = (int64_t)((uint64_t)(uint32_t)half_stage[17 + 2 * e] << 32 |
+                                             (uint32_t)half_stage[16 + 2 * e]);
+                q = A.cslot[at - f];
+            }
         }
         if (q >= 0 && q != S.own) {
             EdmdPart r = A.p[q];

@@ -1,6 +1,8 @@
 """The event loops where they part: what a full cell leaves behind (addToCell,
 EDMD.c:2576-2585, has no bound; the capacity is this library's), and which loop
 a batch gets (the reference has one, mainLoop, EDMD.c:5595-5630)."""
+import time
+
 import numpy as np
 import pytest
 
@@ -67,3 +69,29 @@ def test_residency_names_the_loop_that_runs(gpu):
     b.set_loop_waves(1)
     b.set_residency(gpu.RES_LDS)
     assert b.residency()["lds"]
+
+
+def seconds(b, events, reps=3):
+    """Median time of a run over so many more events of each system."""
+    done, took = b.observables(0)["nevents"], []
+    for _ in range(reps):
+        done += events
+        t = time.perf_counter()
+        b.run(max_events=done)
+        took.append(time.perf_counter() - t)
+    return sorted(took)[reps // 2]
+
+
+def test_any_cell_capacity_costs_alike(gpu):
+    """The scan of cells that the LDS stage does not take (here 28 slots; 24
+    are taken) reads one slot a candidate, not one cell after another, which
+    took 2.4 times as long; both batches run on one wavefront a system."""
+    st = F.lattice_state(200, 0.5, seed=3, lattice="fit")
+    took = []
+    for cap in (24, 28):
+        b = gpu.Batch([st] * 1100, cell_capacity=cap)
+        assert b.wavefronts() == 1
+        b.run(max_events=500)
+        took.append(seconds(b, 1000))
+        b.close()
+    assert took[1] < 1.6 * took[0], took
