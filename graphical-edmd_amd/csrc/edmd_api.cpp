@@ -916,10 +916,24 @@ static int wide_width(int per_cu, int64_t disks) {
     return disks < 300 ? 4 : (disks < 1800 ? 8 : 16);
 }
 
+/* Least cells a system (the batch's mean) has for that loop to be the faster
+ * one.  Events within `reach` cells of one another go one after the other, at a
+ * round's cost each, and the more systems share a CU the more a round costs.
+ * us an event on one wavefront and on several, disks at phi 0.5 in 25, 36, 49
+ * and 64 cells: one system a CU 3.1, 3.7; 3.5, 3.1; 3.5, 2.7; 3.5, 2.4; two
+ * 3.3, 4.3; 3.6, 3.7; 3.7, 3.1; 3.7, 2.9; four 3.5, 5.4; 3.8, 4.6; 3.8, 4.0;
+ * 3.9, 3.8; in a channel under the field (reach 2) in 64, 81 and 144 cells: one
+ * 4.7, 4.9; 4.7, 4.4; 4.8, 3.7; two 5.2, 5.7; 5.1, 5.1; 4.9, 4.0; four 5.2,
+ * 7.1; 5.2, 6.7; 6.1, 5.2.  Of small systems under the thermostat a good part
+ * is the rescales between rounds: two a CU of 49 cells 5.5, 6.1. */
+static int64_t wide_cells(int per_cu, int reach, bool rescales) {
+    return (24 + 12 * (per_cu + (rescales ? 1 : 0))) * reach;
+}
+
 /* Whether the loop runs each system on a workgroup of several wavefronts
  * (edmd_wide.hip): while the device has wavefront slots to spare, i.e. for
  * batches of at most EDMD_WIDE_PER_CU systems a CU, all of them resident at
- * once.  With the arrays in LDS where that mode is in use and they fit beside
+ * once, of at least wide_cells cells.  With the arrays in LDS where that mode is in use and they fit beside
  * the window; asked for LDS and not fitting, the loop of one wavefront runs. */
 static int choose_wide(edmd_batch* b) {
     b->wide_waves[0] = b->wide_waves[1] = 0;
@@ -930,19 +944,25 @@ static int choose_wide(edmd_batch* b) {
     if (per_cu > EDMD_WIDE_PER_CU) return EDMD_OK;
     size_t cal = 0, both[2] = {0, 0};
     bool flat = true;
-    int64_t disks = 0;
+    int64_t disks = 0, cells = 0;
+    int reach = 1; /* cells from which the Normal loop's events read */
+    bool rescales = false;
     for (int s = 0; s < b->nsys; s++) {
         const EdmdConst& c = b->hs[s].c;
         /* the scan of cells in LDS takes rows of whole 16-byte chunks */
         if (edmd_wide_level(&c) < 0 || c.cap > EDMD_STAGE_CAP || (c.cap & 3) != 0) return EDMD_OK;
         flat &= edmd_wide_level(&c) == 0;
         disks += c.n;
+        cells += (int64_t)c.ncx * c.ncy;
+        if (c.field_on || c.damping) reach = 2;
+        rescales |= c.noise != 0;
         cal = std::max(cal, (size_t)edmd_wide_bytes(&c, 0));
         for (int g = 0; g < 2; g++)
             both[g] = std::max(both[g], (size_t)edmd_lds_layout(&c, g).total + (size_t)edmd_wide_bytes(&c, 1));
     }
     const int most = wide_width(per_cu, disks / b->nsys);
-    for (int g = 0; g < (b->any_grow ? 2 : 1); g++)
+    for (int g = 0; g < (b->any_grow ? 2 : 1); g++) {
+        if (cells / b->nsys < wide_cells(per_cu, g ? 1 : reach, rescales)) continue;
         for (int waves = most; waves >= 4 && !b->wide_waves[g]; waves /= 2) {
             int fit = 0;
             b->wide_place[g] = flat ? EDMD_WIDE_LEAVES : EDMD_WIDE_GROUPS;
@@ -961,6 +981,7 @@ static int choose_wide(edmd_batch* b) {
                 b->wide_slots[g] = (int64_t)fit * ncu;
             }
         }
+    }
     return EDMD_OK;
 }
 

@@ -11,6 +11,8 @@ from test_gpu_wide import QUIET, same_state, same_trace
 
 pytestmark = pytest.mark.gpu
 
+FIELD = dict(wall_y=1, res_tan=1.0, add_field=1, field=-0.02)
+
 
 @pytest.mark.parametrize("size,waves,res", [(1, 1, "RES_HBM"), (1, 1, "RES_LDS"),
                                             (2, 2, "RES_HBM"), (1100, 1, "RES_HBM")])
@@ -95,3 +97,28 @@ def test_any_cell_capacity_costs_alike(gpu):
         took.append(seconds(b, 1000))
         b.close()
     assert took[1] < 1.6 * took[0], took
+
+
+@pytest.mark.parametrize("n,phi,kw,size,waves", [
+    (80, 0.5, {}, 1, 1), (100, 0.5, {}, 1, 4), (100, 0.5, {}, 300, 1), (128, 0.5, {}, 300, 4),
+    (128, 0.5, dict(noise=2, dtnoise=0.1, temperature=1.0), 300, 1),
+    (128, 0.5, {}, 1000, 1), (260, 0.5, {}, 1000, 4), (48, 0.2, {}, 1, 4),
+    (160, 0.4, FIELD, 1, 1), (200, 0.4, FIELD, 1, 4), (200, 0.4, FIELD, 300, 1),
+    (300, 0.4, FIELD, 300, 4), (16, 0.1, {}, 1, 1), (50, 0.5, dict(vr=0.3), 300, 1),
+    (150, 0.5, dict(vr=0.3), 300, 4)])
+def test_small_systems_take_one_wavefront(gpu, n, phi, kw, size, waves):
+    """On either side of the cells that the loop of several wavefronts takes,
+    by the systems that share a CU and by the reach of an event; the state of
+    every copy is the same."""
+    if "vr" in kw:
+        st = gpu.init_random(n, phi, seed=n)
+    else:
+        st = F.lattice_state(n, phi, seed=n, lattice="fit")
+    if "wall_y" in kw:
+        st["y"] = 0.51 + st["y"] / st["Ly"] * (st["Ly"] - 1.02)
+    b = gpu.Batch([st] * size, **kw)
+    assert b.wavefronts() == waves
+    b.run(max_events=3000, tmax=3.0 if "vr" in kw else 1e300)
+    first = b.state(0)
+    for k in range(1, size, 7):
+        same_state(b.state(k), first)
