@@ -164,6 +164,10 @@ struct edmd_batch {
     int wide_place[2] = {EDMD_WIDE_GROUPS, EDMD_WIDE_GROUPS};
     size_t wide_dyn[2] = {0, 0};
     int64_t wide_slots[2] = {0, 0};
+    /* the least counters and times of the systems when they were last read
+     * (check_status), and the most events a time unit: how many events a run
+     * has left, roughly */
+    double seen_events = 0, seen_coll = 0, seen_t = 0, seen_rate = 0;
     /* pinned host memory that results come back through (read_rows): two
      * buffers of stage_half bytes, allocated by the first read */
     std::mutex stage_lock;
@@ -664,6 +668,14 @@ static int read_columns(edmd_batch* b, const R* src, size_t n, std::initializer_
 static int check_status(edmd_batch* b) {
     int bad = 0;
     int rc = read_rows(b, b->st, (size_t)b->nsys, [&](size_t s0, const EdmdState* st, size_t k) {
+        for (size_t j = 0; j < k; j++) {
+            const double ev = (double)st[j].nevents, co = (double)st[j].ncol, t = st[j].t;
+            const bool first = s0 + j == 0;
+            b->seen_events = first ? ev : std::min(b->seen_events, ev);
+            b->seen_coll = first ? co : std::min(b->seen_coll, co);
+            b->seen_t = first ? t : std::min(b->seen_t, t);
+            b->seen_rate = std::max(first ? 0.0 : b->seen_rate, t > 0 ? ev / t : 0.0);
+        }
         for (size_t j = 0; j < k && !bad; j++) {
             const int s = (int)(s0 + j);
             if (st[j].status == EDMD_DEV_OVERLAP)
@@ -999,10 +1011,31 @@ static bool runs_in_lds(const edmd_batch* b, int g) {
     return runs_wide(b, g) ? b->wide_place[g] == EDMD_WIDE_LDS : b->use_lds;
 }
 
-/* One launch of the event loop over every system (grow: the growing ones). */
-static hipError_t launch_loop(edmd_batch* b, int grow, const EdmdRunArgs& ra) {
+/* About how many events a system has left in a run (two a collision). */
+static double events_left(const edmd_batch* b, const EdmdRunArgs& ra) {
+    double left = std::min((double)ra.max_events - b->seen_events,
+                           2 * ((double)ra.max_coll - b->seen_coll));
+    if (b->seen_rate > 0 && ra.tmax < 1e299)
+        left = std::min(left, (ra.tmax - b->seen_t) * b->seen_rate);
+    if (ra.stop_mask & (1 << EDMD_EV_COLLISION | 1 << EDMD_EV_CELLCROSS)) left = std::min(left, 4.0);
+    return left;
+}
+
+/* Runs of so few events are over on one wavefront, arrays in HBM, before the
+ * wide loop has its window: it reads every leaf and makes the calendar's levels
+ * again at its end.  us a run of 1 event on one wavefront and on several: 2000
+ * disks 31, 48; 20000 31, 79; 2^18 32, 450; 2^20 32, 1677; as long as one
+ * another at about 9 events of 2000 disks, 20 of 20000, 37 of 2^16, 115 of
+ * 2^18 and 370 of 2^20. */
+static double wide_events(const edmd_batch* b) { return 12 + b->max_n / 2500.0; }
+
+/* One launch of the event loop over every system (grow: the growing ones);
+ * left: about the most events that a system will handle. */
+static hipError_t launch_loop(edmd_batch* b, int grow, const EdmdRunArgs& ra, double left) {
     const int walls = b->any_walls ? 1 : 0;
     const int g = grow ? 1 : 0;
+    if (runs_wide(b, g) && left <= wide_events(b) && b->residency != EDMD_RES_LDS)
+        return edmd_launch_run(b->d_sys, b->nsys, b->max_nlev, grow, walls, 1, ra, b->stream);
     if (runs_wide(b, g))
         return edmd_launch_run_wide(b->d_sys, b->nsys, grow, walls, b->wide_waves[g],
                                     b->wide_place[g], b->wide_dyn[g], ra, b->stream);
@@ -1195,8 +1228,8 @@ extern "C" int edmd_batch_autotune(edmd_batch* b, int sweep_reps, int64_t trial_
             if ((rc = choose_wide(b))) break;
             e = edmd_launch_epoch_begin(b->d_sys, b->nsys, trial_events, ~(uint64_t)0, b->stream);
             if (e == hipSuccess) e = hipEventRecord(e0, b->stream);
-            if (e == hipSuccess && b->any_grow) e = launch_loop(b, 1, ra);
-            if (e == hipSuccess) e = launch_loop(b, 0, ra);
+            if (e == hipSuccess && b->any_grow) e = launch_loop(b, 1, ra, EDMD_NEVER);
+            if (e == hipSuccess) e = launch_loop(b, 0, ra, EDMD_NEVER);
             if (e == hipSuccess) e = hipEventRecord(e1, b->stream);
             if (e == hipSuccess) e = hipEventSynchronize(e1);
             if (e == hipSuccess) e = hipEventElapsedTime(&ms, e0, e1);
@@ -1247,10 +1280,11 @@ static int batch_run_mask(edmd_batch* b, int64_t max_events, uint64_t max_collis
     ra.max_coll = max_collisions;
     ra.tmax = tmax;
     ra.stop_mask = stop_mask & ~(1 << EDMD_EV_GROWSTOP);
+    const double left = events_left(b, ra);
     if (b->any_grow) {
         /* growing systems first: they run until GROWSTOP (then continue in
          * the Normal launch below) or until the bounds */
-        HIPCHK(launch_loop(b, 1, ra));
+        HIPCHK(launch_loop(b, 1, ra, left));
         HIPCHK(hipStreamSynchronize(b->stream));
         int rc = check_status(b);
         if (rc) return rc;
@@ -1260,7 +1294,7 @@ static int batch_run_mask(edmd_batch* b, int64_t max_events, uint64_t max_collis
         for (int s = 0; s < b->nsys; s++) still |= st[s].growing != 0;
         b->any_grow = still;
     }
-    HIPCHK(launch_loop(b, 0, ra));
+    HIPCHK(launch_loop(b, 0, ra, left));
     HIPCHK(hipStreamSynchronize(b->stream));
     return check_status(b);
 }
@@ -1287,6 +1321,7 @@ extern "C" int edmd_batch_run_epochs(edmd_batch* b, int nepochs, int64_t events_
     ra.max_events = INT64_MAX; /* the per-system epoch bounds apply */
     ra.max_coll = ~(uint64_t)0;
     ra.tmax = tmax;
+    const double left = std::min((double)events_per_epoch, 2 * (double)collisions_per_epoch);
     /* one graph holds every epoch: bounds, the growing systems' launch (a
      * no-op for systems that are not growing), the Normal launch and the
      * counters; captured once, launched once */
@@ -1297,8 +1332,8 @@ extern "C" int edmd_batch_run_epochs(edmd_batch* b, int nepochs, int64_t events_
         e = edmd_launch_epoch_begin(b->d_sys, nsys, events_per_epoch, collisions_per_epoch,
                                     b->stream);
         if (e == hipSuccess && b->any_grow)
-            e = launch_loop(b, 1, ra);
-        if (e == hipSuccess) e = launch_loop(b, 0, ra);
+            e = launch_loop(b, 1, ra, left);
+        if (e == hipSuccess) e = launch_loop(b, 0, ra, left);
         if (e == hipSuccess)
             e = edmd_launch_epoch_end(b->d_sys, nsys, d_rows + (size_t)k * nsys, b->stream);
     }
@@ -2248,7 +2283,7 @@ static int tape_overflow_check(edmd_batch* b) {
 /* Runs one checkpoint segment: at most `seg` events per system, new tape. */
 static int run_segment(edmd_batch* b, const EdmdRunArgs& ra) {
     HIPCHK(edmd_launch_seg_begin(b->d_sys, b->nsys, b->seg, 1, b->stream));
-    HIPCHK(launch_loop(b, 0, ra));
+    HIPCHK(launch_loop(b, 0, ra, (double)b->seg));
     HIPCHK(hipStreamSynchronize(b->stream));
     return check_status(b);
 }

@@ -352,7 +352,9 @@ int edmd_batch_set_residency(edmd_batch* b, int mode);
 int edmd_batch_get_residency(edmd_batch* b, int* in_lds, int64_t* lds_bytes,
                              int64_t* lds_slots);
 /* Wavefronts that the loop of the next run gives each system: 16, 8, 4 or 1.
- * No counterpart in the reference; results do not depend on it. */
+ * A run that is known to be of a few events (12, more of large systems) takes
+ * one, with its arrays in device memory unless EDMD_RES_LDS is set.  No
+ * counterpart in the reference; results do not depend on it. */
 int edmd_batch_get_wavefronts(edmd_batch* b, int* per_system);
 
 /* Tile shape of the prediction sweep (collisionEventNormal and

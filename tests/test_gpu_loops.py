@@ -122,3 +122,58 @@ def test_small_systems_take_one_wavefront(gpu, n, phi, kw, size, waves):
     first = b.state(0)
     for k in range(1, size, 7):
         same_state(b.state(k), first)
+
+
+@pytest.mark.parametrize("kw", [{}, FIELD, dict(noise=2, dtnoise=0.02, temperature=1.0)])
+@pytest.mark.parametrize("n", [150, 1000, 6200])
+def test_runs_of_any_length_match_oracle(gpu, oracle, n, kw):
+    """Runs of a few events, which one wavefront handles, and of many, by
+    events, collisions, time and kind, in turn on one system."""
+    st = F.lattice_state(n, 0.4, seed=n, lattice="fit")
+    if "wall_y" in kw:
+        st["y"] = 0.51 + st["y"] / st["Ly"] * (st["Ly"] - 1.02)
+    kw = dict(QUIET, **kw)
+    s = gpu.System(st, trace_capacity=20000, **kw)
+    done, seen = 0, []
+
+    def after():
+        seen.append(s.trace())
+        return s.observables()
+
+    for k in (1, 1, 7, 300, 10, 11, 2, 500, 1):
+        done += k
+        s.run(max_events=done)
+        assert after()["nevents"] == done
+    for k in (1, 2, 400, 3, 5):
+        want = s.observables()["ncol"] + k
+        s.run(max_collisions=want)
+        assert after()["ncol"] == want
+    for k in (1e-9, 1e-3, 0.05, 1e-4):
+        t = s.observables()["t"] + k
+        s.run(tmax=t)
+        assert after()["t"] > t
+    for kind in (gpu.EV_COLLISION, gpu.EV_CELLCROSS):
+        s.run_until_kind(1 << kind)
+        after()
+        assert seen[-1]["type"][-1] == kind
+    nev = s.observables()["nevents"]
+    tr = np.concatenate(seen)
+    assert len(tr) == nev
+    o = oracle.Oracle(st, **kw)
+    code, ref = o.run(nev)
+    assert code == 0
+    same_trace(tr, ref)
+    same_state(s.state(), o.state())
+
+
+def test_one_event_costs_alike_in_any_system(gpu):
+    """A run of one event, of 2^18 disks and of 1000: the loop's window was
+    read and its calendar made again for it, fifteen times as long."""
+    took = []
+    for n in (1000, 1 << 18):
+        b = gpu.Batch([F.lattice_state(n, 0.4, seed=n, lattice="fit")])
+        assert b.wavefronts() > 1
+        b.run(max_events=2000)
+        took.append(seconds(b, 1, reps=15))
+        b.close()
+    assert took[1] < 3 * took[0], took
