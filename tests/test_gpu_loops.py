@@ -177,3 +177,42 @@ def test_one_event_costs_alike_in_any_system(gpu):
         took.append(seconds(b, 1, reps=15))
         b.close()
     assert took[1] < 3 * took[0], took
+
+
+def front(side):
+    """Columns of a square grid closing on one another at one speed: half its
+    collisions and crossings come at one time."""
+    k = np.arange(side * side)
+    L = side * 1.6
+    return {"x": (k % side + 0.5) * (L / side), "y": (k // side + 0.5) * (L / side),
+            "vx": np.where(k % 2 == 0, 1.0, -1.0), "vy": np.zeros(side * side),
+            "rad": np.full(side * side, 0.5), "m": np.ones(side * side), "Lx": L, "Ly": L}
+
+
+@pytest.mark.parametrize("side,waves", [(20, 8), (64, 16), (80, 16)])
+def test_fronts_of_equal_times(gpu, side, waves):
+    """Thousands of events at one time, more than a round's list takes, on
+    several wavefronts and on one (windows of leaves and, at 6400 disks, of
+    groups): the same events."""
+    nev, got = 2 * side * side, []
+    for cap in (0, 10):  # a capacity of 10 is the loop of one wavefront's
+        b = gpu.Batch([front(side)], trace_capacity=nev, cell_capacity=cap, **QUIET)
+        assert b.wavefronts() == (1 if cap else waves)
+        b.run(max_events=nev)
+        got.append((b.trace(0), b.state(0)))
+        b.close()
+    same_trace(got[0][0], got[1][0])
+    same_state(got[0][1], got[1][1])
+
+
+def test_lattice_start_costs_as_the_rest(gpu):
+    """2000 disks on a square lattice, some on their cells' edges, which they
+    cross at time 0: the first 8000 events took twice as long as the next."""
+    st = gpu.init_lattice(2000, 0.3, seed=3)
+    took = []
+    for _ in range(3):
+        b = gpu.Batch([st])
+        took.append((seconds(b, 8000, reps=1), seconds(b, 8000, reps=1)))
+        b.close()
+    first, then = (min(t[k] for t in took) for k in (0, 1))
+    assert first < 1.5 * then, took
