@@ -173,7 +173,8 @@ struct edmd_batch {
     std::mutex stage_lock;
     char* stage = nullptr;
     size_t stage_half = 0;
-    /* checkpoint memory that a new taping of the same shape takes over */
+    /* the last taping's checkpoint memory, until a new one of the same shape has
+     * taken over what it needs of it (ckpt_trim) */
     std::vector<void*> ckpt_free;
 };
 
@@ -197,11 +198,16 @@ static int dalloc(edmd_batch* b, T** p, size_t n) {
     return EDMD_OK;
 }
 
+/* Gives back the checkpoint memory that the present taping has not taken over. */
+static void ckpt_trim(edmd_batch* b) {
+    for (void* p : b->ckpt_free) (void)hipFree(p);
+    b->ckpt_free.clear();
+}
+
 static void deriv_release(edmd_batch* b) {
     for (auto& c : b->ckpts) (void)hipFree(c.mem);
     b->ckpts.clear();
-    for (void* p : b->ckpt_free) (void)hipFree(p);
-    b->ckpt_free.clear();
+    ckpt_trim(b);
     if (b->ckpt_end) (void)hipFree(b->ckpt_end);
     b->ckpt_end = nullptr;
     for (void* p : b->dallocs) (void)hipFree(p);
@@ -2187,7 +2193,8 @@ static int deriv_alloc(edmd_batch* b, T** p, size_t n) {
 }
 
 /* Ends the taping; with `keep` its memory stays for the next one, which has
- * the same tape capacity. */
+ * the same tape capacity: the tape, and until the next one's first run the
+ * checkpoints. */
 static int deriv_stop(edmd_batch* b, bool keep) {
     HIPCHK(hipStreamSynchronize(b->stream));
     if (keep) {
@@ -2262,6 +2269,11 @@ extern "C" int edmd_batch_deriv_begin(edmd_batch* b, int64_t checkpoint_every, i
     b->seg = checkpoint_every;
     b->tape_cap = cap;
     b->deriv_on = true;
+    if (b->seg == 0) { /* a whole tape has no checkpoints */
+        ckpt_trim(b);
+        if (b->ckpt_end) (void)hipFree(b->ckpt_end);
+        b->ckpt_end = nullptr;
+    }
     HIPCHK(hipMemsetAsync(b->dv, 0, 4 * b->np * sizeof(double), b->stream));
     HIPCHK(hipMemsetAsync(b->dr, 0, b->nsys * sizeof(EdmdDeriv), b->stream));
     HIPCHK(edmd_launch_deriv_origin(b->d_sys, b->nsys, b->max_n, b->stream));
@@ -2327,6 +2339,7 @@ extern "C" int edmd_batch_deriv_run(edmd_batch* b, int64_t max_events, uint64_t 
                 more = true;
         if (!more) break;
     }
+    ckpt_trim(b);
     HIPCHK(edmd_launch_seg_begin(b->d_sys, b->nsys, 0, 0, b->stream));
     HIPCHK(hipStreamSynchronize(b->stream));
     return EDMD_OK;

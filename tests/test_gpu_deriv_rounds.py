@@ -4,6 +4,8 @@ chunk waits for others), more disks than the chunk's table has slots, and
 vectors in HBM; walls among the records.  Bit for bit the oracle's, which
 applies one record after another.
 """
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -58,3 +60,37 @@ def test_rounds_match_oracle(gpu, oracle, n, params, ncoll, every):
         assert bits(dw[k]) == bits(rdw) and bits(dtl[k]) == bits(rdtl)
         g = oracle.adjoint(st["m"], s0["t"], tape, o.t, lw[k], lt[k], lam[k])
         np.testing.assert_array_equal(bits(grad[k]), bits(g), err_msg="adjoint %d" % k)
+
+
+def free_bytes():
+    free, total = C.c_size_t(), C.c_size_t()
+    assert C.CDLL("libamdhip64.so").hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+    return free.value
+
+
+def test_checkpoint_memory_is_given_back(gpu):
+    """A taping holds no checkpoint of the one before that it does not use: a
+    whole tape after a checkpointed one of the same capacity none, a shorter
+    one its own."""
+    st = F.lattice_state(400, 0.6, seed=4, lattice="fit")
+    b = gpu.Batch([st] * 256)
+    ev = 0
+
+    def tape(every, events):
+        nonlocal ev
+        b.deriv_begin(checkpoint_every=every, tape_capacity=64)
+        ev += events
+        b.deriv_run(max_events=ev)
+        return free_bytes()
+
+    tape(64, 64)
+    start = free_bytes()
+    long = tape(64, 64 * 40)
+    kept = start - long
+    assert kept > 39 * 256 * 400 * 128  # 40 snapshots of the systems' records
+    assert tape(64, 64 * 40) >= long - (64 << 20)
+    assert tape(64, 64 * 4) >= start - kept // 8
+    tape(64, 64 * 40)
+    b.deriv_begin(checkpoint_every=0, tape_capacity=64)
+    assert free_bytes() >= start - (64 << 20)
+    b.close()
