@@ -1,13 +1,14 @@
 """The event loops where they part: what a full cell leaves behind (addToCell,
-EDMD.c:2576-2585, has no bound; the capacity is this library's), and which loop
-a batch gets (the reference has one, mainLoop, EDMD.c:5595-5630)."""
+EDMD.c:2576-2585, has no bound; the capacity is this library's), which loop a
+batch gets (the reference has one, mainLoop, EDMD.c:5595-5630), and each of
+them, deep calendars and windows of groups among them, against the oracle."""
 import time
 
 import numpy as np
 import pytest
 
 import edmd_fixtures as F
-from test_gpu_wide import QUIET, same_state, same_trace
+from test_gpu_wide import QUIET, VARIANTS, channel, same_state, same_trace
 
 pytestmark = pytest.mark.gpu
 
@@ -216,3 +217,79 @@ def test_lattice_start_costs_as_the_rest(gpu):
         b.close()
     first, then = (min(t[k] for t in took) for k in (0, 1))
     assert first < 1.5 * then, took
+
+
+def states_of(gpu, name, sizes):
+    if "vr" in VARIANTS[name]:
+        out = [gpu.init_random(n, 0.3, seed=n) for n in sizes]
+        if "wall_x" in VARIANTS[name]:
+            for st in out:
+                for key in ("x", "y"):
+                    st[key] = 0.51 + st[key] / st["Lx"] * (st["Lx"] - 1.02)
+        return out
+    if "wall_y" in VARIANTS[name]:
+        return [channel(n, n) for n in sizes]
+    return [F.lattice_state(n, 0.55, seed=n, lattice="fit") for n in sizes]
+
+
+def batch_matches_oracle(gpu, oracle, name, sizes, copies, waves, nev, **engine):
+    kw = dict(QUIET, **{k: v for k, v in VARIANTS[name].items() if "screen" not in k})
+    base = states_of(gpu, name, sizes)
+    b = gpu.Batch(base * copies, trace_capacity=nev, **kw, **engine)
+    assert b.wavefronts() == waves
+    b.run(max_events=nev // 3)
+    b.run(max_events=nev)
+    for k, st in enumerate(base):
+        o = oracle.Oracle(st, **kw)
+        code, tr = o.run(nev)
+        assert code == 0
+        at = (copies - 1) * len(base) + k
+        same_trace(b.trace(at), tr)
+        same_state(b.state(at), o.state())
+    b.close()
+
+
+@pytest.mark.parametrize("sizes,copies,waves", [((6400,), 1, 16), ((70, 70, 70, 6145), 1, 8),
+                                                ((6200,), 260, 4)])
+@pytest.mark.parametrize("name", ["plain", "thermostat", "walls", "field", "damping", "thermal",
+                                  "grow", "grow_walls"])
+def test_windows_of_groups_match_oracle(gpu, oracle, name, sizes, copies, waves):
+    """Above 6144 disks the window is of groups of 64 leaves, of every system of
+    the batch: on 16, 8 and 4 wavefronts."""
+    batch_matches_oracle(gpu, oracle, name, sizes, copies, waves, 1500)
+
+
+@pytest.mark.parametrize("name,n", [("plain", 262145), ("plain", 6400), ("walls", 6400),
+                                    ("field", 6400), ("damping", 6400), ("thermal", 6400),
+                                    ("grow", 6400), ("grow_walls", 6400), ("field", 262145),
+                                    ("grow", 262145)])
+def test_deep_calendars_on_one_wavefront_match_oracle(gpu, oracle, name, n):
+    """The loop of one wavefront above 4096 disks (two levels of groups) and
+    above 2^18 (three), which batches of more than four systems a compute unit
+    run; here by a cell capacity that the other loop does not take."""
+    batch_matches_oracle(gpu, oracle, name, (n,), 1, 1, 1500, cell_capacity=30)
+
+
+@pytest.mark.parametrize("name", list(VARIANTS))
+def test_four_and_eight_wavefronts_agree_with_one(gpu, name):
+    """Three systems of 350 to 400 disks alone (8 wavefronts each, arrays in
+    LDS), in batches of 300 and 600 (4) and of 1200 (1): states, counters, sums,
+    thermo rows and calendars alike."""
+    base = states_of(gpu, name, (350, 380, 400))
+    got = []
+    for size, waves in ((1200, 1), (3, 8), (300, 4), (600, 4)):
+        b = gpu.Batch(base * (size // 3), **VARIANTS[name])
+        assert b.wavefronts() == waves, size
+        b.run(max_events=1500)
+        b.run(max_events=4000, tmax=12.0)
+        got.append([(b.state(size - 3 + k), b.observables(size - 3 + k), b.thermo(size - 3 + k),
+                     b.calendar(size - 3 + k)) for k in range(3)])
+        b.close()
+    for other in got[1:]:
+        for (sa, oa, ta, ca), (sb, ob, tb, cb) in zip(got[0], other):
+            same_state(sb, sa)
+            assert oa == ob
+            assert np.array_equal(ta.view(np.uint8), tb.view(np.uint8))
+            for k in ca:
+                assert np.array_equal(np.asarray(ca[k]).view(np.uint8),
+                                      np.asarray(cb[k]).view(np.uint8)), k
