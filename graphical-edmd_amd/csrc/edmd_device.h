@@ -117,26 +117,6 @@ __device__ __forceinline__ int order_key(double v, double base) {
     return b < 0 ? -m : m;
 }
 
-/* Lane holding the minimum of v over the wave, the lowest lane among equal
- * values, and that minimum.  The search runs on order_key(v, base) with
- * single-instruction DPP steps; the lane holding the exact minimum always
- * has the least key, and only when several lanes share it are their
- * doubles compared.  base should lie near the values for resolution (any
- * finite base is correct). */
-__device__ __forceinline__ int wave_argmin_lane(double v, double base, double& vmin) {
-    const int k = order_key(v, base);
-    const int mk = wave_min_i32(k);
-    const uint64_t tied = __ballot(k == mk);
-    if (__popcll(tied) == 1) {
-        const int w = (int)__builtin_ctzll(tied);
-        vmin = lane_value(v, w);
-        return w;
-    }
-    const double vv = (k == mk) ? v : INF_D;
-    vmin = wave_min(vv);
-    return (int)__builtin_ctzll(__ballot(vv == vmin));
-}
-
 /* Two independent int minima over the wave at once: the same DPP steps as
  * wave_min_i32 with the two chains interleaved, so each DPP step's latency
  * is covered by the other chain's step. */
@@ -155,33 +135,6 @@ __device__ __forceinline__ void wave_min_i32x2(int& a, int& b) {
     const int b2 = __builtin_amdgcn_readlane(b, 32), b3 = __builtin_amdgcn_readlane(b, 48);
     a = imin(imin(a0, a1), imin(a2, a3));
     b = imin(imin(b0, b1), imin(b2, b3));
-}
-
-/* wave_argmin_lane of two values at once (the minima of two owners over the
- * same candidate pass): the key searches run interleaved; each result is
- * the one wave_argmin_lane gives for that value alone. */
-__device__ __forceinline__ void wave_argmin_lane2(double va, double vb, double base, double& ma,
-                                                  int& wa, double& mb, int& wb) {
-    const int ka = order_key(va, base), kb = order_key(vb, base);
-    int mka = ka, mkb = kb;
-    wave_min_i32x2(mka, mkb);
-    const uint64_t ta = __ballot(ka == mka), tb = __ballot(kb == mkb);
-    if (__popcll(ta) == 1) {
-        wa = (int)__builtin_ctzll(ta);
-        ma = lane_value(va, wa);
-    } else {
-        const double vv = (ka == mka) ? va : INF_D;
-        ma = wave_min(vv);
-        wa = (int)__builtin_ctzll(__ballot(vv == ma));
-    }
-    if (__popcll(tb) == 1) {
-        wb = (int)__builtin_ctzll(tb);
-        mb = lane_value(vb, wb);
-    } else {
-        const double vv = (kb == mkb) ? vb : INF_D;
-        mb = wave_min(vv);
-        wb = (int)__builtin_ctzll(__ballot(vv == mb));
-    }
 }
 
 /* ------------------------------------------------------------ kinematics */

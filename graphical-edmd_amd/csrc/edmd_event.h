@@ -1,8 +1,10 @@
 /*
- * One particle event in two steps, shared by the event loops: event_open
- * (records read, free flight, collision rule, cell or wall change) and
- * event_predict (new collision and crossing times), neither of which writes
- * to the system, and event_commit, which does.
+ * One particle event in steps, shared by the event loops: event_open (records
+ * read, free flight, collision rule, cell or wall change) and event_predict
+ * (new collision and crossing times), which write nothing to the system
+ * (event_predict only where SPEC is false, the neighbours' flights under the
+ * field or damping), then event_cells, event_store, event_enter, event_sums and
+ * event_slots, which do.
  *
  * Half-wave layout: lanes 0-31 hold the event's first disk, lanes 32-63 its
  * second one (a valid collision's partner; else the first disk again), so
