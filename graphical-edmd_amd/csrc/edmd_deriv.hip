@@ -59,6 +59,7 @@
 #include <stdint.h>
 
 #include "edmd_internal.h"
+#include "edmd_lanes.h"
 #include "edmd_math.h"
 #include "edmd_types.h"
 
@@ -173,8 +174,8 @@ __device__ __forceinline__ uint64_t chain_mask(unsigned long long* who, int lane
     unsigned long long* const wi = who + (i & (CHAIN_SLOTS - 1));
     unsigned long long* const wj = who + ((j >= 0 ? j : i) & (CHAIN_SLOTS - 1));
     if (on) {
-        atomicOr(wi, 1ull << lane);
-        atomicOr(wj, 1ull << lane);
+        atomicOr(wi, (unsigned long long)bit_mask(lane));
+        atomicOr(wj, (unsigned long long)bit_mask(lane));
     }
     WAVE_SYNC();
     const uint64_t m = on ? *wi | *wj : 0;
@@ -214,7 +215,7 @@ __global__ __launch_bounds__(64) void k_tangent(const EdmdSys* __restrict__ syst
         next = tape_load(A.tape, base + 64 + lane, base + 64 + lane < nt);
         const bool on = base + lane < nt;
         const int i = r.i, j = r.j;
-        const uint64_t before = chain_mask(who, lane, on, i, j) & (((uint64_t)1 << lane) - 1);
+        const uint64_t before = chain_mask(who, lane, on, i, j) & bits_below(lane);
         const bool pair = on && j >= 0;
         double* const ti = V.v + 4 * i;
         double* const tj = V.v + 4 * (j >= 0 ? j : i);
@@ -224,7 +225,7 @@ __global__ __launch_bounds__(64) void k_tangent(const EdmdSys* __restrict__ syst
         const double kap = ff / b;
         double term = 0, dt = 0;
         for (uint64_t todo = __ballot(on); todo;) {
-            const bool now = ((todo >> lane) & 1) != 0 && (before & todo) == 0;
+            const bool now = lane_in(todo) && (before & todo) == 0;
             if (now) {
                 double ti0 = ti[0], ti1 = ti[1], ti2 = ti[2], ti3 = ti[3];
                 tan_fly(ti0, ti1, ti2, ti3, r.t - V.tl[i], g);
@@ -322,7 +323,7 @@ __global__ __launch_bounds__(64) void k_adjoint(const EdmdSys* __restrict__ syst
         k = top - 128 + lane;
         next = tape_load(A.tape, k, k >= 0);
         const int i = r.i, j = r.j;
-        const uint64_t after = chain_mask(who, lane, on, i, j) & ~(((uint64_t)2 << lane) - 1);
+        const uint64_t after = chain_mask(who, lane, on, i, j) & ~bits_below(lane + 1);
         const bool pair = on && j >= 0;
         const uint64_t pairs = __ballot(pair);
         /* the tape's last pair takes the seed on its time */
@@ -335,7 +336,7 @@ __global__ __launch_bounds__(64) void k_adjoint(const EdmdSys* __restrict__ syst
         const double b = ax * cx + ay * cy;
         const double kap = ff / b;
         for (uint64_t todo = __ballot(on); todo;) {
-            const bool now = ((todo >> lane) & 1) != 0 && (after & todo) == 0;
+            const bool now = lane_in(todo) && (after & todo) == 0;
             if (now) {
                 double li0 = li[0], li1 = li[1], li2 = li[2], li3 = li[3];
                 adj_fly(li0, li1, li2, li3, V.tl[i] - r.t, g);

@@ -19,6 +19,7 @@
 #include <stdint.h>
 
 #include "edmd_internal.h"
+#include "edmd_lanes.h"
 #include "edmd_math.h"
 #include "edmd_types.h"
 
@@ -946,7 +947,7 @@ __device__ __forceinline__ void wave_argmin_finish(const AR& A, int kk, int mkk,
         /* equal keys: the earlier in the reference's queue (lower rank) */
         /* loaded by every lane (padding lanes read leaf 0) and selected,
          * not loaded under a divergent branch */
-        const bool tie = ((tied >> (threadIdx.x & 63)) & 1) != 0;
+        const bool tie = lane_in(tied);
         const int64_t rl = A.lrank[tie ? i : 0];
         int64_t r = tie ? rl : INT64_MAX;
         int l = tie ? (int)(threadIdx.x & 63) : 64;

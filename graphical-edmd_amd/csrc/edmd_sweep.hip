@@ -143,11 +143,7 @@ __device__ __forceinline__ void pair_terms(const EdmdConst& C, double ox, double
 /* The bits of the 64-bit mark word starting at candidate base that stay
  * set: candidates k < tot other than kself. */
 __device__ __forceinline__ uint64_t keep_bits(int tot, int kself, int base) {
-    const int r = tot - base;
-    uint64_t m = r >= 64 ? ~(uint64_t)0 : (r <= 0 ? (uint64_t)0 : ((uint64_t)1 << r) - 1);
-    const int sb = kself - base;
-    if (sb >= 0 && sb < 64) m &= ~((uint64_t)1 << sb);
-    return m;
+    return bits_below(tot - base) & ~bit_mask(kself - base);
 }
 
 /* The predictions of a staged tile's own disks, one thread per disk.  The

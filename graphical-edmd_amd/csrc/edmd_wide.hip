@@ -232,7 +232,7 @@ __device__ __forceinline__ void group_min(int lane, double& k, int& i, int& x, i
     const uint64_t at = __ballot(k == mk);
     int w = (int)__builtin_ctzll(at);
     if (__popcll(at) > 1 && mk < INF_D) {
-        const bool tie = ((at >> lane) & 1) != 0;
+        const bool tie = lane_in(at);
         int64_t q = tie ? r : INT64_MAX;
         int l = tie ? lane : 64;
 #pragma unroll
@@ -528,8 +528,7 @@ __device__ __forceinline__ bool wide_pick(const EdmdConst& C, WideShared<NW>& Sh
     uint64_t use = __ballot(lane < n && !(flags & WO_SHADOWED));
     const uint64_t end = __ballot((flags & WO_STOP) != 0);
     if (end) use &= ((uint64_t)1 << __builtin_ctzll(end)) - 1;
-    const int pos = (int)__popcll(use & (((uint64_t)1 << lane) - 1));
-    const uint64_t mine = __ballot(pos == wave && ((use >> lane) & 1) != 0);
+    const uint64_t mine = __ballot(lanes_before(use) == wave && lane_in(use));
     const int ord = mine ? (int)__builtin_ctzll(mine) : 0;
     double paul;
     int steps;
@@ -593,7 +592,7 @@ __device__ __forceinline__ void wide_first(const WideCal& Wc, WideShared<NW>& Sh
         e.rank = r1;
         e.p = Wc.ls > 0 ? Wc.idx[node] : node;
         e.aux = Wc.aux[node];
-        Sh.list[__popcll(all & (((uint64_t)1 << lane) - 1))] = e;
+        Sh.list[lanes_before(all)] = e;
     }
     const double k0 = wave_min(k1);
     WAVE_SYNC();
@@ -922,7 +921,7 @@ __device__ __forceinline__ void wide_loop(const EdmdConst& Cs, const AR& As, Edm
 #pragma unroll
                         for (int u = 0; u < 4; ++u) {
                             const uint64_t in = __ballot(k[u] < lim);
-                            const int to = at + (int)__popcll(in & (((uint64_t)1 << lane) - 1));
+                            const int to = at + lanes_before(in);
                             at += (int)__popcll(in);
                             if (k[u] < lim && to < WIDE_LIST<NW>) {
                                 const int g = g0 + u * (NT - 64);

@@ -293,3 +293,23 @@ def test_four_and_eight_wavefronts_agree_with_one(gpu, name):
             for k in ca:
                 assert np.array_equal(np.asarray(ca[k]).view(np.uint8),
                                       np.asarray(cb[k]).view(np.uint8)), k
+
+
+@pytest.mark.parametrize("n,mode,res", [(300, "run", "RES_AUTO"), (400, "run", "RES_AUTO"),
+                                        (900, "run", "RES_AUTO"), (50, "grow", "RES_AUTO"),
+                                        (300, "grow", "RES_AUTO"), (300, "grow", "RES_HBM")])
+def test_copies_that_share_a_compute_unit_end_alike(gpu, n, mode, res):
+    """512 copies, two a compute unit: each ends as the one alone does."""
+    if mode == "run":
+        st, kw, run = F.lattice_state(n, 0.6, seed=n, lattice="fit"), {}, dict(max_events=12000)
+    else:
+        st, kw, run = gpu.init_random(n, 0.55, seed=n), dict(vr=0.3), dict(max_events=30000, tmax=2.0)
+    ends = []
+    for size in (1, 512):
+        b = gpu.Batch([st] * size, **kw)
+        b.set_residency(getattr(gpu, res))
+        b.run(**run)
+        ends.append([b.state(k) for k in range(size)])
+        b.close()
+    for s in ends[1]:
+        same_state(s, ends[0][0])
