@@ -923,14 +923,15 @@ static int choose_residency(edmd_batch* b) {
 /* Wavefronts a system of so many disks (the batch's mean) gets of the 16 a CU
  * has at the loop's registers (128), which per_cu systems share.  A round
  * commits the events up to the first two that lie near each other, so what
- * more wavefronts give depends on the disks:
- * of 16 events 12 commit at 2000 disks, of 8 there 7.3, at 400 disks 3.4,
- * while every wavefront adds to the round's length.  us a collision with 4, 8,
+ * more wavefronts give depends on the disks: of 16 events 11.8 commit at 2000
+ * disks, of 8 at 400 disks 3.7, while every wavefront adds to the round's
+ * length.  us a collision with 4, 8,
  * 16 wavefronts: one system of 200 disks 3.18, 3.45, 4.25; 400 2.67, 2.52,
  * 3.17; 1500 2.50, 1.65, 1.75; 2000 2.54, 1.57, 1.49; 4000 2.82, 1.61, 1.25;
- * 2^18 3.85, 2.05, 1.45.  512 systems with 4, 8, arrays in HBM: 400 disks
- * 3.38, 3.54; 1000 3.23, 2.51.  1024 systems with 4, and in the loop of one wavefront: 400
- * disks 4.25, 6.55; 1000 3.83, 6.72. */
+ * 2^18 3.85, 2.05, 1.45.  512 systems with 4, 8: 350 disks 3.49, 3.87 (arrays in
+ * LDS); 400 3.22 in LDS, 3.58 in HBM; 450 3.28, 3.27; 500 3.40, 3.37; 600 3.18,
+ * 2.94; 1000 3.23, 2.52 (HBM).  1024 systems with 4, and in the loop of one
+ * wavefront: 400 disks 4.25, 6.55; 1000 3.83, 6.72. */
 static int wide_width(int per_cu, int64_t disks) {
     if (per_cu > 2) return 4;
     if (per_cu > 1) return disks < 500 ? 4 : 8;
@@ -954,8 +955,12 @@ static int64_t wide_cells(int per_cu, int reach, bool rescales) {
 /* Whether the loop runs each system on a workgroup of several wavefronts
  * (edmd_wide.hip): while the device has wavefront slots to spare, i.e. for
  * batches of at most EDMD_WIDE_PER_CU systems a CU, all of them resident at
- * once, of at least wide_cells cells.  With the arrays in LDS where that mode is in use and they fit beside
- * the window; asked for LDS and not fitting, the loop of one wavefront runs. */
+ * once, of at least wide_cells cells.  A window of leaves (20 bytes a disk)
+ * leaves room for four systems a CU up to 1500 disks, three up to 2180 and two
+ * up to 3540; the kernels with a window of groups on 4 and 8 wavefronts have
+ * 196 registers, so two systems a CU at most.  With the arrays in LDS where
+ * that mode is in use and they fit beside the window; asked for LDS and not
+ * fitting, the loop of one wavefront runs. */
 static int choose_wide(edmd_batch* b) {
     b->wide_waves[0] = b->wide_waves[1] = 0;
     int dev = 0, ncu = 0;

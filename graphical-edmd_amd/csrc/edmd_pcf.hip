@@ -163,8 +163,9 @@ __device__ __forceinline__ double pcf_apart(double a0, double a1, double b0, dou
  * A pair's bin is (int)(sqrt(d2) / dr) with the reference's roundings: the
  * 64-bit square root and division take it only where a 32-bit quotient (error
  * below 3.2e-7 of it: four roundings of half a unit, a root good to one) lies
- * within `tol` = 1e-6 + 4e-7 nb of a whole number, or at the bins' end.  With a
- * 64-bit reciprocal root in its place the kernel took 121 us for 117. */
+ * within `tol` = 1e-6 + 4e-7 nb of a whole number, or at the bins' end.  With the
+ * 64-bit root and division for every pair the kernel takes 88.5 us for 59.4
+ * (60000 disks, 500 bins up to 10 diameters). */
 template <bool WRAP>
 __device__ __forceinline__ void pcf_tile(const double2* stage, int jn, double2 a, bool act,
                                          int first, double Lx, double Ly, double dr, float inv,

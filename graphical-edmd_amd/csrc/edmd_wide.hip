@@ -32,12 +32,17 @@
  * the limit or the spatial distribution; scheduled events and ring wraps are
  * handled between rounds by the whole workgroup.
  *
- * Each round has a fixed cost beside its events: of 19000 cycles (2000 disks)
- * the scan took 2600 and the ordering 4250 while the first wavefront alone did
- * it, a chain of some thirty dependent LDS accesses.  Spread over the
- * wavefronts, one comparison of 64 lanes per entry, and with one count for a
- * scan's four nodes a lane, the round takes 17400 (2000 disks, 4000
- * collisions on 8 wavefronts: 6.76 ms to 6.20).
+ * What a round costs and gives (cycles, and events committed): 400 disks in
+ * LDS on 8 wavefronts 16100, 3.7; 512 such systems on 4 wavefronts each 16900,
+ * 3.0; 2000 disks on 16 wavefronts 21800, 11.8; 2^20 disks 40800, 13.2; 1000
+ * disks in a channel under the field on 8 wavefronts 24300, 4.5.  More than half
+ * of the wavefronts' cycles are waits (52 to 65%), for memory and at the
+ * barriers.  The scan and the ordering are a part that no event shares: while
+ * the first wavefront alone did them, a chain of some thirty dependent LDS
+ * accesses, they took 2600 and 4250 of 19000 cycles (2000 disks on 8
+ * wavefronts).  Spread over the wavefronts, one comparison of 64 lanes per
+ * entry, and with one count for a scan's four nodes a lane, that round went to
+ * 17400 (4000 collisions 6.76 ms to 6.20).
  *
  * The calendar's window level lives in LDS: the leaves themselves up to
  * EDMD_WIDE_FLAT disks, else the first level of at most EDMD_WIDE_NODES

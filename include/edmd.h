@@ -286,9 +286,13 @@ int edmd_queue_remove(edmd_ctx* ctx, int kind, int i);
 /* ---- batched replicas ---------------------------------------------------- */
 typedef struct edmd_batch edmd_batch;
 
-/* nsys independent systems of any sizes, in one persistent launch: each on
- * 4 to 16 wavefronts in batches of up to four systems per compute unit, on
- * one in larger ones. */
+/* nsys independent systems of any sizes, in one persistent launch.  Each runs
+ * on 4, 8 or 16 wavefronts where the batch holds at most four systems per
+ * compute unit, their calendars' windows fit its LDS, they have cells enough (about 36 each with one system per
+ * compute unit, 72 with four, twice that under the field or damping), every
+ * cell capacity is at most 24 and a multiple of 4 (the one the library
+ * chooses where the smallest radius is 0.3 and more) and the run is longer
+ * than a few events; on one wavefront else.  Results are the same. */
 int edmd_batch_create(const edmd_system_desc* descs, int nsys, edmd_batch** out);
 int edmd_batch_destroy(edmd_batch* b);
 /* Every system runs until its own event counter reaches max_events or its
