@@ -611,8 +611,9 @@ __device__ __forceinline__ void wide_first(const WideCal& Wc, WideShared<NW>& Sh
 
 /* The leader's decision where a round cannot start from the gathered nodes:
  * too many of them (the first of them, WT_SCAN) or none (another limit,
- * WT_SCAN; the earliest event alone after twelve), or the earliest one is not plain (what findNextEvent does
- * next, EDMD.c:2313-2327, one ring wrap at a time). */
+ * WT_SCAN; the earliest event alone after twelve), or the earliest one is not
+ * plain (what findNextEvent does next, EDMD.c:2313-2327, one ring wrap at a
+ * time). */
 template <int NW, class AR>
 __device__ __forceinline__ int wide_decide(const EdmdConst& C, const AR& A, int lane,
                                            const WideCal& Wc, WideShared<NW>& Sh, bool ordered) {
